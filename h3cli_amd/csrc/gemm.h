@@ -1,0 +1,44 @@
+// Shared by the projection GEMM translation units: arguments, epilogue math and
+// the launchers that h3_gemm chooses between.
+#pragma once
+#include "common.h"
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+struct GemmArgs {
+    uint16_t *y;
+    const uint16_t *x;
+    const void *w;            // bf16 [N,K] or int8 [N,K]
+    const float *scales;      // q8: [N, groups]
+    const uint16_t *bias;     // optional [N]
+    const float *alpha;       // EPI bit 2: device scalar multiplying the accumulator
+    unsigned m, n, k, group, groups;
+    int gelu;
+};
+
+__device__ inline float gelu_tanh(float v) {
+    // Reference h3_gelu_bf16, approximate form (src/cuda/cuda_kernels.cuh:879-902):
+    // 0.5 v (1 + tanh(c (v + 0.044715 v^3))), c = sqrt(2 / pi), written as
+    // v / (1 + exp(-2 c (v + 0.044715 v^3))) with the hardware exp and
+    // reciprocal (no IEEE division, no branches). Large |v| saturate through
+    // exp: to v (exp -> 0) or to a signed zero (exp -> inf, reciprocal 0).
+    const float u = v * (1.5957691216057308f + 0.071354816272192f * v * v);
+    return v * __builtin_amdgcn_rcpf(1.0f + __expf(-u));
+}
+
+// 16 int8 codes of one scale group -> BF16 values w = bf16(code * scale), the
+// reconstruction of the reference's Metal kernel (src/metal/shaders.metal:825-827).
+__device__ inline void dequant16(const i32x4 &q, float s, bf16x8 *half) {
+#pragma unroll
+    for (int e = 0; e < 16; e += 2) {
+        const int word = q[e / 4];
+        f32x2 f = {(float)(int8_t)(word >> (8 * (e % 4))) * s, (float)(int8_t)(word >> (8 * (e % 4 + 1))) * s};
+        bf16x2 b = __builtin_convertvector(f, bf16x2);
+        half[e / 8][e % 8] = b[0];
+        half[e / 8][e % 8 + 1] = b[1];
+    }
+}
+
+// gemm_skinny.hip: at most 32 rows.
+bool h3_gemm_skinny_fits(const GemmArgs &a, bool q8);
+int h3_gemm_skinny(h3_gpu *g, const GemmArgs &a, bool q8);

@@ -33,6 +33,7 @@
 // shapes (and as H3_HIP_GEMM_VARIANT=3 for comparison).
 #include "common.h"
 #include "internal.h"
+#include "gemm.h"
 #include <cmath>
 
 
@@ -59,29 +60,6 @@ __device__ inline unsigned swz(unsigned row, unsigned ch) { return ch ^ ((row >>
 // parity, so their LDS stores hit eight different chunks.
 __device__ inline unsigned w_row(unsigned c) { const unsigned l = c % 16; return (c / 64) * 16 + 2 * (l % 8) + l / 8; }
 __device__ inline unsigned w_part(unsigned c) { return (c / 16) % 4; }
-
-struct GemmArgs {
-    uint16_t *y;
-    const uint16_t *x;
-    const void *w;            // bf16 [N,K] or int8 [N,K]
-    const float *scales;      // q8: [N, groups]
-    const uint16_t *bias;     // optional [N]
-    const float *alpha;       // EPI bit 2: device scalar multiplying the accumulator
-    unsigned m, n, k, group, groups;
-    int gelu;
-};
-
-__device__ inline float gelu_tanh(float v) {
-    // Reference h3_gelu_bf16, approximate form (src/cuda/cuda_kernels.cuh:879-902):
-    // 0.5 v (1 + tanh(c (v + 0.044715 v^3))), c = sqrt(2 / pi), written as
-    // v / (1 + exp(-2 c (v + 0.044715 v^3))) with the hardware exp and
-    // reciprocal (no IEEE division, no branches). Large |v| saturate through
-    // exp: to v (exp -> 0) or to a signed zero (exp -> inf, reciprocal 0).
-    const float u = v * (1.5957691216057308f + 0.071354816272192f * v * v);
-    return v * __builtin_amdgcn_rcpf(1.0f + __expf(-u));
-}
-
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // WM x WN waves; each wave owns a (256 / WM) x (256 / WN) output tile of
 // 32 x 32 MFMA blocks. 2 x 4 waves (128 x 64 per wave, two waves per SIMD) or
@@ -814,6 +792,7 @@ int h3_gemm_bf16_alpha(h3_gpu *g, uint16_t *y, const uint16_t *x, const uint16_t
                        uint32_t k, uint32_t n) {
     GemmArgs a{};
     a.y = y; a.x = x; a.w = w; a.alpha = alpha; a.m = m; a.n = n; a.k = k; a.group = 1; a.groups = 1;
+    if (h3_gemm_skinny_fits(a, false)) return h3_gemm_skinny(g, a, false);
     if (pipe_fits(a) && g->gemm_variant != 3) return launch_pipe<4>(g, a);
     if (n % TN == 0 && k % TK == 0 && m >= 32) return launch_tiled<false, false, 4>(g, a);
     const size_t total = (size_t)m * n;
@@ -834,7 +813,9 @@ int h3_gemm(h3_gpu *g, uint16_t *y, const uint16_t *x, const h3_gpu_tensor *w, c
     const int epi = (bias ? 1 : 0) | (gelu ? 2 : 0);
     // Variant 3 keeps the earlier kernels (gemm_q8_staged, gemm_kernel) for A/B.
     const bool pipe = tiled && pipe_fits(a) && g->gemm_variant != 3;
-    if (pipe && !w->q8) {
+    if (h3_gemm_skinny_fits(a, w->q8 != 0)) {
+        ok = h3_gemm_skinny(g, a, w->q8 != 0);
+    } else if (pipe && !w->q8) {
         ok = launch_pipe_epi(g, a, epi);
     } else if (pipe) {
         // W8A16: a dequantization pass into the context's BF16 weight buffer

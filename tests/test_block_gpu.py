@@ -93,6 +93,46 @@ def test_w8a16_linear(gpu, m, k, n, group, bias, gelu):
     assert np.mean(ulp_diff(got, ref) <= 1) > 0.99
 
 
+@pytest.mark.parametrize("m,k,n,group,bias,gelu", [
+    (1, 64, 16, 0, False, False),       # one K step: seven of the eight waves have none
+    (2, 576, 30, 0, True, False),       # nine steps, a ragged column block
+    (16, 320, 8200, 0, False, True),    # the most rows of one row block
+    (17, 2176, 48, 0, True, True),      # two row blocks, 34 steps
+    (32, 192, 8200, 0, True, False),    # four column blocks per workgroup, the last one ragged
+    (5, 640, 37, 16, False, False),     # W8A16, smallest scale group
+    (16, 320, 8200, 64, True, False),   # W8A16, two column blocks per workgroup
+    (31, 1088, 8200, 1088, False, True),
+])
+def test_few_rows_linear(gpu, m, k, n, group, bias, gelu):
+    """At most 32 rows against FP64: one BF16 rounding (two with the GELU) of the
+    result plus the FP32 sum's k 2^-24 sum |x w|."""
+    print(f"[few rows] m={m} k={k} n={n} group={group} bias={bias} gelu={gelu}", flush=True)
+    x = synth.normal_bf16(m + 3, m * k)
+    b = synth.normal_bf16(7, n, scale=0.1) if bias else None
+    if group:
+        codes, scales = synthetic_q8(m + n, n, k, group)
+        w = q8_weight(gpu, codes, scales, n, k, group)
+        wide = np.repeat(scales.reshape(n, -1), group, axis=1)[:, :k]
+        wv = bf16(synth.f32_to_bf16(codes.reshape(n, k).astype(np.float32) * wide)).astype(np.float64)
+    else:
+        bits = synth.normal_bf16(m + 4, n * k, scale=1 / math.sqrt(k))
+        w, wv = gpu.from_bf16(bits), bf16(bits).reshape(n, k).astype(np.float64)
+    tx, tb, out = gpu.from_bf16(x), gpu.from_bf16(b) if bias else None, gpu.empty(m * n)
+    fn = gpu.lib.h3_hip_linear_gelu_bf16 if gelu else gpu.lib.h3_gpu_linear_bf16
+    run(gpu, fn, out.handle, tx.handle, w.handle, tb.handle if bias else None, m, k, n)
+    got = bf16(out.read()).reshape(m, n).astype(np.float64)
+    xv = bf16(x).reshape(m, k).astype(np.float64)
+    want = xv @ wv.T + (bf16(b).astype(np.float64) if bias else 0.0)
+    bound = 2.0 ** -8 * np.abs(want) + k * 2.0 ** -24 * (np.abs(xv) @ np.abs(wv).T)
+    if gelu:
+        # |gelu'| <= 1.13; the second rounding, and the hardware exp and reciprocal.
+        want = 0.5 * want * (1 + np.tanh(math.sqrt(2 / math.pi) * (want + 0.044715 * want ** 3)))
+        bound = 1.13 * bound + 2.0 ** -8 * np.abs(want) + 2.0 ** -20
+    assert np.all(np.abs(got - want) <= bound), float(np.max(np.abs(got - want) / bound))
+    for t in (tx, out, w) + ((tb,) if bias else ()):
+        gpu.free(t)
+
+
 def test_bf16_linear_exact_pattern(gpu):
     """tests/quant_native.c:31-50 power-of-two pattern: the BF16 GEMM output must
     equal bf16(exact sum) bit for bit, for several row counts."""
