@@ -39,6 +39,10 @@ __device__ inline void dequant16(const i32x4 &q, float s, bf16x8 *half) {
     }
 }
 
-// gemm_skinny.hip: at most 32 rows.
+// gemm_skinny.hip: at most 32 rows. Sums of up to H3_GEMM_SHORT_K products stay with
+// gemm_small: a chain of that length is short (2 rows, 256 -> 5376: 8.3 us against
+// 3.2), and its sums, in K order, keep the timestep embedding's bits, which every
+// block's modulation depends on.
+constexpr unsigned H3_GEMM_SHORT_K = 256;
 bool h3_gemm_skinny_fits(const GemmArgs &a, bool q8);
 int h3_gemm_skinny(h3_gpu *g, const GemmArgs &a, bool q8);

@@ -137,7 +137,7 @@ int choose(h3_gpu *g, const GemmArgs &a) {
 }  // namespace
 
 bool h3_gemm_skinny_fits(const GemmArgs &a, bool q8) {
-    return a.m <= 32 && a.k % STEP == 0 && (!q8 || a.group % 16 == 0);
+    return a.m <= 32 && a.k > H3_GEMM_SHORT_K && a.k % STEP == 0 && (!q8 || a.group % 16 == 0);
 }
 
 int h3_gemm_skinny(h3_gpu *g, const GemmArgs &a, bool q8) { return q8 ? choose<true>(g, a) : choose<false>(g, a); }
