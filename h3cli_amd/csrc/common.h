@@ -119,6 +119,12 @@ struct h3_gpu_tensor {
 
 struct h3_gpu_event { hipEvent_t event; };
 
+// Grow-only device buffer; growing waits for queued work that may read the old one.
+struct h3_device_buffer {
+    void *ptr = nullptr;
+    size_t bytes = 0;
+};
+
 struct h3_attention_state;  // attention.hip
 struct h3_stream_state;     // context.hip (weight streaming bounce buffers)
 
@@ -151,6 +157,8 @@ struct h3_gpu {
     // (grow-only; reused by every projection on the compute stream).
     void *gemm_weights;
     size_t gemm_weights_bytes;
+    h3_device_buffer gemm_partials; // FP32 partial sums of the tiles split over K
+    unsigned cus;                   // compute units of the device
 };
 
 // ---------------------------------------------------------------- helpers

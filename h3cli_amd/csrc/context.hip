@@ -100,6 +100,7 @@ extern "C" h3_gpu *h3_gpu_create(const char *shader_source_path, char *error, si
     h3_gpu *g = new (std::nothrow) h3_gpu();
     if (!g) { if (error && error_size) snprintf(error, error_size, "out of host memory"); return nullptr; }
     g->device = device;
+    g->cus = prop.multiProcessorCount > 0 ? (unsigned)prop.multiProcessorCount : 256;
     g->created = now_seconds();
     g->profiling = getenv("H3_PROFILE") != nullptr;
     if (const char *v = getenv("H3_HIP_ATTENTION_VARIANT")) g->attention_variant = atoi(v);
@@ -131,6 +132,7 @@ extern "C" void h3_gpu_free(h3_gpu *g) {
     delete g->kernel_events;
     if (g->fault) hipFree(g->fault);
     if (g->gemm_weights) hipFree(g->gemm_weights);
+    h3_buffer_free(&g->gemm_partials);
     if (g->compute) hipStreamDestroy(g->compute);
     if (g->copy) hipStreamDestroy(g->copy);
     delete g;
@@ -673,6 +675,24 @@ int h3_buffer_reserve(h3_gpu *g, h3_device_buffer *b, size_t bytes, const char *
     if (!h3_hip_check(g, hipMalloc(&b->ptr, bytes), what)) { b->ptr = nullptr; return 0; }
     b->bytes = bytes;
     return 1;
+}
+
+bool h3_buffer_try(h3_gpu *g, h3_device_buffer *b, size_t bytes) {
+    if (b->bytes >= bytes) return true;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(g->compute, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (b->ptr && hipStreamSynchronize(g->compute) != hipSuccess) return false;
+    h3_buffer_free(b);
+    if (hipMalloc(&b->ptr, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        b->ptr = nullptr;
+        return false;
+    }
+    b->bytes = bytes;
+    return true;
 }
 
 void h3_buffer_free(h3_device_buffer *b) {

@@ -14,6 +14,10 @@ struct GemmArgs {
     const float *alpha;       // EPI bit 2: device scalar multiplying the accumulator
     unsigned m, n, k, group, groups;
     int gelu;
+    // gemm_bf16_pipe: tiles [0, full) are whole; each later one is split over K
+    // into `split` workgroups, whose FP32 partial sums go to part.
+    unsigned full, split;
+    float *part;
 };
 
 __device__ inline float gelu_tanh(float v) {

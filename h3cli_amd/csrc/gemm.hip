@@ -529,6 +529,56 @@ constexpr int PIPE_GROUP_M = 4;
     [S##x3] "=&v"(S##f[11]), [S##x4] "=&v"(S##f[12]), [S##x5] "=&v"(S##f[13]), [S##x6] "=&v"(S##f[14]),      \
     [S##x7] "=&v"(S##f[15])
 
+// First row and column of output tile pid: bands of PIPE_GROUP_M row tiles sweep
+// the columns together.
+__device__ inline void pipe_tile(const GemmArgs &a, unsigned pid, unsigned &m0, unsigned &n0) {
+    const unsigned tiles_m = (a.m + TM - 1) / TM, tiles_n = a.n / TN;
+    const unsigned band = pid / (PIPE_GROUP_M * tiles_n), first_m = band * PIPE_GROUP_M;
+    const unsigned rows_in_band = min(tiles_m - first_m, (unsigned)PIPE_GROUP_M);
+    const unsigned tm = first_m + (pid % (PIPE_GROUP_M * tiles_n)) % rows_in_band;
+    const unsigned tn = (pid % (PIPE_GROUP_M * tiles_n)) / rows_in_band;
+    m0 = __builtin_amdgcn_readfirstlane(tm * TM);
+    n0 = __builtin_amdgcn_readfirstlane(tn * TN);
+}
+
+// Output row `row`, columns col0 .. col0 + 127 of a wave: accumulator block i of
+// a lane holds columns col0 + 16 i + 4 q4 + 0..3. Blocks i and i + 1 go out
+// together as 16-byte stores: v_permlane16_swap hands the odd lane rows' block-i
+// values to the even rows and the even rows' block-(i+1) values to the odd rows,
+// so each lane holds eight consecutive columns.
+template <int EPI>
+__device__ inline void pipe_store(const GemmArgs &a, unsigned row, unsigned col0, unsigned q4, const f32x4 *c) {
+    uint16_t *dst = a.y + (size_t)row * a.n;
+#pragma unroll
+    for (int ip = 0; ip < 4; ip++) {
+        unsigned w[2][2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int i = 2 * ip + h;
+            const unsigned col = col0 + i * 16 + 4 * q4;
+            u16x4 out;
+            u16x4 bias4 = {};
+            if constexpr (EPI & 1) bias4 = *reinterpret_cast<const u16x4 *>(a.bias + col);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                float x = c[i][e];
+                if constexpr (EPI & 4) x *= a.alpha[0];
+                if constexpr (EPI & 1) x += bf16_to_f32(bias4[e]);
+                uint16_t b = f32_to_bf16(x);
+                if constexpr (EPI & 2) b = f32_to_bf16(gelu_tanh(bf16_to_f32(b)));
+                out[e] = b;
+            }
+            w[h][0] = out[0] | ((unsigned)out[1] << 16);
+            w[h][1] = out[2] | ((unsigned)out[3] << 16);
+        }
+        const auto s0 = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+        const auto s1 = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+        const unsigned col = col0 + 2 * ip * 16 + ((q4 & 1) ? 16 + 4 * (q4 - 1) : 4 * q4);
+        u32x4 v = {s0[0], s1[0], s0[1], s1[1]};
+        *reinterpret_cast<u32x4 *>(dst + col) = v;
+    }
+}
+
 template <int EPI>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
 void gemm_bf16_pipe(GemmArgs a) {
@@ -536,24 +586,33 @@ void gemm_bf16_pipe(GemmArgs a) {
     const unsigned tid = threadIdx.x, lane = tid % 64, n16 = lane % 16, q4 = lane / 16;
     const unsigned wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const unsigned wm = wave / 2, wn = wave % 2;
-    const unsigned tiles_m = (a.m + TM - 1) / TM, tiles_n = a.n / TN;
-    const unsigned pid = xcd_remap(blockIdx.x, gridDim.x);
-    const unsigned band = pid / (PIPE_GROUP_M * tiles_n), first_m = band * PIPE_GROUP_M;
-    const unsigned rows_in_band = min(tiles_m - first_m, (unsigned)PIPE_GROUP_M);
-    const unsigned tm = first_m + (pid % (PIPE_GROUP_M * tiles_n)) % rows_in_band;
-    const unsigned tn = (pid % (PIPE_GROUP_M * tiles_n)) / rows_in_band;
-    const unsigned m0 = __builtin_amdgcn_readfirstlane(tm * TM), n0 = __builtin_amdgcn_readfirstlane(tn * TN);
-    const unsigned ksteps = a.k / TK;
+    // Whole tiles first; a split tile's workgroups take the K stage pairs in
+    // `split` consecutive shares. Neighbouring workgroups share a K range.
+    unsigned pid, share = 0, k0 = 0, ksteps = a.k / TK;
+    const bool partial = blockIdx.x >= a.full;
+    if (!partial) {
+        pid = xcd_remap(blockIdx.x, a.full);
+    } else {
+        const unsigned count = gridDim.x - a.full, rest = count / a.split;
+        const unsigned id = xcd_remap(blockIdx.x - a.full, count);
+        share = id / rest;
+        pid = a.full + id % rest;
+        const unsigned pairs = ksteps / 2, p0 = share * pairs / a.split, p1 = (share + 1) * pairs / a.split;
+        k0 = p0 * 2 * TK;
+        ksteps = (p1 - p0) * 2;
+    }
+    unsigned m0, n0;
+    pipe_tile(a, pid, m0, n0);
 
-    const uint64_t xbase = (uint64_t)(a.x + (size_t)m0 * a.k);
-    const uint64_t wbase = (uint64_t)((const uint16_t *)a.w + (size_t)n0 * a.k);
+    const uint64_t xbase = (uint64_t)(a.x + (size_t)m0 * a.k + k0);
+    const uint64_t wbase = (uint64_t)((const uint16_t *)a.w + (size_t)n0 * a.k + k0);
     const unsigned xrows = min(a.m - m0, (unsigned)TM);
     const i32x4 sx = {(int)__builtin_amdgcn_readfirstlane((unsigned)xbase),
                       (int)__builtin_amdgcn_readfirstlane((unsigned)(xbase >> 32)),
-                      (int)__builtin_amdgcn_readfirstlane(xrows * a.k * 2), 0x00020000};
+                      (int)__builtin_amdgcn_readfirstlane((xrows * a.k - k0) * 2), 0x00020000};
     const i32x4 sw = {(int)__builtin_amdgcn_readfirstlane((unsigned)wbase),
                       (int)__builtin_amdgcn_readfirstlane((unsigned)(wbase >> 32)),
-                      (int)__builtin_amdgcn_readfirstlane(TN * a.k * 2), 0x00020000};
+                      (int)__builtin_amdgcn_readfirstlane((TN * a.k - k0) * 2), 0x00020000};
     const unsigned lrow = 8 * wave + lane / 8;
     // X and W tiles share the lane offsets: row lrow + 32 t, swizzled chunk.
     unsigned o[8];
@@ -610,48 +669,80 @@ void gemm_bf16_pipe(GemmArgs a) {
           [pw0] "v"(pw[0]), [pw1] "v"(pw[1]), [px0] "v"(px[0]), [px1] "v"(px[1])
         : "m0", "scc", "memory");
 
+    if (partial) {
+        // Partial sums of (split tile, share): element (i, j) of thread t at
+        // ((8 j + i) * 256 + t), so that every store instruction is contiguous.
+        f32x4 *dst = reinterpret_cast<f32x4 *>(a.part) + ((size_t)(pid - a.full) * a.split + share) * (TM * TN / 4) + tid;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            if (m0 + wm * 128 + j * 16 >= a.m) break;
+#pragma unroll
+            for (int i = 0; i < 8; i++) dst[(8 * j + i) * 256] = c[i][j];
+        }
+        return;
+    }
     // Block (i, j): lane holds output row m0 + wm*128 + j*16 + n16 and columns
-    // n0 + wn*128 + i*16 + 4*q4 + 0..3. Blocks i and i + 1 go out together
-    // as 16-byte stores: v_permlane16_swap hands the odd lane rows' block-i
-    // values to the even rows and the even rows' block-(i+1) values to the
-    // odd rows, so each lane holds eight consecutive columns.
+    // n0 + wn*128 + i*16 + 4*q4 + 0..3.
 #pragma unroll
     for (int j = 0; j < 8; j++) {
         const unsigned row = m0 + wm * 128 + j * 16 + n16;
         if (row >= a.m) continue;
-        uint16_t *dst = a.y + (size_t)row * a.n;
+        f32x4 block[8];
 #pragma unroll
-        for (int ip = 0; ip < 4; ip++) {
-            unsigned w[2][2];
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int i = 2 * ip + h;
-                const unsigned col = n0 + wn * 128 + i * 16 + 4 * q4;
-                u16x4 out;
-                u16x4 bias4 = {};
-                if constexpr (EPI & 1) bias4 = *reinterpret_cast<const u16x4 *>(a.bias + col);
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    float x = c[i][j][e];
-                    if constexpr (EPI & 4) x *= a.alpha[0];
-                    if constexpr (EPI & 1) x += bf16_to_f32(bias4[e]);
-                    uint16_t b = f32_to_bf16(x);
-                    if constexpr (EPI & 2) b = f32_to_bf16(gelu_tanh(bf16_to_f32(b)));
-                    out[e] = b;
-                }
-                w[h][0] = out[0] | ((unsigned)out[1] << 16);
-                w[h][1] = out[2] | ((unsigned)out[3] << 16);
-            }
-            const auto s0 = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
-            const auto s1 = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
-            const unsigned col = n0 + wn * 128 + 2 * ip * 16 + ((q4 & 1) ? 16 + 4 * (q4 - 1) : 4 * q4);
-            u32x4 v = {s0[0], s1[0], s0[1], s1[1]};
-            *reinterpret_cast<u32x4 *>(dst + col) = v;
-        }
+        for (int i = 0; i < 8; i++) block[i] = c[i][j];
+        pipe_store<EPI>(a, row, n0 + wn * 128, q4, block);
     }
 }
+
+// The split tiles' shares added in order, and the pipe kernel's epilogue. One
+// workgroup per (tile, accumulator row j); HBM-bound.
 template <int EPI>
-int launch_pipe(h3_gpu *g, const GemmArgs &a, bool timed = true) {
+__global__ __launch_bounds__(256) void gemm_pipe_reduce(GemmArgs a) {
+    const unsigned tile = blockIdx.x / 8, j = blockIdx.x % 8, tid = threadIdx.x;
+    const unsigned lane = tid % 64, wave = tid / 64, n16 = lane % 16, q4 = lane / 16;
+    unsigned m0, n0;
+    pipe_tile(a, a.full + tile, m0, n0);
+    const unsigned row = m0 + (wave / 2) * 128 + j * 16 + n16;
+    if (row >= a.m) return;
+    const f32x4 *src = reinterpret_cast<const f32x4 *>(a.part) + (size_t)tile * a.split * (TM * TN / 4) + 8 * j * 256 + tid;
+    f32x4 block[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) block[i] = src[i * 256];
+#pragma unroll 4
+    for (unsigned s = 1; s < a.split; s++) {
+        src += TM * TN / 4;
+#pragma unroll
+        for (int i = 0; i < 8; i++) block[i] += src[i * 256];
+    }
+    pipe_store<EPI>(a, row, n0 + (wave % 2) * 128, q4, block);
+}
+
+// How many K shares the tiles of the last, incomplete wave of workgroups get (1:
+// none). Modelled time of that wave in microseconds: 1.3 per 64 values of K, 2 per
+// workgroup, 0.13 per share for its 256 KB of partial sums written and read, and
+// 3 plus 0.9 for each share added in turn by the reduction launch. Measured,
+// BF16 weights, in microseconds, unsplit against the shares taken here: 63 tiles
+// (729 rows, 7168 -> 5376) 134.6, 4 shares 66.6; the same with K = 14336 312.7, 4
+// shares 111.3; 100 tiles (1200 rows, 13824 -> 5120) 291.9, 2 shares 173.1; 3 tiles
+// (729 rows, 5376 -> 256) 86.8, 8 shares 25.8; 336 tiles (729 rows, 5376 -> 28672),
+// the last 80 split, 242.6, 3 shares 201.8. Where the last wave is two thirds full
+// nothing is gained (693 tiles, 14336 -> 5376: 998, 2 shares 1018; 224 tiles,
+// 5376 -> 28672: 145.1, 2 shares 171.1). At most 512 shares (128 MB).
+unsigned pipe_split(const h3_gpu *g, unsigned tiles, unsigned k) {
+    const unsigned rest = tiles % g->cus, pairs = k / (2 * TK);
+    if (!rest) return 1;
+    unsigned best = 1;
+    float least = pairs * 2.6f + 2.f;
+    for (unsigned s = 2; s <= 32 && s <= pairs && rest * s <= 512; s++) {
+        const float waves = (float)((rest * s + g->cus - 1) / g->cus);
+        const float t = waves * ((pairs + s - 1) / s * 2.6f + 2.f) + rest * s * 0.13f + 3.f + 0.9f * s;
+        if (t < least) { least = t; best = s; }
+    }
+    return best;
+}
+
+template <int EPI>
+int launch_pipe(h3_gpu *g, GemmArgs a, bool timed = true) {
     constexpr size_t shared = PIPE_LDS;
     static bool configured = false;
     auto kernel = gemm_bf16_pipe<EPI>;
@@ -661,9 +752,17 @@ int launch_pipe(h3_gpu *g, const GemmArgs &a, bool timed = true) {
             return 0;
         configured = true;
     }
-    unsigned tiles = (a.m + TM - 1) / TM * (a.n / TN);
+    const unsigned tiles = (a.m + TM - 1) / TM * (a.n / TN);
+    unsigned rest = tiles % g->cus;
+    a.split = pipe_split(g, tiles, a.k);
+    if (a.split > 1 && !h3_buffer_try(g, &g->gemm_partials, (size_t)rest * a.split * TM * TN * 4)) a.split = 1;
+    if (a.split == 1) rest = 0;
+    a.full = tiles - rest;
+    a.part = (float *)g->gemm_partials.ptr;
     hipEvent_t timing = timed ? h3_kernel_timing_begin(g) : nullptr;
-    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(256), shared, g->compute, a);
+    hipLaunchKernelGGL(kernel, dim3(a.full + rest * a.split), dim3(256), shared, g->compute, a);
+    if (rest && h3_launch_status(g, "BF16 GEMM"))
+        hipLaunchKernelGGL(gemm_pipe_reduce<EPI>, dim3(rest * 8), dim3(256), 0, g->compute, a);
     h3_kernel_timing_end(g, timing);
     return h3_launch_status(g, "BF16 GEMM");
 }

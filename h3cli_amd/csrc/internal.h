@@ -49,7 +49,6 @@ int h3_launch_attention_sol(h3_gpu *g, void *workspace, uint16_t *out, const uin
                             const uint16_t *v, uint32_t seq, uint32_t heads, float scale, bool head_major,
                             uint32_t q_block, const h3_sol_lists *lists, uint32_t head0, uint32_t group);
 
-// Grow-only device buffer; growing waits for queued work that may read the old one.
 // FP8 projections (quant.hip): y = FP8 GEMM of x with a packed weight; teardown.
 int h3_quant_gemm(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tensor *in, const h3_gpu_tensor *w, uint32_t rows,
                   uint32_t k, uint32_t n);
@@ -58,11 +57,11 @@ void h3_quant_destroy(h3_gpu *g);
 int h3_gemm_bf16_alpha(h3_gpu *g, uint16_t *y, const uint16_t *x, const uint16_t *w, const float *alpha, uint32_t m,
                        uint32_t k, uint32_t n);
 
-struct h3_device_buffer {
-    void *ptr = nullptr;
-    size_t bytes = 0;
-};
 int h3_buffer_reserve(h3_gpu *g, h3_device_buffer *b, size_t bytes, const char *what);
+// As h3_buffer_reserve for a workspace that the caller can do without: false,
+// with no error left behind, when memory is short or the compute stream is being
+// captured (nothing may be allocated then).
+bool h3_buffer_try(h3_gpu *g, h3_device_buffer *b, size_t bytes);
 void h3_buffer_free(h3_device_buffer *b);
 
 // Dominant-kernel timing: h3_kernel_timing_begin records a start event on the

@@ -133,6 +133,43 @@ def test_few_rows_linear(gpu, m, k, n, group, bias, gelu):
         gpu.free(t)
 
 
+@pytest.mark.parametrize("m,k,n,q8,bias,gelu", [
+    (600, 4096, 512, False, False, False),    # six tiles, all split; the last row tile ragged
+    (600, 4224, 512, True, True, True),       # 33 stage pairs in uneven shares, every epilogue
+    (33, 2048, 256, False, True, False),      # one tile of 33 rows
+    (300, 1024, 33280, False, False, False),  # 260 tiles: 256 whole ones and four split ones
+])
+def test_linear_split_over_k(gpu, m, k, n, q8, bias, gelu):
+    """Tiles of an incomplete wave, whose K shares a second launch adds, against
+    FP64 within the bound of test_few_rows_linear."""
+    print(f"[split K] m={m} k={k} n={n} q8={q8} bias={bias} gelu={gelu}", flush=True)
+    x = synth.normal_bf16(m + 3, m * k)
+    b = synth.normal_bf16(7, n, scale=0.1) if bias else None
+    if q8:
+        codes, scales = synthetic_q8(m + n, n, k, k)
+        w = q8_weight(gpu, codes, scales, n, k, k)
+        wv = bf16(synth.f32_to_bf16(codes.reshape(n, k).astype(np.float32) * scales[:, None]))
+    else:
+        bits = synth.normal_bf16(m + 4, n * k, scale=1 / math.sqrt(k))
+        w, wv = gpu.from_bf16(bits), bf16(bits).reshape(n, k)
+    tx, tb, out = gpu.from_bf16(x), gpu.from_bf16(b) if bias else None, gpu.empty(m * n)
+    fn = gpu.lib.h3_hip_linear_gelu_bf16 if gelu else gpu.lib.h3_gpu_linear_bf16
+    run(gpu, fn, out.handle, tx.handle, w.handle, tb.handle if bias else None, m, k, n)
+    got = bf16(out.read()).reshape(m, n)
+    rows = np.unique(np.concatenate([np.arange(0, m, 37), [m - 1, min(255, m - 1), min(256, m - 1)]]))
+    xv = bf16(x).reshape(m, k)[rows].astype(np.float64)
+    for at in range(0, n, 4096):
+        wt = wv[at:at + 4096].astype(np.float64)
+        want = xv @ wt.T + (bf16(b)[at:at + 4096].astype(np.float64) if bias else 0.0)
+        bound = 2.0 ** -8 * np.abs(want) + k * 2.0 ** -24 * (np.abs(xv) @ np.abs(wt).T)
+        if gelu:
+            want = 0.5 * want * (1 + np.tanh(math.sqrt(2 / math.pi) * (want + 0.044715 * want ** 3)))
+            bound = 1.13 * bound + 2.0 ** -8 * np.abs(want) + 2.0 ** -20
+        assert np.all(np.abs(got[rows, at:at + 4096] - want) <= bound)
+    for t in (tx, out, w) + ((tb,) if bias else ()):
+        gpu.free(t)
+
+
 def test_bf16_linear_exact_pattern(gpu):
     """tests/quant_native.c:31-50 power-of-two pattern: the BF16 GEMM output must
     equal bf16(exact sum) bit for bit, for several row counts."""
