@@ -158,6 +158,7 @@ struct h3_gpu {
     void *gemm_weights;
     size_t gemm_weights_bytes;
     h3_device_buffer gemm_partials; // FP32 partial sums of the tiles split over K
+    h3_device_buffer mlp_workspace; // h3_gpu_mlp_bf16: activated rows (and the fused product)
     unsigned cus;                   // compute units of the device
 };
 

@@ -133,6 +133,7 @@ extern "C" void h3_gpu_free(h3_gpu *g) {
     if (g->fault) hipFree(g->fault);
     if (g->gemm_weights) hipFree(g->gemm_weights);
     h3_buffer_free(&g->gemm_partials);
+    h3_buffer_free(&g->mlp_workspace);
     if (g->compute) hipStreamDestroy(g->compute);
     if (g->copy) hipStreamDestroy(g->copy);
     delete g;

@@ -30,6 +30,12 @@ __device__ inline float gelu_tanh(float v) {
     return v * __builtin_amdgcn_rcpf(1.0f + __expf(-u));
 }
 
+// silu(gate) * up with the hardware exp and reciprocal, as gelu_tanh: large |gate|
+// saturate through exp to gate * up or a signed zero.
+__device__ inline float swiglu_fast(float gate, float up) {
+    return gate * __builtin_amdgcn_rcpf(1.0f + __expf(-gate)) * up;
+}
+
 // 16 int8 codes of one scale group -> BF16 values w = bf16(code * scale), the
 // reconstruction of the reference's Metal kernel (src/metal/shaders.metal:825-827).
 __device__ inline void dequant16(const i32x4 &q, float s, bf16x8 *half) {
@@ -42,6 +48,14 @@ __device__ inline void dequant16(const i32x4 &q, float s, bf16x8 *half) {
         half[e / 8][e % 8 + 1] = b[1];
     }
 }
+
+// Epilogue of h3_gemm after the bias. SwiGLU (no bias): the weight holds hidden gate
+// rows, then hidden up rows, n = 2 * hidden, and y is [m, hidden]; only where
+// h3_gemm_swiglu_fits.
+enum { H3_GEMM_PLAIN = 0, H3_GEMM_GELU = 1, H3_GEMM_SWIGLU = 2 };
+int h3_gemm(h3_gpu *g, uint16_t *y, const uint16_t *x, const h3_gpu_tensor *w, const uint16_t *bias, uint32_t m,
+            uint32_t k, uint32_t n, int activation);
+bool h3_gemm_swiglu_fits(const h3_gpu *g, const h3_gpu_tensor *w, uint32_t m, uint32_t k, uint32_t hidden);
 
 // gemm_skinny.hip: at most 32 rows. Sums of up to H3_GEMM_SHORT_K products stay with
 // gemm_small: a chain of that length is short (2 rows, 256 -> 5376: 8.3 us against

@@ -470,7 +470,7 @@ constexpr int PIPE_GROUP_M = 4;
 #define PIPE_LD_X(ST, T) "s_add_u32 m0, %[mb], 32768*" #ST "+4096*" #T "\n"                                  \
     "buffer_load_dwordx4 %[o" #T "], %[sx], %[kc] offen lds\n"
 #define PIPE_LD_W(ST, T) "s_add_u32 m0, %[mb], 65536+32768*" #ST "+4096*" #T "\n"                            \
-    "buffer_load_dwordx4 %[o" #T "], %[sw], %[kc] offen lds\n"
+    "buffer_load_dwordx4 %[w" #T "], %[sw], %[kc] offen lds\n"
 #define PIPE_LOADS_X(ST) PIPE_LD_X(ST, 0) PIPE_LD_X(ST, 1) PIPE_LD_X(ST, 2) PIPE_LD_X(ST, 3)                      \
     PIPE_LD_X(ST, 4) PIPE_LD_X(ST, 5) PIPE_LD_X(ST, 6) PIPE_LD_X(ST, 7)
 #define PIPE_LOADS_W(ST) PIPE_LD_W(ST, 0) PIPE_LD_W(ST, 1) PIPE_LD_W(ST, 2) PIPE_LD_W(ST, 3)                      \
@@ -548,6 +548,31 @@ __device__ inline void pipe_tile(const GemmArgs &a, unsigned pid, unsigned &m0, 
 // so each lane holds eight consecutive columns.
 template <int EPI>
 __device__ inline void pipe_store(const GemmArgs &a, unsigned row, unsigned col0, unsigned q4, const f32x4 *c) {
+    if constexpr (EPI & 8) {
+        // Blocks 2 i and 2 i + 1 are gate and up of output columns col0 / 2 + 16 i + 4 q4
+        // + 0..3: both rounded to BF16, as the separate SwiGLU reads them.
+        uint16_t *dst = a.y + (size_t)row * (a.n / 2);
+#pragma unroll
+        for (int ip = 0; ip < 2; ip++) {
+            unsigned w[2][2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                u16x4 out;
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    out[e] = f32_to_bf16(swiglu_fast(bf16_to_f32(f32_to_bf16(c[4 * ip + 2 * h][e])),
+                                                     bf16_to_f32(f32_to_bf16(c[4 * ip + 2 * h + 1][e]))));
+                w[h][0] = out[0] | ((unsigned)out[1] << 16);
+                w[h][1] = out[2] | ((unsigned)out[3] << 16);
+            }
+            const auto s0 = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+            const auto s1 = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+            const unsigned col = col0 / 2 + 32 * ip + ((q4 & 1) ? 16 + 4 * (q4 - 1) : 4 * q4);
+            u32x4 v = {s0[0], s1[0], s0[1], s1[1]};
+            *reinterpret_cast<u32x4 *>(dst + col) = v;
+        }
+        return;
+    }
     uint16_t *dst = a.y + (size_t)row * a.n;
 #pragma unroll
     for (int ip = 0; ip < 4; ip++) {
@@ -608,19 +633,27 @@ void gemm_bf16_pipe(GemmArgs a) {
     pipe_tile(a, pid, m0, n0);
 
     const uint64_t xbase = (uint64_t)(a.x + (size_t)m0 * a.k + k0);
-    const uint64_t wbase = (uint64_t)((const uint16_t *)a.w + (size_t)n0 * a.k + k0);
+    const unsigned wrow = EPI & 8 ? n0 / 2 : n0, wrows = EPI & 8 ? a.n / 2 + TN / 2 : TN;
+    const uint64_t wbase = (uint64_t)((const uint16_t *)a.w + (size_t)wrow * a.k + k0);
     const unsigned xrows = min(a.m - m0, (unsigned)TM);
     const i32x4 sx = {(int)__builtin_amdgcn_readfirstlane((unsigned)xbase),
                       (int)__builtin_amdgcn_readfirstlane((unsigned)(xbase >> 32)),
                       (int)__builtin_amdgcn_readfirstlane((xrows * a.k - k0) * 2), 0x00020000};
     const i32x4 sw = {(int)__builtin_amdgcn_readfirstlane((unsigned)wbase),
                       (int)__builtin_amdgcn_readfirstlane((unsigned)(wbase >> 32)),
-                      (int)__builtin_amdgcn_readfirstlane((TN * a.k - k0) * 2), 0x00020000};
+                      (int)__builtin_amdgcn_readfirstlane((wrows * a.k - k0) * 2), 0x00020000};
     const unsigned lrow = 8 * wave + lane / 8;
     // X and W tiles share the lane offsets: row lrow + 32 t, swizzled chunk.
     unsigned o[8];
 #pragma unroll
     for (int t = 0; t < 8; t++) o[t] = (lrow + 32 * t) * a.k * 2 + swz(lrow, lane % 8) * 16;
+    // SwiGLU: weight row 16 b + r of the tile (b < 16) is gate (b even) or up (b odd)
+    // row n0 / 2 + 16 (b / 2) + r, so that a lane's accumulator blocks 2 i and 2 i + 1
+    // hold both for the same columns.
+    unsigned ow[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++)
+        ow[t] = EPI & 8 ? (lrow / 16 * (a.n / 2) + 16 * t + lrow % 16) * a.k * 2 + swz(lrow, lane % 8) * 16 : o[t];
     const unsigned mb = __builtin_amdgcn_readfirstlane(wave * 1024);
     unsigned kn = 2 * TK * 2, kc = 0;
     const unsigned kmax = __builtin_amdgcn_readfirstlane((ksteps - 1) * TK * 2);
@@ -668,8 +701,9 @@ void gemm_bf16_pipe(GemmArgs a) {
           P16_SET(a), P16_SET(b),
           [kc] "+s"(kc), [kn] "+s"(kn), [pairs] "+s"(pairs)
         : [sx] "s"(sx), [sw] "s"(sw), [o0] "v"(o[0]), [o1] "v"(o[1]), [o2] "v"(o[2]), [o3] "v"(o[3]),
-          [o4] "v"(o[4]), [o5] "v"(o[5]), [o6] "v"(o[6]), [o7] "v"(o[7]), [mb] "s"(mb), [kmax] "s"(kmax),
-          [pw0] "v"(pw[0]), [pw1] "v"(pw[1]), [px0] "v"(px[0]), [px1] "v"(px[1])
+          [o4] "v"(o[4]), [o5] "v"(o[5]), [o6] "v"(o[6]), [o7] "v"(o[7]), [w0] "v"(ow[0]), [w1] "v"(ow[1]),
+          [w2] "v"(ow[2]), [w3] "v"(ow[3]), [w4] "v"(ow[4]), [w5] "v"(ow[5]), [w6] "v"(ow[6]), [w7] "v"(ow[7]),
+          [mb] "s"(mb), [kmax] "s"(kmax), [pw0] "v"(pw[0]), [pw1] "v"(pw[1]), [px0] "v"(px[0]), [px1] "v"(px[1])
         : "m0", "scc", "memory");
 
     if (partial) {
@@ -784,6 +818,7 @@ int launch_pipe_epi(h3_gpu *g, const GemmArgs &a, int epi, bool timed = true) {
     case 1: return launch_pipe<1>(g, a, timed);
     case 2: return launch_pipe<2>(g, a, timed);
     case 3: return launch_pipe<3>(g, a, timed);
+    case 8: return launch_pipe<8>(g, a, timed);
     default: return launch_pipe<4>(g, a, timed);
     }
 }
@@ -978,8 +1013,18 @@ int h3_gemm_bf16_alpha(h3_gpu *g, uint16_t *y, const uint16_t *x, const uint16_t
     return launch_small(g, a, false);
 }
 
+// Whether h3_gemm takes SwiGLU as its epilogue for this weight (gate rows, then up
+// rows; 2 * hidden in all): the pipe kernel's shapes.
+bool h3_gemm_swiglu_fits(const h3_gpu *g, const h3_gpu_tensor *w, uint32_t m, uint32_t k, uint32_t hidden) {
+    GemmArgs a{};
+    if (hidden > UINT32_MAX / 2) return false;
+    a.m = m; a.k = k; a.n = 2 * hidden;
+    return m > 32 && pipe_fits(a) && g->gemm_variant != 3 && (!w->q8 || w->q8_group % 16 == 0);
+}
+
 int h3_gemm(h3_gpu *g, uint16_t *y, const uint16_t *x, const h3_gpu_tensor *w, const uint16_t *bias, uint32_t m,
-            uint32_t k, uint32_t n, int gelu) {
+            uint32_t k, uint32_t n, int activation) {
+    const bool gelu = activation == H3_GEMM_GELU;
     GemmArgs a{};
     a.y = y; a.x = x; a.w = w->data; a.bias = bias; a.m = m; a.n = n; a.k = k; a.gelu = gelu;
     a.scales = w->q8 ? w->q8_scales : nullptr;
@@ -988,7 +1033,7 @@ int h3_gemm(h3_gpu *g, uint16_t *y, const uint16_t *x, const h3_gpu_tensor *w, c
     if (!h3_tensor_acquire(g, w)) return 0;
     int ok;
     const bool tiled = n % TN == 0 && k % TK == 0 && m >= 32 && (!w->q8 || a.group % 16 == 0);
-    const int epi = (bias ? 1 : 0) | (gelu ? 2 : 0);
+    const int epi = (bias ? 1 : 0) | (gelu ? 2 : 0) | (activation == H3_GEMM_SWIGLU ? 8 : 0);
     // Variant 3 keeps the earlier kernels (gemm_q8_staged, gemm_kernel) for A/B.
     const bool pipe = tiled && pipe_fits(a) && g->gemm_variant != 3;
     if (h3_gemm_skinny_fits(a, w->q8 != 0)) {

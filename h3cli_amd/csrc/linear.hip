@@ -2,6 +2,7 @@
 // fused QKV projection + norm/RoPE, the SwiGLU MLP, and q8 weight tensors.
 #include "common.h"
 #include "internal.h"
+#include "gemm.h"
 #include <cerrno>
 #include <cmath>
 #include <fcntl.h>
@@ -9,21 +10,19 @@
 #include <unistd.h>
 #include <vector>
 
-int h3_gemm(h3_gpu *g, uint16_t *y, const uint16_t *x, const h3_gpu_tensor *w, const uint16_t *bias, uint32_t m,
-            uint32_t k, uint32_t n, int gelu);
-
+// activation: H3_GEMM_PLAIN, _GELU or (n = 2 * hidden, where it fits) _SWIGLU.
 static int linear(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tensor *in, const h3_gpu_tensor *w,
-                  const h3_gpu_tensor *bias, uint32_t rows, uint32_t k, uint32_t n, int gelu) {
+                  const h3_gpu_tensor *bias, uint32_t rows, uint32_t k, uint32_t n, int activation) {
     if (!h3_launch_ready(g)) return 0;
     if (!rows || !k || !n || !w || w->owner != g)
         return h3_set_error(g, "linear %ux%ux%u: invalid shape or weight", rows, n, k);
     if (!h3_require(g, in, H3_GPU_BF16, (size_t)rows * k, "linear input") ||
-        !h3_require(g, out, H3_GPU_BF16, (size_t)rows * n, "linear output") ||
+        !h3_require(g, out, H3_GPU_BF16, (size_t)rows * (activation == H3_GEMM_SWIGLU ? n / 2 : n), "linear output") ||
         (bias && !h3_require(g, bias, H3_GPU_BF16, n, "linear bias")))
         return 0;
     if (w->quant_mode) {
         // Reference gpu_cuda.cu:928-930: packed FP8 weights take no bias or epilogue.
-        if (bias || gelu) return h3_set_error(g, "unsupported quantized projection offset/bias/type");
+        if (bias || activation) return h3_set_error(g, "unsupported quantized projection offset/bias/type");
         if (out == in) return h3_set_error(g, "linear: output aliases input");
         return h3_quant_gemm(g, out, in, w, rows, k, n);
     }
@@ -35,17 +34,17 @@ static int linear(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tensor *in, const 
     }
     if (out == in) return h3_set_error(g, "linear: output aliases input");
     return h3_gemm(g, (uint16_t *)out->data, (const uint16_t *)in->data, w,
-                   bias ? (const uint16_t *)bias->data : nullptr, rows, k, n, gelu);
+                   bias ? (const uint16_t *)bias->data : nullptr, rows, k, n, activation);
 }
 
 extern "C" int h3_gpu_linear_bf16(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tensor *in, const h3_gpu_tensor *w,
                                   const h3_gpu_tensor *bias, uint32_t rows, uint32_t k, uint32_t n) {
-    return g && linear(g, out, in, w, bias, rows, k, n, 0);
+    return g && linear(g, out, in, w, bias, rows, k, n, H3_GEMM_PLAIN);
 }
 
 extern "C" int h3_hip_linear_gelu_bf16(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tensor *in, const h3_gpu_tensor *w,
                                        const h3_gpu_tensor *bias, uint32_t rows, uint32_t k, uint32_t n) {
-    return g && linear(g, out, in, w, bias, rows, k, n, 1);
+    return g && linear(g, out, in, w, bias, rows, k, n, H3_GEMM_GELU);
 }
 
 extern "C" int h3_gpu_grouped_qkv_linear_rope_bf16(h3_gpu *g, h3_gpu_tensor *q, h3_gpu_tensor *k, h3_gpu_tensor *v,
@@ -57,16 +56,44 @@ extern "C" int h3_gpu_grouped_qkv_linear_rope_bf16(h3_gpu *g, h3_gpu_tensor *q, 
            h3_gpu_grouped_qkv_rope_bf16(g, q, k, v, qkv, qw, kw, c, s, rows, heads, dim, half, eps);
 }
 
+// The MLP's intermediates stay in a grow-only workspace of the context: allocating
+// and freeing them in each call waits for the GPU (8193 rows, 5376 -> 14336 -> 5376,
+// alone: 20.0 ms a call, of which 3.4 ms computing). Larger ones than this are
+// allocated per call, so the context keeps no more.
+constexpr size_t MLP_WORKSPACE = (size_t)1 << 30;
+
+// A BF16 tensor over workspace memory, for the operators of one call.
+static h3_gpu_tensor workspace_tensor(h3_gpu *g, void *data, size_t elements) {
+    h3_gpu_tensor t{};
+    t.owner = g; t.data = data; t.elements = elements; t.bytes = t.bytes_alloc = elements * 2;
+    t.dtype = H3_GPU_BF16; t.storage = H3_GPU_DEVICE_ONLY;
+    return t;
+}
+
 // fc1 (2*hidden, gate rows then up rows) -> SwiGLU -> fc2, as src/cuda/gpu_cuda.cu:1108-1112.
+// Where the projection kernel takes it, SwiGLU is fc1's epilogue and the 2 * hidden
+// wide product is never written.
 extern "C" int h3_gpu_mlp_bf16(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tensor *in, const h3_gpu_tensor *w1,
                                const h3_gpu_tensor *w2, uint32_t rows, uint32_t width, uint32_t hidden, uint32_t output_dim) {
     if (!g) return 0;
-    h3_gpu_tensor *fused = h3_gpu_tensor_new_bf16(g, (size_t)rows * hidden * 2);
-    h3_gpu_tensor *act = h3_gpu_tensor_new_bf16(g, (size_t)rows * hidden);
-    int ok = fused && act && h3_gpu_linear_bf16(g, fused, in, w1, nullptr, rows, width, hidden * 2) &&
-             h3_gpu_swiglu_bf16(g, act, fused, rows, hidden) &&
+    const size_t n = (size_t)rows * hidden;
+    const bool fused = w1 && w1->owner == g && !w1->quant_mode && h3_gemm_swiglu_fits(g, w1, rows, width, hidden);
+    // Each part with the slack of h3_gpu_tensor_alloc behind it.
+    const size_t part = (n * 2 + 511) & ~(size_t)255, product = fused ? 0 : (n * 4 + 511) & ~(size_t)255;
+    if (n && n <= MLP_WORKSPACE && part + product <= MLP_WORKSPACE && h3_buffer_try(g, &g->mlp_workspace, part + product)) {
+        h3_gpu_tensor act = workspace_tensor(g, g->mlp_workspace.ptr, n);
+        h3_gpu_tensor both = workspace_tensor(g, (char *)g->mlp_workspace.ptr + part, fused ? 0 : n * 2);
+        const int ok = fused ? linear(g, &act, in, w1, nullptr, rows, width, hidden * 2, H3_GEMM_SWIGLU)
+                             : h3_gpu_linear_bf16(g, &both, in, w1, nullptr, rows, width, hidden * 2) &&
+                                   h3_gpu_swiglu_bf16(g, &act, &both, rows, hidden);
+        return ok && h3_gpu_linear_bf16(g, out, &act, w2, nullptr, rows, hidden, output_dim);
+    }
+    h3_gpu_tensor *both = h3_gpu_tensor_new_bf16(g, n * 2);
+    h3_gpu_tensor *act = h3_gpu_tensor_new_bf16(g, n);
+    int ok = both && act && h3_gpu_linear_bf16(g, both, in, w1, nullptr, rows, width, hidden * 2) &&
+             h3_gpu_swiglu_bf16(g, act, both, rows, hidden) &&
              h3_gpu_linear_bf16(g, out, act, w2, nullptr, rows, hidden, output_dim);
-    h3_gpu_tensor_free(fused);
+    h3_gpu_tensor_free(both);
     h3_gpu_tensor_free(act);
     return ok;
 }

@@ -170,6 +170,45 @@ def test_linear_split_over_k(gpu, m, k, n, q8, bias, gelu):
         gpu.free(t)
 
 
+@pytest.mark.parametrize("m,k,hidden,n,group", [
+    (300, 512, 384, 256, 0),       # SwiGLU in fc1's epilogue, a ragged row tile
+    (600, 4096, 256, 512, 4096),   # the same from split tiles, W8A16
+    (33, 256, 128, 256, 64),       # one tile: 128 gate and 128 up rows
+    (20, 320, 128, 192, 0),        # few rows: separate SwiGLU
+    (70, 100, 30, 50, 0),          # unaligned
+])
+def test_mlp(gpu, m, k, hidden, n, group):
+    """fc1 -> SwiGLU -> fc2 against FP64. Gate, up, the activation and the result
+    are rounded to BF16 once each (2^-9 relative at most, |silu'| <= 1.1), so the
+    2-norms differ by at most about 4 * 2^-9."""
+    print(f"[mlp] m={m} k={k} hidden={hidden} n={n} group={group}", flush=True)
+    x = synth.normal_bf16(m + 5, m * k)
+    ws, wv = [], []
+    for seed, rows, cols in ((1, 2 * hidden, k), (2, n, hidden)):
+        if group:
+            gr = min(group, cols)
+            codes, scales = synthetic_q8(m + seed, rows, cols, gr)
+            scales /= 3 * math.sqrt(cols) / 10
+            ws.append(q8_weight(gpu, codes, scales, rows, cols, gr))
+            wide = np.repeat(scales.reshape(rows, -1), gr, axis=1)[:, :cols]
+            wv.append(bf16(synth.f32_to_bf16(codes.reshape(rows, cols).astype(np.float32) * wide)).astype(np.float64))
+        else:
+            bits = synth.normal_bf16(m + seed, rows * cols, scale=1 / math.sqrt(cols))
+            ws.append(gpu.from_bf16(bits))
+            wv.append(bf16(bits).reshape(rows, cols).astype(np.float64))
+    tx, out = gpu.from_bf16(x), gpu.empty(m * n)
+    for _ in range(2):   # the second call finds the workspace in use by the first
+        run(gpu, gpu.lib.h3_gpu_mlp_bf16, out.handle, tx.handle, ws[0].handle, ws[1].handle, m, k, hidden, n)
+    got = bf16(out.read()).reshape(m, n)
+    both = bf16(x).reshape(m, k).astype(np.float64) @ wv[0].T
+    gate, up = both[:, :hidden], both[:, hidden:]
+    want = (gate / (1 + np.exp(-gate)) * up) @ wv[1].T
+    met = metrics(got, want)
+    assert met["rel_l2"] <= 4 * 2.0 ** -9, met
+    for t in (tx, out, *ws):
+        gpu.free(t)
+
+
 def test_bf16_linear_exact_pattern(gpu):
     """tests/quant_native.c:31-50 power-of-two pattern: the BF16 GEMM output must
     equal bf16(exact sum) bit for bit, for several row counts."""
