@@ -145,7 +145,6 @@ struct h3_gpu {
     // Kernel-shape selector for measurement (H3_HIP_ATTENTION_VARIANT): 0 is the
     // default shape, other values pick the alternatives each kernel documents.
     int attention_variant;
-    int gemm_variant;
     char label[64];         // h3_gpu_profile_set_label
     double created;         // wall clock at creation (profile marks)
     bool allocation_failed; // a device allocation ran out of memory
@@ -155,8 +154,7 @@ struct h3_gpu {
     std::vector<std::pair<hipEvent_t, hipEvent_t>> *kernel_events;
     // gemm.hip: BF16 values of the W8A16 weight of the current projection
     // (grow-only; reused by every projection on the compute stream).
-    void *gemm_weights;
-    size_t gemm_weights_bytes;
+    h3_device_buffer gemm_weights;
     h3_device_buffer gemm_partials; // FP32 partial sums of the tiles split over K
     h3_device_buffer mlp_workspace; // h3_gpu_mlp_bf16: activated rows (and the fused product)
     unsigned cus;                   // compute units of the device

@@ -104,7 +104,6 @@ extern "C" h3_gpu *h3_gpu_create(const char *shader_source_path, char *error, si
     g->created = now_seconds();
     g->profiling = getenv("H3_PROFILE") != nullptr;
     if (const char *v = getenv("H3_HIP_ATTENTION_VARIANT")) g->attention_variant = atoi(v);
-    if (const char *v = getenv("H3_HIP_GEMM_VARIANT")) g->gemm_variant = atoi(v);
     // Both streams keep the default priority.
     if ((e = hipStreamCreateWithFlags(&g->compute, hipStreamNonBlocking)) != hipSuccess ||
         (e = hipStreamCreateWithFlags(&g->copy, hipStreamNonBlocking)) != hipSuccess) {
@@ -131,7 +130,7 @@ extern "C" void h3_gpu_free(h3_gpu *g) {
     kernel_events_clear(g);
     delete g->kernel_events;
     if (g->fault) hipFree(g->fault);
-    if (g->gemm_weights) hipFree(g->gemm_weights);
+    h3_buffer_free(&g->gemm_weights);
     h3_buffer_free(&g->gemm_partials);
     h3_buffer_free(&g->mlp_workspace);
     if (g->compute) hipStreamDestroy(g->compute);

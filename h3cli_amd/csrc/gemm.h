@@ -5,6 +5,11 @@
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
+// Epilogue of h3_gemm after the bias. SwiGLU (no bias): the weight holds hidden gate
+// rows, then hidden up rows, n = 2 * hidden, and y is [m, hidden]; only where
+// h3_gemm_swiglu_fits.
+enum { H3_GEMM_PLAIN = 0, H3_GEMM_GELU = 1, H3_GEMM_SWIGLU = 2 };
+
 struct GemmArgs {
     uint16_t *y;
     const uint16_t *x;
@@ -13,8 +18,8 @@ struct GemmArgs {
     const uint16_t *bias;     // optional [N]
     const float *alpha;       // EPI bit 2: device scalar multiplying the accumulator
     unsigned m, n, k, group, groups;
-    int gelu;
-    // gemm_bf16_pipe: tiles [0, full) are whole; each later one is split over K
+    int gelu;                 // H3_GEMM_PLAIN, _GELU or (pipe and mid kernels) _SWIGLU
+    // gemm_bf16_pipe and gemm_mid: tiles [0, full) are whole; each later one is split over K
     // into `split` workgroups, whose FP32 partial sums go to part.
     unsigned full, split;
     float *part;
@@ -49,18 +54,19 @@ __device__ inline void dequant16(const i32x4 &q, float s, bf16x8 *half) {
     }
 }
 
-// Epilogue of h3_gemm after the bias. SwiGLU (no bias): the weight holds hidden gate
-// rows, then hidden up rows, n = 2 * hidden, and y is [m, hidden]; only where
-// h3_gemm_swiglu_fits.
-enum { H3_GEMM_PLAIN = 0, H3_GEMM_GELU = 1, H3_GEMM_SWIGLU = 2 };
 int h3_gemm(h3_gpu *g, uint16_t *y, const uint16_t *x, const h3_gpu_tensor *w, const uint16_t *bias, uint32_t m,
             uint32_t k, uint32_t n, int activation);
-bool h3_gemm_swiglu_fits(const h3_gpu *g, const h3_gpu_tensor *w, uint32_t m, uint32_t k, uint32_t hidden);
+bool h3_gemm_swiglu_fits(const h3_gpu_tensor *w, uint32_t m, uint32_t k, uint32_t hidden);
 
-// gemm_skinny.hip: at most 32 rows. Sums of up to H3_GEMM_SHORT_K products stay with
+// gemm_skinny.hip: at most 16 rows. Sums of up to H3_GEMM_SHORT_K products stay with
 // gemm_small: a chain of that length is short (2 rows, 256 -> 5376: 8.3 us against
 // 3.2), and its sums, in K order, keep the timestep embedding's bits, which every
 // block's modulation depends on.
 constexpr unsigned H3_GEMM_SHORT_K = 256;
 bool h3_gemm_skinny_fits(const GemmArgs &a, bool q8);
 int h3_gemm_skinny(h3_gpu *g, const GemmArgs &a, bool q8);
+
+// gemm_mid.hip: row tiles of tm = 64, 128 or 256, the last wave of tiles in split
+// shares of K.
+bool h3_gemm_mid_fits(const GemmArgs &a, bool q8);
+int h3_gemm_mid(h3_gpu *g, const GemmArgs &a, bool q8, unsigned tm, unsigned split, bool timed = true);

@@ -8,29 +8,19 @@
 // (src/metal/shaders.metal:799-855): every weight is reconstructed as
 // w = bf16(code * scale) and multiplied in FP32 accumulation, bf16 output (+bias).
 //
-// MI355X design:
-//  * C^T = W . X^T on v_mfma_f32_32x32x16_bf16, so a lane owns one output row and
-//    four consecutive columns per register group (8-byte row-major stores);
-//  * 256 x 256 output tile per workgroup of 8 waves (each 128 x 64, 8
-//    accumulator blocks, two waves per SIMD), K staged 64 at a time, double
-//    buffered in LDS, operand fragments of the next k-step read during MFMAs;
-//  * X tiles go global -> LDS directly (global_load_lds_dwordx4, XOR-swizzled
-//    16-byte chunks); int8 weight tiles are loaded into registers one tile ahead,
-//    dequantized in registers (w = bf16(code * scale)) and written to LDS as BF16,
-//    so each weight is converted once per workgroup, not per wave;
-//  * tile ids are XCD-remapped and grouped along M so that the workgroups an XCD
-//    runs together share weight columns in its L2;
-//  * per-channel q8 (group == K) runs gemm_q8_staged: the int8 tile two steps
-//    ahead goes straight to LDS, and the next step's dequantization shares a
-//    basic block with this step's MFMAs, so its VALU work issues between them.
-// Shapes with K % 128 == 0 and N % 256 == 0 (every DiT projection) run
-// gemm_bf16_pipe instead: a hand-scheduled K loop at one wave per SIMD (see
-// its comment). For W8A16 weights a dequantization pass first writes
-// w = bf16(code * scale) for the whole weight into a BF16 buffer of the
-// context (in registers, 16 codes per thread: the same reconstruction as
-// above), which costs about 1% of the GEMM at M = 32400 and leaves the MFMA
-// loop free of VALU work. gemm_q8_staged and gemm_kernel remain for the other
-// shapes (and as H3_HIP_GEMM_VARIANT=3 for comparison).
+// Kernels, chosen per call (choose(), at the end):
+//  * gemm_bf16_pipe, here: a hand-scheduled K loop at one wave per SIMD (see its
+//    comment), for many rows. For W8A16 weights a conversion pass first writes
+//    w = bf16(code * scale) for the whole weight into a BF16 buffer of the context
+//    (in registers, 16 codes per thread), which costs about 1% of the GEMM at
+//    M = 32400 and leaves the MFMA loop free of VALU work;
+//  * gemm_mid.hip: fewer rows, any N, int8 weights converted in the kernel;
+//  * gemm_skinny.hip: at most 16 rows;
+//  * gemm_small, here: any shape.
+// Both tiled kernels compute C^T = W . X^T, so a lane owns one output row and
+// consecutive columns, move operands global -> LDS directly (XOR-swizzled 16-byte
+// chunks), and remap tile ids so that the workgroups an XCD runs together share
+// weight columns in its L2.
 #include "common.h"
 #include "internal.h"
 #include "gemm.h"
@@ -44,399 +34,15 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 constexpr int TM = 256, TN = 256, TK = 64;
 constexpr int ROW_BYTES = TK * 2;               // 128 B per BF16 tile row
 constexpr int TILE_BYTES = 256 * ROW_BYTES;     // 32 KB per operand tile
-constexpr int STAGE = 2 * TILE_BYTES;           // X tile + W tile
-constexpr int GROUP_M = 8;                      // tile rows per grouped band
 
 // 16-byte chunk swizzle of a 128-byte LDS row. A ds_read_b128 serves sixteen
 // lanes (sixteen consecutive rows) per cycle across 256 bytes of banks: rows
 // 2i and 2i+1 sit in different halves, and (row >> 1) & 7 spreads the eight
-// pairs over eight chunks. Writes are served eight lanes per cycle across 128
-// bytes; the weight store therefore gives eight consecutive lanes eight rows
-// of the same parity (see w_row).
+// pairs over eight chunks.
 __device__ inline unsigned swz(unsigned row, unsigned ch) { return ch ^ ((row >> 1) & 7); }
 
-// Weight staging map: chunk c (0..1023) of a 256 x 64 int8 tile -> (row, part).
-// A wave covers 16 rows x 4 parts; lanes 8i..8i+7 of a part take rows of one
-// parity, so their LDS stores hit eight different chunks.
-__device__ inline unsigned w_row(unsigned c) { const unsigned l = c % 16; return (c / 64) * 16 + 2 * (l % 8) + l / 8; }
-__device__ inline unsigned w_part(unsigned c) { return (c / 16) % 4; }
-
-// WM x WN waves; each wave owns a (256 / WM) x (256 / WN) output tile of
-// 32 x 32 MFMA blocks. 2 x 4 waves (128 x 64 per wave, two waves per SIMD) or
-// 2 x 2 waves (128 x 128 per wave, one wave per SIMD: the 256 accumulator
-// registers sit in AGPRs, and each fragment read from LDS feeds four MFMAs
-// instead of two or four). CHANNEL: one scale per output row (group == K),
-// loaded once. EPI bit 0: bias, bit 1: GELU, bit 2: alpha (before the bias).
-template <bool Q8, bool CHANNEL, int EPI, int WM = 2, int WN = 4>
-__global__ __attribute__((amdgpu_flat_work_group_size(64 * WM * WN, 64 * WM * WN),
-                          amdgpu_waves_per_eu(WM * WN / 4, WM * WN / 4)))
-void gemm_kernel(GemmArgs a) {
-    constexpr int T = 64 * WM * WN;            // threads
-    constexpr int NBM = TM / WM / 32, NBN = TN / WN / 32;
-    constexpr int WCH = 1024 / T;              // weight chunks per thread
-    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
-    const unsigned tid = threadIdx.x, wave = tid / 64, lane = tid % 64, n32 = lane % 32, hf = lane / 32;
-    const unsigned tiles_m = (a.m + TM - 1) / TM, tiles_n = a.n / TN;
-    // XCD-aware id, then grouped ordering: GROUP_M tile rows sweep the columns together.
-    const unsigned pid = xcd_remap(blockIdx.x, gridDim.x);
-    const unsigned band = pid / (GROUP_M * tiles_n), first_m = band * GROUP_M;
-    const unsigned rows_in_band = min(tiles_m - first_m, (unsigned)GROUP_M);
-    const unsigned tm = first_m + (pid % (GROUP_M * tiles_n)) % rows_in_band;
-    const unsigned tn = (pid % (GROUP_M * tiles_n)) / rows_in_band;
-    const unsigned m0 = tm * TM, n0 = tn * TN;
-    const unsigned wm = wave / WN, wn = wave % WN;   // wave rows m0 + wm*32*NBM, columns n0 + wn*32*NBN
-    const unsigned ksteps = a.k / TK;
-
-    f32x16 acc[NBN][NBM];   // [n block][m block], C^T layout: lane = output row, regs = columns
-#pragma unroll
-    for (int i = 0; i < NBN; i++)
-#pragma unroll
-        for (int j = 0; j < NBM; j++) acc[i][j] = f32x16{};
-
-    // Weight staging (q8): 256 rows x 64 int8 = 1024 16-byte chunks, WCH per thread.
-    i32x4 wq[WCH];
-    float wscale[WCH];
-    if constexpr (Q8 && CHANNEL) {
-#pragma unroll
-        for (int j = 0; j < WCH; j++) wscale[j] = a.scales[n0 + w_row(tid + T * j)];
-    }
-    auto load_w = [&](unsigned kt) {
-        if constexpr (Q8) {
-            const int8_t *w8 = reinterpret_cast<const int8_t *>(a.w);
-#pragma unroll
-            for (int j = 0; j < WCH; j++) {
-                unsigned c = tid + T * j, row = w_row(c), part = w_part(c);
-                wq[j] = *reinterpret_cast<const i32x4 *>(w8 + (size_t)(n0 + row) * a.k + kt * TK + part * 16);
-                if constexpr (!CHANNEL)
-                    wscale[j] = a.scales[(size_t)(n0 + row) * a.groups + (kt * TK + part * 16) / a.group];
-            }
-        }
-    };
-    auto x_stage = [&](int stage) { return lds + stage * STAGE; };
-    auto w_stage = [&](int stage) { return lds + stage * STAGE + TILE_BYTES; };
-    auto store_w = [&](int stage) {
-        if constexpr (Q8) {
-            uint8_t *ws = w_stage(stage);
-#pragma unroll
-            for (int j = 0; j < WCH; j++) {
-                unsigned c = tid + T * j, row = w_row(c), part = w_part(c);
-                bf16x8 half[2];
-#pragma unroll
-                for (int e = 0; e < 16; e += 2) {
-                    int word = wq[j][e / 4];
-                    f32x2 f = {(float)(int8_t)(word >> (8 * (e % 4))) * wscale[j],
-                               (float)(int8_t)(word >> (8 * (e % 4 + 1))) * wscale[j]};
-                    bf16x2 b = __builtin_convertvector(f, bf16x2);
-                    half[e / 8][e % 8] = b[0];
-                    half[e / 8][e % 8 + 1] = b[1];
-                }
-                *reinterpret_cast<bf16x8 *>(ws + row * ROW_BYTES + swz(row, part * 2) * 16) = half[0];
-                *reinterpret_cast<bf16x8 *>(ws + row * ROW_BYTES + swz(row, part * 2 + 1) * 16) = half[1];
-            }
-        }
-    };
-    // Direct global -> LDS loads: X rows (clamped at M) and, for BF16 weights, W rows.
-    auto load_direct = [&](unsigned kt, int stage) {
-        uint8_t *xs = x_stage(stage);
-#pragma unroll
-        for (unsigned b = wave; b < 32; b += WM * WN) {
-            unsigned row = 8 * b + lane / 8, ph = lane % 8;
-            unsigned gm = min(m0 + row, a.m - 1);
-            const uint16_t *src = a.x + (size_t)gm * a.k + kt * TK + swz(row, ph) * 8;
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
-                                             (__attribute__((address_space(3))) void *)(xs + b * 1024), 16, 0, 0);
-            if constexpr (!Q8) {
-                const uint16_t *wsrc = reinterpret_cast<const uint16_t *>(a.w) + (size_t)(n0 + row) * a.k + kt * TK + swz(row, ph) * 8;
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)wsrc,
-                                                 (__attribute__((address_space(3))) void *)(xs + TILE_BYTES + b * 1024), 16, 0, 0);
-            }
-        }
-    };
-    auto frags = [&](const uint8_t *xs, const uint8_t *ws, int ks, bf16x8 *wf, bf16x8 *xf) {
-#pragma unroll
-        for (int i = 0; i < NBN; i++) {
-            unsigned wr = wn * 32 * NBN + i * 32 + n32;
-            wf[i] = *reinterpret_cast<const bf16x8 *>(ws + wr * ROW_BYTES + swz(wr, ks * 2 + hf) * 16);
-        }
-#pragma unroll
-        for (int j = 0; j < NBM; j++) {
-            unsigned xr = wm * 32 * NBM + j * 32 + n32;
-            xf[j] = *reinterpret_cast<const bf16x8 *>(xs + xr * ROW_BYTES + swz(xr, ks * 2 + hf) * 16);
-        }
-    };
-
-    {
-    load_direct(0, 0);
-    load_w(0);
-    store_w(0);
-    wait_vm_loads();
-    __syncthreads();
-
-    for (unsigned kt = 0; kt < ksteps; kt++) {
-        const int cur = kt & 1;
-        const bool more = kt + 1 < ksteps;
-        if (more) { load_direct(kt + 1, cur ^ 1); load_w(kt + 1); }
-        const uint8_t *xs = x_stage(cur);
-        const uint8_t *ws = w_stage(cur);
-        // Fragments of k-step ks+1 are read while the MFMAs of ks run.
-        bf16x8 wf[2][NBN], xf[2][NBM];
-        frags(xs, ws, 0, wf[0], xf[0]);
-#pragma unroll
-        for (int ks = 0; ks < TK / 16; ks++) {
-            if (ks + 1 < TK / 16) frags(xs, ws, ks + 1, wf[(ks + 1) & 1], xf[(ks + 1) & 1]);
-#pragma unroll
-            for (int i = 0; i < NBN; i++)
-#pragma unroll
-                for (int j = 0; j < NBM; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[ks & 1][i], xf[ks & 1][j], acc[i][j], 0, 0, 0);
-        }
-        if (more) store_w(cur ^ 1);
-        wait_vm_loads();
-        __syncthreads();
-    }
-    }
-
-    // Epilogue: lane holds output row m = m0 + wm*32*NBM + j*32 + n32 and columns
-    // n0 + wn*32*NBN + i*32 + g*8 + hf*4 + 0..3 for register group g.
-#pragma unroll
-    for (int j = 0; j < NBM; j++) {
-        const unsigned row = m0 + wm * 32 * NBM + j * 32 + n32;
-        if (row >= a.m) continue;
-        uint16_t *dst = a.y + (size_t)row * a.n;
-#pragma unroll
-        for (int i = 0; i < NBN; i++)
-#pragma unroll
-            for (int g4 = 0; g4 < 4; g4++) {
-                const unsigned col = n0 + wn * 32 * NBN + i * 32 + g4 * 8 + hf * 4;
-                u16x4 out;
-                u16x4 bias4 = {};
-                if constexpr (EPI & 1) bias4 = *reinterpret_cast<const u16x4 *>(a.bias + col);
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    float v = acc[i][j][g4 * 4 + e];
-                    if constexpr (EPI & 4) v *= a.alpha[0];
-                    if constexpr (EPI & 1) v += bf16_to_f32(bias4[e]);
-                    uint16_t b = f32_to_bf16(v);
-                    if constexpr (EPI & 2) b = f32_to_bf16(gelu_tanh(bf16_to_f32(b)));
-                    out[e] = b;
-                }
-                *reinterpret_cast<u16x4 *>(dst + col) = out;
-            }
-    }
-}
-
-// W8A16 with the int8 weight tile staged in LDS: 8 waves (2 x 4, 128 x 64
-// per wave, two per SIMD) as gemm_kernel, but the int8 tile of step kt + 2 is
-// fetched straight into LDS (buffer_load ... lds) during step kt, and the
-// dequantization of step kt + 1 (LDS int8 -> registers -> BF16 LDS tile) runs
-// in the same basic block as step kt's MFMAs, so its VALU work can issue
-// between them instead of after them. No register is held across a step for
-// the weights. LDS: two stages of X and BF16 W (128 KB) plus two int8 stages
-// (32 KB). X rows past M load zeros (BUFFER_OOB lane offsets); W8 rows never
-// pass N, a multiple of 256.
-constexpr int W8_BYTES = 256 * TK;                  // 16 KB int8 tile
-// Per-output-channel scales (group == K) only: they are loaded once.
-template <int EPI>
-__global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2)))
-void gemm_q8_staged(GemmArgs a) {
-    constexpr int WM = 2, WN = 4, T = 512;
-    constexpr int NBM = TM / WM / 32, NBN = TN / WN / 32;
-    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
-    uint8_t *const w8s = lds + 2 * STAGE;
-    // wave is read as a uniform value, so LDS destinations and buffer offsets
-    // stay scalar (no waterfall loop around the buffer loads).
-    const unsigned tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
-    const unsigned n32 = lane % 32, hf = lane / 32;
-    const unsigned tiles_m = (a.m + TM - 1) / TM, tiles_n = a.n / TN;
-    const unsigned pid = xcd_remap(blockIdx.x, gridDim.x);
-    const unsigned band = pid / (GROUP_M * tiles_n), first_m = band * GROUP_M;
-    const unsigned rows_in_band = min(tiles_m - first_m, (unsigned)GROUP_M);
-    const unsigned tm = first_m + (pid % (GROUP_M * tiles_n)) % rows_in_band;
-    const unsigned tn = (pid % (GROUP_M * tiles_n)) / rows_in_band;
-    const unsigned m0 = __builtin_amdgcn_readfirstlane(tm * TM), n0 = __builtin_amdgcn_readfirstlane(tn * TN);
-    const unsigned wm = wave / WN, wn = wave % WN;
-    const unsigned ksteps = a.k / TK;
-
-    const __amdgpu_buffer_rsrc_t xr =
-        __builtin_amdgcn_make_buffer_rsrc((void *)a.x, (short)0, (int)((size_t)a.m * a.k * 2), 0x00020000);
-    const __amdgpu_buffer_rsrc_t wr =
-        __builtin_amdgcn_make_buffer_rsrc((void *)a.w, (short)0, (int)((size_t)a.n * a.k), 0x00020000);
-    // X block b = wave + 8 t: rows 8 b + lane / 8, 16-byte chunk lane % 8
-    // (swizzled); the swizzle does not depend on t, so one lane offset serves
-    // all four loads.
-    const uint32_t xoff = ((8 * wave + lane / 8) * a.k + swz(8 * wave + lane / 8, lane % 8) * 8) * 2;
-    // Weight chunks c = tid + 512 j: row w_row(c) = w_row(tid) + 128 j, part w_part(tid).
-    const unsigned wrow = w_row(tid), wpart = w_part(tid);
-    const uint32_t woff = wrow * a.k + wpart * 16;
-
-    f32x16 acc[NBN][NBM];
-#pragma unroll
-    for (int i = 0; i < NBN; i++)
-#pragma unroll
-        for (int j = 0; j < NBM; j++) acc[i][j] = f32x16{};
-
-    float wscale[2];
-#pragma unroll
-    for (int j = 0; j < 2; j++) wscale[j] = a.scales[n0 + wrow + 128 * j];
-    // Loads of step kt's data into the stages of step `at` (the step numbers
-    // of the stages are unclamped, so a clamped reload never lands in a stage
-    // that the current step reads).
-    // In the last row tile, lanes whose row is at or past M take BUFFER_OOB
-    // and load zeros (those output rows are not stored).
-    const bool m_tail = m0 + TM > a.m;
-    // TAIL: compiled in only for the last row tile's loop.
-    auto load_x = [&](unsigned kt, unsigned at, auto tail_tag) {
-        constexpr bool TAIL = decltype(tail_tag)::value;
-        uint8_t *xs = lds + (at & 1) * STAGE;
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            auto *dst = (__attribute__((address_space(3))) void *)(xs + (wave + 8 * t) * 1024);
-            const uint32_t so = (uint32_t)(((size_t)m0 + 64 * t) * a.k * 2 + kt * TK * 2);
-            if constexpr (TAIL) {
-                const unsigned row = m0 + 64 * t + 8 * wave + lane / 8;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, dst, 16, row < a.m ? xoff : BUFFER_OOB, so, 0, 0);
-            } else {
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, dst, 16, xoff, so, 0, 0);
-            }
-        }
-    };
-    auto load_w8 = [&](unsigned kt, unsigned at) {
-        uint8_t *ws8 = w8s + (at & 1) * W8_BYTES;
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                wr, (__attribute__((address_space(3))) void *)(ws8 + (wave + 8 * j) * 1024), 16, woff,
-                (uint32_t)(((size_t)n0 + 128 * j) * a.k + kt * TK), 0, 0);
-    };
-    // int8 chunks of stage `at` (this thread's own two) -> BF16 W stage at & 1.
-    auto dequant = [&](unsigned at) {
-        const uint8_t *ws8 = w8s + (at & 1) * W8_BYTES;
-        uint8_t *ws = lds + (at & 1) * STAGE + TILE_BYTES;
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const i32x4 q = *reinterpret_cast<const i32x4 *>(ws8 + (tid + T * j) * 16);
-            const unsigned row = wrow + 128 * j;
-            bf16x8 half[2];
-#pragma unroll
-            for (int e = 0; e < 16; e += 2) {
-                int word = q[e / 4];
-                f32x2 f = {(float)(int8_t)(word >> (8 * (e % 4))) * wscale[j],
-                           (float)(int8_t)(word >> (8 * (e % 4 + 1))) * wscale[j]};
-                bf16x2 b = __builtin_convertvector(f, bf16x2);
-                half[e / 8][e % 8] = b[0];
-                half[e / 8][e % 8 + 1] = b[1];
-            }
-            *reinterpret_cast<bf16x8 *>(ws + row * ROW_BYTES + swz(row, wpart * 2) * 16) = half[0];
-            *reinterpret_cast<bf16x8 *>(ws + row * ROW_BYTES + swz(row, wpart * 2 + 1) * 16) = half[1];
-        }
-    };
-    auto frags = [&](const uint8_t *xs, const uint8_t *ws, int ks, bf16x8 *wf, bf16x8 *xf) {
-#pragma unroll
-        for (int i = 0; i < NBN; i++) {
-            unsigned wr_ = wn * 32 * NBN + i * 32 + n32;
-            wf[i] = *reinterpret_cast<const bf16x8 *>(ws + wr_ * ROW_BYTES + swz(wr_, ks * 2 + hf) * 16);
-        }
-#pragma unroll
-        for (int j = 0; j < NBM; j++) {
-            unsigned xr_ = wm * 32 * NBM + j * 32 + n32;
-            xf[j] = *reinterpret_cast<const bf16x8 *>(xs + xr_ * ROW_BYTES + swz(xr_, ks * 2 + hf) * 16);
-        }
-    };
-
-    // Prologue: X(0), W8(0), W8(1); W(0) dequantized.
-    if (m_tail) load_x(0, 0, std::true_type{});
-    else load_x(0, 0, std::false_type{});
-    load_w8(0, 0);
-    load_w8(min(1u, ksteps - 1), 1);
-    wait_vm_loads();
-    __syncthreads();
-    dequant(0);
-    __syncthreads();
-
-    // The K loop, instantiated for the last row tile and for the others.
-    // Fragments are read one sub-step ahead of their MFMAs; in the last
-    // sub-step the barrier comes first and the next tile's first fragments are
-    // read before this sub-step's MFMAs, so their LDS latency sits under them
-    // (after the last tile those reads land in registers nobody uses). The
-    // sched_barrier keeps hipcc from sinking the reads below the MFMAs.
-    auto kloop = [&](auto tail_tag) {
-    bf16x8 wf[2][NBN], xf[2][NBM];
-    frags(lds, lds + TILE_BYTES, 0, wf[0], xf[0]);
-    for (unsigned kt = 0; kt < ksteps; kt++) {
-        const unsigned k1 = min(kt + 1, ksteps - 1), k2 = min(kt + 2, ksteps - 1);
-        load_x(k1, kt + 1, tail_tag);
-        load_w8(k2, kt + 2);
-        const uint8_t *xs = lds + (kt & 1) * STAGE;
-        const uint8_t *ws = xs + TILE_BYTES;
-#pragma unroll
-        for (int ks = 0; ks < TK / 16; ks++) {
-            if (ks + 1 < TK / 16) {
-                frags(xs, ws, ks + 1, wf[(ks + 1) & 1], xf[(ks + 1) & 1]);
-            } else {
-                wait_vm_loads();
-                __syncthreads();
-                const uint8_t *nx = lds + ((kt + 1) & 1) * STAGE;
-                frags(nx, nx + TILE_BYTES, 0, wf[0], xf[0]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int i = 0; i < NBN; i++)
-#pragma unroll
-                for (int j = 0; j < NBM; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[ks & 1][i], xf[ks & 1][j], acc[i][j], 0, 0, 0);
-            if (ks == 0) dequant(kt + 1);
-        }
-    }
-    };
-    if (m_tail) kloop(std::true_type{});
-    else kloop(std::false_type{});
-
-#pragma unroll
-    for (int j = 0; j < NBM; j++) {
-        const unsigned row = m0 + wm * 32 * NBM + j * 32 + n32;
-        if (row >= a.m) continue;
-        uint16_t *dst = a.y + (size_t)row * a.n;
-#pragma unroll
-        for (int i = 0; i < NBN; i++)
-#pragma unroll
-            for (int g4 = 0; g4 < 4; g4++) {
-                const unsigned col = n0 + wn * 32 * NBN + i * 32 + g4 * 8 + hf * 4;
-                u16x4 out;
-                u16x4 bias4 = {};
-                if constexpr (EPI & 1) bias4 = *reinterpret_cast<const u16x4 *>(a.bias + col);
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    float v = acc[i][j][g4 * 4 + e];
-                    if constexpr (EPI & 1) v += bf16_to_f32(bias4[e]);
-                    uint16_t b = f32_to_bf16(v);
-                    if constexpr (EPI & 2) b = f32_to_bf16(gelu_tanh(bf16_to_f32(b)));
-                    out[e] = b;
-                }
-                *reinterpret_cast<u16x4 *>(dst + col) = out;
-            }
-    }
-}
-
-template <int EPI>
-int launch_staged(h3_gpu *g, const GemmArgs &a) {
-    constexpr size_t shared = 2 * STAGE + 2 * W8_BYTES;
-    static bool configured = false;
-    auto kernel = gemm_q8_staged<EPI>;
-    if (!configured) {
-        if (!h3_hip_check(g, hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 (int)shared), "GEMM shared memory"))
-            return 0;
-        configured = true;
-    }
-    unsigned tiles = (a.m + TM - 1) / TM * (a.n / TN);
-    hipEvent_t timing = h3_kernel_timing_begin(g);
-    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(512), shared, g->compute, a);
-    h3_kernel_timing_end(g, timing);
-    return h3_launch_status(g, "W8A16 GEMM");
-}
-
 // ------------------------------------------------------------ hand-scheduled BF16 GEMM
-// gemm_bf16_pipe: the same 256 x 256 output tile as gemm_kernel, computed by
+// gemm_bf16_pipe: a 256 x 256 output tile per workgroup, computed by
 // four waves of 128 x 128 (one per SIMD, 2 x 2) on v_mfma_f32_16x16x32_bf16,
 // each wave with 8 x 8 accumulator blocks of 16 x 16 in AGPRs, so one
 // fragment read from LDS feeds eight MFMAs. (The same loop on 32 x 32 x 16
@@ -754,32 +360,8 @@ __global__ __launch_bounds__(256) void gemm_pipe_reduce(GemmArgs a) {
     pipe_store<EPI>(a, row, n0 + (wave % 2) * 128, q4, block);
 }
 
-// How many K shares the tiles of the last, incomplete wave of workgroups get (1:
-// none). Modelled time of that wave in microseconds: 1.3 per 64 values of K, 2 per
-// workgroup, 0.13 per share for its 256 KB of partial sums written and read, and
-// 3 plus 0.9 for each share added in turn by the reduction launch. Measured,
-// BF16 weights, in microseconds, unsplit against the shares taken here: 63 tiles
-// (729 rows, 7168 -> 5376) 134.6, 4 shares 66.6; the same with K = 14336 312.7, 4
-// shares 111.3; 100 tiles (1200 rows, 13824 -> 5120) 291.9, 2 shares 173.1; 3 tiles
-// (729 rows, 5376 -> 256) 86.8, 8 shares 25.8; 336 tiles (729 rows, 5376 -> 28672),
-// the last 80 split, 242.6, 3 shares 201.8. Where the last wave is two thirds full
-// nothing is gained (693 tiles, 14336 -> 5376: 998, 2 shares 1018; 224 tiles,
-// 5376 -> 28672: 145.1, 2 shares 171.1). At most 512 shares (128 MB).
-unsigned pipe_split(const h3_gpu *g, unsigned tiles, unsigned k) {
-    const unsigned rest = tiles % g->cus, pairs = k / (2 * TK);
-    if (!rest) return 1;
-    unsigned best = 1;
-    float least = pairs * 2.6f + 2.f;
-    for (unsigned s = 2; s <= 32 && s <= pairs && rest * s <= 512; s++) {
-        const float waves = (float)((rest * s + g->cus - 1) / g->cus);
-        const float t = waves * ((pairs + s - 1) / s * 2.6f + 2.f) + rest * s * 0.13f + 3.f + 0.9f * s;
-        if (t < least) { least = t; best = s; }
-    }
-    return best;
-}
-
 template <int EPI>
-int launch_pipe(h3_gpu *g, GemmArgs a, bool timed = true) {
+int launch_pipe(h3_gpu *g, GemmArgs a, unsigned split, bool timed) {
     constexpr size_t shared = PIPE_LDS;
     static bool configured = false;
     if (!configured) {
@@ -791,7 +373,7 @@ int launch_pipe(h3_gpu *g, GemmArgs a, bool timed = true) {
     }
     const unsigned tiles = (a.m + TM - 1) / TM * (a.n / TN);
     unsigned rest = tiles % g->cus;
-    a.split = pipe_split(g, tiles, a.k);
+    a.split = split;
     if (a.split > 1 && !h3_buffer_try(g, &g->gemm_partials, (size_t)rest * a.split * TM * TN * 4)) a.split = 1;
     if (a.split == 1) rest = 0;
     a.full = tiles - rest;
@@ -812,19 +394,20 @@ bool pipe_fits(const GemmArgs &a) {
     return a.n % TN == 0 && a.k % (2 * TK) == 0 && a.m >= 32 && (size_t)a.m * a.k * 2 < (1ull << 31) &&
            (size_t)a.n * a.k * 2 < (1ull << 31);
 }
-int launch_pipe_epi(h3_gpu *g, const GemmArgs &a, int epi, bool timed = true) {
+// epi: bit 0 bias, 1 GELU, 2 alpha, 3 SwiGLU.
+int launch_pipe_epi(h3_gpu *g, const GemmArgs &a, int epi, unsigned split, bool timed) {
     switch (epi) {
-    case 0: return launch_pipe<0>(g, a, timed);
-    case 1: return launch_pipe<1>(g, a, timed);
-    case 2: return launch_pipe<2>(g, a, timed);
-    case 3: return launch_pipe<3>(g, a, timed);
-    case 8: return launch_pipe<8>(g, a, timed);
-    default: return launch_pipe<4>(g, a, timed);
+    case 0: return launch_pipe<0>(g, a, split, timed);
+    case 1: return launch_pipe<1>(g, a, split, timed);
+    case 2: return launch_pipe<2>(g, a, split, timed);
+    case 3: return launch_pipe<3>(g, a, split, timed);
+    case 8: return launch_pipe<8>(g, a, split, timed);
+    default: return launch_pipe<4>(g, a, split, timed);
     }
 }
 
 // W8A16 weights -> BF16 values w = bf16(code * scale[row, k / group]), the
-// reconstruction of gemm_kernel and of the reference's Metal kernel
+// reconstruction of gemm_mid and of the reference's Metal kernel
 // (shaders.metal:825-827), written once per projection call for
 // gemm_bf16_pipe. HBM-bound: each thread reads 16 codes (one 16-byte load)
 // and writes 32 bytes. group is a multiple of 16, so one scale covers them.
@@ -864,7 +447,7 @@ __global__ __launch_bounds__(256) void gemm_small(GemmArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t ws[64 * SMALL_ROW];
     __shared__ __attribute__((aligned(16))) float xs[4 * SMALL_R][SMALL_K];
     const unsigned tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-    const unsigned n0 = blockIdx.x * 64, m0 = blockIdx.y * 4 * SMALL_R, col = n0 + lane;
+    const unsigned n0 = blockIdx.y * 64, m0 = blockIdx.x * 4 * SMALL_R, col = n0 + lane;
     float acc[SMALL_R] = {};
     for (unsigned k0 = 0; k0 < a.k; k0 += SMALL_K) {
         const unsigned kn = min(SMALL_K, a.k - k0);
@@ -940,7 +523,7 @@ __global__ __launch_bounds__(256) void gemm_small(GemmArgs a) {
 
 int launch_small(h3_gpu *g, const GemmArgs &a, bool q8) {
     const bool vec = a.k % 8 == 0 && (!q8 || a.group % 8 == 0);
-    const dim3 grid((a.n + 63) / 64, (a.m + 4 * SMALL_R - 1) / (4 * SMALL_R));
+    const dim3 grid((a.m + 4 * SMALL_R - 1) / (4 * SMALL_R), (a.n + 63) / 64);
     if (q8 && vec) hipLaunchKernelGGL((gemm_small<true, true>), grid, dim3(256), 0, g->compute, a);
     else if (q8) hipLaunchKernelGGL((gemm_small<true, false>), grid, dim3(256), 0, g->compute, a);
     else if (vec) hipLaunchKernelGGL((gemm_small<false, true>), grid, dim3(256), 0, g->compute, a);
@@ -948,55 +531,93 @@ int launch_small(h3_gpu *g, const GemmArgs &a, bool q8) {
     return h3_launch_status(g, "small GEMM");
 }
 
-template <bool Q8, bool CHANNEL, int EPI, int WM = 2, int WN = 4>
-int launch_tiled(h3_gpu *g, const GemmArgs &a) {
-    constexpr size_t shared = 2 * STAGE;
-    static bool configured = false;
-    auto kernel = gemm_kernel<Q8, CHANNEL, EPI, WM, WN>;
-    if (!configured) {
-        if (!h3_hip_check(g, hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 (int)shared), "GEMM shared memory"))
-            return 0;
-        configured = true;
+// ------------------------------------------------------------ choice of the kernel
+struct Plan {
+    float us;             // modelled time
+    unsigned tm;          // row tile of gemm_mid, 0: gemm_bf16_pipe
+    unsigned split;       // K shares of each tile of the last, incomplete wave
+    bool dequant;         // W8A16: convert the whole weight to BF16 first
+};
+
+// Modelled time in microseconds of tiles output tiles of `units` K units, unit_us
+// each: 2 more per workgroup, share_us per share of a split tile for its partial sums
+// written and read, 3 for the reduction launch and 0.9 for each share added in turn.
+// At most `most` shares (128 MB).
+Plan last_wave(const h3_gpu *g, unsigned tiles, unsigned units, float unit_us, float share_us, unsigned most) {
+    const unsigned rest = tiles % g->cus;
+    Plan p{(float)(tiles / g->cus) * (units * unit_us + 2.f), 0, 1, false};
+    if (!rest) return p;
+    float least = units * unit_us + 2.f;
+    for (unsigned s = 2; s <= 32 && s <= units && rest * s <= most; s++) {
+        const float waves = (float)((rest * s + g->cus - 1) / g->cus);
+        const float t = waves * ((units + s - 1) / s * unit_us + 2.f) + rest * s * share_us + 3.f + 0.9f * s;
+        if (t < least) { least = t; p.split = s; }
     }
-    unsigned tiles = (a.m + TM - 1) / TM * (a.n / TN);
-    hipEvent_t timing = h3_kernel_timing_begin(g);
-    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(64 * WM * WN), shared, g->compute, a);
-    h3_kernel_timing_end(g, timing);
-    return h3_launch_status(g, Q8 ? "W8A16 GEMM" : "BF16 GEMM");
+    p.us += least;
+    return p;
 }
 
-template <bool Q8, bool CHANNEL>
-int launch_epi(h3_gpu *g, const GemmArgs &a) {
-    const int epi = (a.bias ? 1 : 0) | (a.gelu ? 2 : 0);
-    if constexpr (Q8 && CHANNEL) {
-        // Per-channel W8A16 (the synthetic DiT): int8 tiles
-        // staged in LDS (buffer offsets are 32-bit). Variant 2 keeps the
-        // register-staged weights of gemm_kernel (3-4% slower on config 4).
-        if (g->gemm_variant != 2 && (size_t)a.m * a.k * 2 < (1ull << 31) && (size_t)a.n * a.k < (1ull << 31)) {
-            switch (epi) {
-            case 0: return launch_staged<0>(g, a);
-            case 1: return launch_staged<1>(g, a);
-            case 2: return launch_staged<2>(g, a);
-            default: return launch_staged<3>(g, a);
-            }
+// The faster of the kernels that take this projection, by the model above with these
+// rates (microseconds per 64 values of K, one workgroup on each CU, measured at 64 to
+// 8193 rows): pipe 1.5; mid, BF16 weights 1.0 / 1.2 / 1.95 for 64 / 128 / 256 rows;
+// mid, int8 weights 1.3 / 1.25 / 2.1; converting a weight to BF16 first 0.5 per million
+// values. Measured, in microseconds, the runner-up in brackets: 63 tiles of 256
+// (729 rows, 7168 -> 5376), BF16: pipe in 4 shares 66.6 (unsplit 134.6); 336 tiles
+// (729 rows, 5376 -> 28672), BF16: pipe, the last 80 tiles in 3 shares, 201.8 (242.6);
+// 693 tiles (8193 rows, 14336 -> 5376): unsplit 998 (2 shares 1018); 729 rows,
+// 5376 -> 28672, int8: mid 256 in 3 shares 247 (pipe 287); 1200 rows, 13824 -> 5120,
+// int8: pipe in 2 shares 209 (mid 202); 2000 rows, 5120 -> 5120, int8: pipe 116 (mid
+// 140); 300 rows, 7168 -> 5376, BF16: mid 128 in 4 shares 38.7 (pipe 50.9); 8193 rows,
+// 5440 -> 5120, int8, which pipe does not take: converted first 442 (mid 475).
+Plan choose(const h3_gpu *g, const GemmArgs &a, bool q8) {
+    static constexpr float BF16_STEP[3] = {1.0f, 1.2f, 1.95f}, Q8_STEP[3] = {1.3f, 1.25f, 2.1f};
+    Plan best{3.4e38f, 0, 1, false};
+    const bool pipe = pipe_fits(a);
+    const float convert = q8 ? (float)a.n * a.k * 0.5e-6f + 4.f : 0.f;
+    auto consider = [&](Plan p, unsigned tm, bool dequant) {
+        p.tm = tm;
+        p.dequant = dequant;
+        if (dequant) p.us += convert;
+        if (p.us < best.us) best = p;
+    };
+    if (pipe) consider(last_wave(g, (a.m + TM - 1) / TM * (a.n / TN), a.k / (2 * TK), 3.0f, 0.09f, 512), 0, q8);
+    if (h3_gemm_mid_fits(a, q8))
+        for (unsigned i = 0; i < 3; i++) {
+            const unsigned tm = 64u << i, tiles = (a.m + tm - 1) / tm * ((a.n + TN - 1) / TN);
+            const float share = 0.09f * tm / 256;
+            if (q8) consider(last_wave(g, tiles, a.k / TK, Q8_STEP[i], share, 512 * 256 / tm), tm, false);
+            if (i < 2 || !pipe) consider(last_wave(g, tiles, a.k / TK, BF16_STEP[i], share, 512 * 256 / tm), tm, q8);
         }
+    return best;
+}
+
+// Runs a projection that pipe or mid takes. Both kernels of a converted projection are
+// inside one kernel-timing window.
+int run(h3_gpu *g, const GemmArgs &a, bool q8, int epi) {
+    Plan p = choose(g, a, q8);
+    const size_t weights = (size_t)a.n * a.k;
+    if (p.dequant && !h3_buffer_try(g, &g->gemm_weights, weights * 2)) {
+        // No room for the converted weight: the same tiles on the codes.
+        if (!h3_gemm_mid_fits(a, true)) return h3_set_error(g, "GEMM weight buffer: out of device memory");
+        p.tm = 256;
+        p.split = 1;
+        p.dequant = false;
     }
-    // Variant 1: 2 x 2 waves of 128 x 128 (one wave per SIMD), about 10% slower.
-    if (g->gemm_variant == 1) {
-        switch (epi) {
-        case 0: return launch_tiled<Q8, CHANNEL, 0, 2, 2>(g, a);
-        case 1: return launch_tiled<Q8, CHANNEL, 1, 2, 2>(g, a);
-        case 2: return launch_tiled<Q8, CHANNEL, 2, 2, 2>(g, a);
-        default: return launch_tiled<Q8, CHANNEL, 3, 2, 2>(g, a);
-        }
-    }
-    switch (epi) {
-    case 0: return launch_tiled<Q8, CHANNEL, 0>(g, a);
-    case 1: return launch_tiled<Q8, CHANNEL, 1>(g, a);
-    case 2: return launch_tiled<Q8, CHANNEL, 2>(g, a);
-    default: return launch_tiled<Q8, CHANNEL, 3>(g, a);
-    }
+    if (!p.dequant) return p.tm ? h3_gemm_mid(g, a, q8, p.tm, p.split) : launch_pipe_epi(g, a, epi, p.split, true);
+    const size_t chunks = weights / 16;
+    hipEvent_t timing = h3_kernel_timing_begin(g);
+    hipLaunchKernelGGL(q8_dequant_bf16, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, g->compute,
+                       (const int8_t *)a.w, a.scales, (uint16_t *)g->gemm_weights.ptr, a.k, a.group, a.groups, chunks);
+    GemmArgs b = a;
+    b.w = g->gemm_weights.ptr;
+    const int ok = h3_launch_status(g, "W8A16 dequantization") &&
+                   (p.tm ? h3_gemm_mid(g, b, false, p.tm, p.split, false) : launch_pipe_epi(g, b, epi, p.split, false));
+    h3_kernel_timing_end(g, timing);
+    return ok;
+}
+
+bool tiled(const GemmArgs &a, bool q8) {
+    return !(a.m < 32 && a.k <= H3_GEMM_SHORT_K) && h3_gemm_mid_fits(a, q8);
 }
 
 }  // namespace
@@ -1008,75 +629,37 @@ int h3_gemm_bf16_alpha(h3_gpu *g, uint16_t *y, const uint16_t *x, const uint16_t
     GemmArgs a{};
     a.y = y; a.x = x; a.w = w; a.alpha = alpha; a.m = m; a.n = n; a.k = k; a.group = 1; a.groups = 1;
     if (h3_gemm_skinny_fits(a, false)) return h3_gemm_skinny(g, a, false);
-    if (pipe_fits(a) && g->gemm_variant != 3) return launch_pipe<4>(g, a);
-    if (n % TN == 0 && k % TK == 0 && m >= 32) return launch_tiled<false, false, 4>(g, a);
-    return launch_small(g, a, false);
+    return tiled(a, false) ? run(g, a, false, 4) : launch_small(g, a, false);
 }
 
-// Whether h3_gemm takes SwiGLU as its epilogue for this weight (gate rows, then up
-// rows; 2 * hidden in all): the pipe kernel's shapes.
-bool h3_gemm_swiglu_fits(const h3_gpu *g, const h3_gpu_tensor *w, uint32_t m, uint32_t k, uint32_t hidden) {
+static GemmArgs gemm_args(uint16_t *y, const uint16_t *x, const h3_gpu_tensor *w, const uint16_t *bias, uint32_t m,
+                          uint32_t k, uint32_t n, int activation) {
     GemmArgs a{};
+    a.y = y; a.x = x; a.w = w->data; a.bias = bias; a.m = m; a.n = n; a.k = k; a.gelu = activation;
+    a.scales = w->q8 ? w->q8_scales : nullptr;
+    a.group = w->q8 ? w->q8_group : 1;
+    a.groups = w->q8 ? (k + a.group - 1) / a.group : 1;
+    return a;
+}
+
+bool h3_gemm_swiglu_fits(const h3_gpu_tensor *w, uint32_t m, uint32_t k, uint32_t hidden) {
     if (hidden > UINT32_MAX / 2) return false;
-    a.m = m; a.k = k; a.n = 2 * hidden;
-    return m > 32 && pipe_fits(a) && g->gemm_variant != 3 && (!w->q8 || w->q8_group % 16 == 0);
+    const GemmArgs a = gemm_args(nullptr, nullptr, w, nullptr, m, k, 2 * hidden, H3_GEMM_SWIGLU);
+    return !h3_gemm_skinny_fits(a, w->q8 != 0) && tiled(a, w->q8 != 0);
 }
 
 int h3_gemm(h3_gpu *g, uint16_t *y, const uint16_t *x, const h3_gpu_tensor *w, const uint16_t *bias, uint32_t m,
             uint32_t k, uint32_t n, int activation) {
-    const bool gelu = activation == H3_GEMM_GELU;
-    GemmArgs a{};
-    a.y = y; a.x = x; a.w = w->data; a.bias = bias; a.m = m; a.n = n; a.k = k; a.gelu = gelu;
-    a.scales = w->q8 ? w->q8_scales : nullptr;
-    a.group = w->q8 ? w->q8_group : 1;
-    a.groups = w->q8 ? (k + a.group - 1) / a.group : 1;
+    const bool q8 = w->q8 != 0;
+    const GemmArgs a = gemm_args(y, x, w, bias, m, k, n, activation);
     if (!h3_tensor_acquire(g, w)) return 0;
-    int ok;
-    const bool tiled = n % TN == 0 && k % TK == 0 && m >= 32 && (!w->q8 || a.group % 16 == 0);
-    const int epi = (bias ? 1 : 0) | (gelu ? 2 : 0) | (activation == H3_GEMM_SWIGLU ? 8 : 0);
-    // Variant 3 keeps the earlier kernels (gemm_q8_staged, gemm_kernel) for A/B.
-    const bool pipe = tiled && pipe_fits(a) && g->gemm_variant != 3;
-    if (h3_gemm_skinny_fits(a, w->q8 != 0)) {
-        ok = h3_gemm_skinny(g, a, w->q8 != 0);
-    } else if (pipe && !w->q8) {
-        ok = launch_pipe_epi(g, a, epi);
-    } else if (pipe) {
-        // W8A16: a dequantization pass into the context's BF16 weight buffer
-        // (HBM-bound, ~1% of the GEMM at M = 32400), then the BF16 GEMM on it;
-        // both inside one kernel-timing window.
-        const size_t bytes = (size_t)n * k * 2;
-        if (g->gemm_weights_bytes < bytes) {
-            // An earlier projection may still read the old buffer.
-            if (g->gemm_weights && !h3_hip_check(g, hipStreamSynchronize(g->compute), "GEMM weight buffer")) return 0;
-            if (g->gemm_weights) hipFree(g->gemm_weights);
-            g->gemm_weights = nullptr;
-            g->gemm_weights_bytes = 0;
-            if (!h3_hip_check(g, hipMalloc(&g->gemm_weights, bytes), "GEMM weight buffer")) {
-                g->gemm_weights = nullptr;
-                return 0;
-            }
-            g->gemm_weights_bytes = bytes;
-        }
-        const size_t chunks = (size_t)n * k / 16;
-        hipEvent_t timing = h3_kernel_timing_begin(g);
-        hipLaunchKernelGGL(q8_dequant_bf16, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, g->compute,
-                           (const int8_t *)w->data, w->q8_scales, (uint16_t *)g->gemm_weights, k, a.group, a.groups,
-                           chunks);
-        GemmArgs b = a;
-        b.w = g->gemm_weights;
-        ok = h3_launch_status(g, "W8A16 dequantization") && launch_pipe_epi(g, b, epi, false);
-        h3_kernel_timing_end(g, timing);
-    } else if (tiled) {
-        if (!w->q8) ok = launch_epi<false, false>(g, a);
-        else if (a.group == k) ok = launch_epi<true, true>(g, a);
-        else ok = launch_epi<true, false>(g, a);
-    }
-    else {
-        ok = launch_small(g, a, w->q8 != 0);
-    }
+    const int epi = (bias ? 1 : 0) | (activation == H3_GEMM_GELU ? 2 : 0) | (activation == H3_GEMM_SWIGLU ? 8 : 0);
+    const int ok = h3_gemm_skinny_fits(a, q8) ? h3_gemm_skinny(g, a, q8)
+                   : tiled(a, q8)             ? run(g, a, q8, epi)
+                                              : launch_small(g, a, q8);
     if (ok) {
         g->stats.linear_dispatches++;
-        if (w->q8) { g->stats.q8_dispatches++; g->stats.quant_projection_dispatches++; }
+        if (q8) { g->stats.q8_dispatches++; g->stats.quant_projection_dispatches++; }
     }
     return ok && h3_tensor_release(g, w);
 }

@@ -77,7 +77,7 @@ extern "C" int h3_gpu_mlp_bf16(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tenso
                                const h3_gpu_tensor *w2, uint32_t rows, uint32_t width, uint32_t hidden, uint32_t output_dim) {
     if (!g) return 0;
     const size_t n = (size_t)rows * hidden;
-    const bool fused = w1 && w1->owner == g && !w1->quant_mode && h3_gemm_swiglu_fits(g, w1, rows, width, hidden);
+    const bool fused = n && w1 && w1->owner == g && !w1->quant_mode && h3_gemm_swiglu_fits(w1, rows, width, hidden);
     // Each part with the slack of h3_gpu_tensor_alloc behind it.
     const size_t part = (n * 2 + 511) & ~(size_t)255, product = fused ? 0 : (n * 4 + 511) & ~(size_t)255;
     if (n && n <= MLP_WORKSPACE && part + product <= MLP_WORKSPACE && h3_buffer_try(g, &g->mlp_workspace, part + product)) {

@@ -170,12 +170,30 @@ def test_linear_split_over_k(gpu, m, k, n, q8, bias, gelu):
         gpu.free(t)
 
 
+@pytest.mark.parametrize("m,k,n,group,bias,gelu", [
+    (17, 64, 30, 0, False, False),        # one K step, a ragged column tile of odd width
+    (64, 1088, 256, 0, True, False),      # 17 steps, split
+    (65, 128, 300, 64, True, True),       # W8A16, two steps, one row past a 64-row tile
+    (64, 2176, 512, 16, False, False),    # W8A16, smallest scale group
+    (129, 640, 4096, 640, False, True),   # W8A16 per channel
+    (300, 1088, 2562, 64, True, False),   # width not a multiple of four
+    (513, 2112, 768, 2112, False, False), # K of 64 only
+    (1000, 192, 90, 0, False, False),     # many rows, few columns
+])
+def test_mid_rows_linear(gpu, m, k, n, group, bias, gelu):
+    """Row tiles of 64 to 256 and their remainders against FP64, bound as in
+    test_few_rows_linear."""
+    test_few_rows_linear(gpu, m, k, n, group, bias, gelu)
+
+
 @pytest.mark.parametrize("m,k,hidden,n,group", [
     (300, 512, 384, 256, 0),       # SwiGLU in fc1's epilogue, a ragged row tile
     (600, 4096, 256, 512, 4096),   # the same from split tiles, W8A16
     (33, 256, 128, 256, 64),       # one tile: 128 gate and 128 up rows
     (20, 320, 128, 192, 0),        # few rows: separate SwiGLU
     (70, 100, 30, 50, 0),          # unaligned
+    (100, 640, 100, 64, 64),       # SwiGLU over 200 weight rows: gate and up rows ragged
+    (200, 2048, 512, 300, 64),     # the same from split tiles, W8A16
 ])
 def test_mlp(gpu, m, k, hidden, n, group):
     """fc1 -> SwiGLU -> fc2 against FP64. Gate, up, the activation and the result
