@@ -19,6 +19,12 @@ int h3_launch_attention_bf16(h3_gpu *g, void *workspace, uint16_t *out, const ui
                              const uint16_t *v, uint32_t seq, uint32_t heads, float scale,
                              bool head_major, const uint32_t *kv_list, const uint32_t *kv_count,
                              uint32_t list_stride);
+// attn_small.hip: dense attention of few query rows, in one launch with no workspace.
+// The 32-query blocks per workgroup it takes for this shape (1 or 2), 0 where the
+// 256-query tiles are faster.
+int h3_attention_small_blocks(const h3_gpu *g, uint32_t seq, uint32_t heads);
+int h3_launch_attention_small(h3_gpu *g, int blocks, uint16_t *out, const uint16_t *q, const uint16_t *k,
+                              const uint16_t *v, uint32_t seq, uint32_t heads, float scale, bool head_major);
 // Dense attention of qrows query rows (q, out offset to the first) over seq
 // keys with the FP32 natural-log LSE per (head, query row) into lse [heads, qrows].
 int h3_launch_attention_flash(h3_gpu *g, void *workspace, uint16_t *out, const uint16_t *q, const uint16_t *k,

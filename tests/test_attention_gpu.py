@@ -156,6 +156,62 @@ def test_scheduled_kernel_matches_wide_kernel(gpu, monkeypatch, case):
         g14.close()
 
 
+@pytest.mark.parametrize("variant,kind", [("14", "rise"), ("14", "fall"), ("14", "spike"), ("3", "spike")])
+def test_tile_kernels_agree_at_many_heads(gpu, monkeypatch, variant, kind):
+    """As the two tests above, with enough query rows that the 256-query tile
+    kernels run (few rows take a kernel of their own under every variant)."""
+    seq, heads = 1500, 42
+    q, k, v = (np.tile(x.reshape(seq, 2, 128), (1, 21, 1)).reshape(-1) for x in _growth_inputs(seq, 2, kind))
+    fast = sdpa(gpu, q, k, v, seq, heads)
+    monkeypatch.setenv("H3_HIP_ATTENTION_VARIANT", variant)
+    g = Gpu()
+    try:
+        assert np.array_equal(sdpa(g, q, k, v, seq, heads), fast)
+    finally:
+        g.close()
+
+
+@pytest.mark.parametrize("head_major", [False, True])
+@pytest.mark.parametrize("seq,heads", [
+    (31, 2),      # part of one query block, one wave's tile
+    (33, 1),      # two query blocks
+    (64, 3),      # one whole tile
+    (257, 3),     # five tiles: one wave takes two
+    (1024, 8),    # the most rows of one block per workgroup
+    (2050, 8),    # two blocks per workgroup, ragged
+])
+def test_few_rows_every_element(gpu, seq, heads, head_major):
+    """Few query rows (a kernel of their own) against FP64 on every element:
+    P and the output are rounded to BF16 (2^-9 relative), so an output is
+    within 2^-8 sum p |v| of the exact one."""
+    print(f"[attention] few rows seq={seq} heads={heads} head_major={head_major}", flush=True)
+    q, k, v = synth.attention_inputs(seq, heads, seed=seq, scale=1.0)
+    got = bf16(sdpa(gpu, q, k, v, seq, heads, head_major=head_major)).reshape(seq, heads, 128)
+    scale = scale_bf16(1 / math.sqrt(128))
+    qf, kf, vf = (bf16(x).reshape(seq, heads, 128).astype(np.float64) for x in (q, k, v))
+    for h in range(heads):
+        s = qf[:, h] @ kf[:, h].T * scale
+        p = np.exp(s - s.max(axis=1, keepdims=True))
+        p /= p.sum(axis=1, keepdims=True)
+        bound = 2.0 ** -8 * (p @ np.abs(vf[:, h])) + 2.0 ** -20
+        assert np.all(np.abs(got[:, h] - p @ vf[:, h]) <= bound), h
+
+
+@pytest.mark.parametrize("row", [0, 200, 383, 699])
+@pytest.mark.parametrize("which,value", [(0, np.inf), (1, -np.inf), (1, np.nan), (2, np.inf)])
+def test_few_rows_nonfinite(gpu, which, value, row):
+    """One Inf or NaN anywhere in Q, K or V is reported, also where its scores
+    are all -Inf and the output stays finite."""
+    seq, heads = 700, 3
+    x = [synth.bf16_to_f32(t).reshape(seq, heads, 128).copy() for t in synth.attention_inputs(seq, heads, seed=3)]
+    if which == 1 and value == -np.inf:
+        x[0] = np.abs(x[0])      # -Inf times positive queries: every score -Inf
+    x[which][row, 1, 77] = value
+    bits = [synth.f32_to_bf16(t.reshape(-1)) for t in x]
+    with Gpu() as g, pytest.raises(Exception, match="nonfinite"):
+        sdpa(g, *bits, seq, heads)
+
+
 def test_large_values_after_score_jump(gpu):
     """A 41-log2-unit score jump with |V| near 1e26: P that large must not
     reach O unscaled (it would overflow FP32). The rows go to the
