@@ -5,6 +5,32 @@
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
+struct GemmPlan {
+    float us;             // modelled time
+    unsigned tm;          // row tile of gemm_mid, 0: gemm_bf16_pipe
+    unsigned split;       // K shares of each tile of the last, incomplete wave
+    bool dequant;         // W8A16: convert the whole weight to BF16 first
+};
+
+// Modelled time in microseconds of tiles output tiles of `units` K units, unit_us
+// each: 2 more per workgroup, share_us per share of a split tile for its partial sums
+// written and read, 3 for the reduction launch and 0.9 for each share added in turn.
+// At most `most` shares in all (128 MB), each of `least_units` or more.
+inline GemmPlan gemm_last_wave(const h3_gpu *g, unsigned tiles, unsigned units, float unit_us, float share_us, unsigned most,
+                               unsigned least_units = 1) {
+    const unsigned rest = tiles % g->cus;
+    GemmPlan p{(float)(tiles / g->cus) * (units * unit_us + 2.f), 0, 1, false};
+    if (!rest) return p;
+    float least = units * unit_us + 2.f;
+    for (unsigned s = 2; s <= 32 && s * least_units <= units && rest * s <= most; s++) {
+        const float waves = (float)((rest * s + g->cus - 1) / g->cus);
+        const float t = waves * ((units + s - 1) / s * unit_us + 2.f) + rest * s * share_us + 3.f + 0.9f * s;
+        if (t < least) { least = t; p.split = s; }
+    }
+    p.us += least;
+    return p;
+}
+
 // Epilogue of h3_gemm after the bias. SwiGLU (no bias): the weight holds hidden gate
 // rows, then hidden up rows, n = 2 * hidden, and y is [m, hidden]; only where
 // h3_gemm_swiglu_fits.
@@ -39,6 +65,20 @@ __device__ inline float gelu_tanh(float v) {
 // saturate through exp to gate * up or a signed zero.
 __device__ inline float swiglu_fast(float gate, float up) {
     return gate * __builtin_amdgcn_rcpf(1.0f + __expf(-gate)) * up;
+}
+
+// Tile (row, column) of workgroup pid: bands of at most `rows` row tiles sweep the
+// columns together, so that the workgroups an XCD runs at a time share both operands in
+// its L2. The row tiles are spread evenly over the bands: a last band of one row would
+// read the whole weight for it alone (FP8, 8193 rows, 5376 -> 21504, in bands of four:
+// 832 us, in nine bands of three or four: 780 us).
+__device__ inline void band_tile(unsigned tiles_m, unsigned tiles_n, unsigned rows, unsigned pid, unsigned &tm,
+                                 unsigned &tn) {
+    const unsigned bands = (tiles_m + rows - 1) / rows, band = ((pid / tiles_n + 1) * bands - 1) / tiles_m;
+    const unsigned first = band * tiles_m / bands, count = (band + 1) * tiles_m / bands - first;
+    const unsigned at = pid - first * tiles_n;
+    tm = first + at % count;
+    tn = at / count;
 }
 
 // 16 int8 codes of one scale group -> BF16 values w = bf16(code * scale), the

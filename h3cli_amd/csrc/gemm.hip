@@ -138,6 +138,8 @@ constexpr int PIPE_GROUP_M = 4;
 // First row and column of output tile pid: bands of PIPE_GROUP_M row tiles sweep
 // the columns together.
 __device__ inline void pipe_tile(const GemmArgs &a, unsigned pid, unsigned &m0, unsigned &n0) {
+    // A last band of fewer rows, not even bands: 8193 rows, 5376 -> 28672 -> 5376 (33 row
+    // tiles) 2.87 ms against 2.93 in nine bands of three or four.
     const unsigned tiles_m = (a.m + TM - 1) / TM, tiles_n = a.n / TN;
     const unsigned band = pid / (PIPE_GROUP_M * tiles_n), first_m = band * PIPE_GROUP_M;
     const unsigned rows_in_band = min(tiles_m - first_m, (unsigned)PIPE_GROUP_M);
@@ -532,31 +534,6 @@ int launch_small(h3_gpu *g, const GemmArgs &a, bool q8) {
 }
 
 // ------------------------------------------------------------ choice of the kernel
-struct Plan {
-    float us;             // modelled time
-    unsigned tm;          // row tile of gemm_mid, 0: gemm_bf16_pipe
-    unsigned split;       // K shares of each tile of the last, incomplete wave
-    bool dequant;         // W8A16: convert the whole weight to BF16 first
-};
-
-// Modelled time in microseconds of tiles output tiles of `units` K units, unit_us
-// each: 2 more per workgroup, share_us per share of a split tile for its partial sums
-// written and read, 3 for the reduction launch and 0.9 for each share added in turn.
-// At most `most` shares (128 MB).
-Plan last_wave(const h3_gpu *g, unsigned tiles, unsigned units, float unit_us, float share_us, unsigned most) {
-    const unsigned rest = tiles % g->cus;
-    Plan p{(float)(tiles / g->cus) * (units * unit_us + 2.f), 0, 1, false};
-    if (!rest) return p;
-    float least = units * unit_us + 2.f;
-    for (unsigned s = 2; s <= 32 && s <= units && rest * s <= most; s++) {
-        const float waves = (float)((rest * s + g->cus - 1) / g->cus);
-        const float t = waves * ((units + s - 1) / s * unit_us + 2.f) + rest * s * share_us + 3.f + 0.9f * s;
-        if (t < least) { least = t; p.split = s; }
-    }
-    p.us += least;
-    return p;
-}
-
 // The faster of the kernels that take this projection, by the model above with these
 // rates (microseconds per 64 values of K, one workgroup on each CU, measured at 64 to
 // 8193 rows): pipe 1.5; mid, BF16 weights 1.0 / 1.2 / 1.95 for 64 / 128 / 256 rows;
@@ -569,24 +546,24 @@ Plan last_wave(const h3_gpu *g, unsigned tiles, unsigned units, float unit_us, f
 // int8: pipe in 2 shares 209 (mid 202); 2000 rows, 5120 -> 5120, int8: pipe 116 (mid
 // 140); 300 rows, 7168 -> 5376, BF16: mid 128 in 4 shares 38.7 (pipe 50.9); 8193 rows,
 // 5440 -> 5120, int8, which pipe does not take: converted first 442 (mid 475).
-Plan choose(const h3_gpu *g, const GemmArgs &a, bool q8) {
+GemmPlan choose(const h3_gpu *g, const GemmArgs &a, bool q8) {
     static constexpr float BF16_STEP[3] = {1.0f, 1.2f, 1.95f}, Q8_STEP[3] = {1.3f, 1.25f, 2.1f};
-    Plan best{3.4e38f, 0, 1, false};
+    GemmPlan best{3.4e38f, 0, 1, false};
     const bool pipe = pipe_fits(a);
     const float convert = q8 ? (float)a.n * a.k * 0.5e-6f + 4.f : 0.f;
-    auto consider = [&](Plan p, unsigned tm, bool dequant) {
+    auto consider = [&](GemmPlan p, unsigned tm, bool dequant) {
         p.tm = tm;
         p.dequant = dequant;
         if (dequant) p.us += convert;
         if (p.us < best.us) best = p;
     };
-    if (pipe) consider(last_wave(g, (a.m + TM - 1) / TM * (a.n / TN), a.k / (2 * TK), 3.0f, 0.09f, 512), 0, q8);
+    if (pipe) consider(gemm_last_wave(g, (a.m + TM - 1) / TM * (a.n / TN), a.k / (2 * TK), 3.0f, 0.09f, 512), 0, q8);
     if (h3_gemm_mid_fits(a, q8))
         for (unsigned i = 0; i < 3; i++) {
             const unsigned tm = 64u << i, tiles = (a.m + tm - 1) / tm * ((a.n + TN - 1) / TN);
             const float share = 0.09f * tm / 256;
-            if (q8) consider(last_wave(g, tiles, a.k / TK, Q8_STEP[i], share, 512 * 256 / tm), tm, false);
-            if (i < 2 || !pipe) consider(last_wave(g, tiles, a.k / TK, BF16_STEP[i], share, 512 * 256 / tm), tm, q8);
+            if (q8) consider(gemm_last_wave(g, tiles, a.k / TK, Q8_STEP[i], share, 512 * 256 / tm), tm, false);
+            if (i < 2 || !pipe) consider(gemm_last_wave(g, tiles, a.k / TK, BF16_STEP[i], share, 512 * 256 / tm), tm, q8);
         }
     return best;
 }
@@ -594,7 +571,7 @@ Plan choose(const h3_gpu *g, const GemmArgs &a, bool q8) {
 // Runs a projection that pipe or mid takes. Both kernels of a converted projection are
 // inside one kernel-timing window.
 int run(h3_gpu *g, const GemmArgs &a, bool q8, int epi) {
-    Plan p = choose(g, a, q8);
+    GemmPlan p = choose(g, a, q8);
     const size_t weights = (size_t)a.n * a.k;
     if (p.dequant && !h3_buffer_try(g, &g->gemm_weights, weights * 2)) {
         // No room for the converted weight: the same tiles on the codes.

@@ -67,11 +67,10 @@ __device__ inline __amdgpu_buffer_rsrc_t uniform_resource(const void *p, unsigne
 
 template <int TM>
 __device__ inline void mid_tile(const GemmArgs &a, unsigned pid, unsigned &m0, unsigned &n0) {
-    const unsigned tiles_m = (a.m + TM - 1) / TM, tiles_n = (a.n + TN - 1) / TN;
-    const unsigned band = pid / (GROUP_M * tiles_n), first_m = band * GROUP_M;
-    const unsigned rows_in_band = min(tiles_m - first_m, (unsigned)GROUP_M);
-    m0 = __builtin_amdgcn_readfirstlane((first_m + (pid % (GROUP_M * tiles_n)) % rows_in_band) * TM);
-    n0 = __builtin_amdgcn_readfirstlane((pid % (GROUP_M * tiles_n)) / rows_in_band * TN);
+    unsigned tm, tn;
+    band_tile((a.m + TM - 1) / TM, (a.n + TN - 1) / TN, GROUP_M, pid, tm, tn);
+    m0 = __builtin_amdgcn_readfirstlane(tm * TM);
+    n0 = __builtin_amdgcn_readfirstlane(tn * TN);
 }
 
 // Row of the weight that tile row r holds. SwiGLU: 32 gate rows and the 32 up rows of

@@ -1,7 +1,6 @@
 // FP8 W8A8 DiT projections (reference src/cuda/cuda_quant.cuh): tensorwide
 // E4M3 packing of weights and activations, the content-hashed packed-weight
-// artifacts (H3QWT001), and an FP8 GEMM on gfx950's v_mfma_f32_32x32x64_f8f6f4
-// in place of cuBLASLt.
+// artifacts (H3QWT001), and an FP8 GEMM (gemm_fp8.hip) in place of cuBLASLt.
 //
 // Arithmetic contract (cuda_quant.cuh:26-49, 362-394):
 //   scale = max(max|x| / 448, 1e-20), code = E4M3(x / scale), RNE, saturating;
@@ -14,15 +13,11 @@
 // MI355X design:
 //  * packing is HBM-bound: a max pass (16-byte loads, per-workgroup maxima),
 //    a one-workgroup finish, and an encode pass (16-byte loads, 8-byte stores);
-//  * the GEMM computes C^T = W . X^T with 256 x 256 output tiles, 8 waves (two
-//    per SIMD, 128 x 64 each), 128-byte K stages of both operands loaded
-//    global -> LDS directly (XOR-swizzled 16-byte chunks), double buffered;
-//    each K stage is two 32x32x64 FP8 MFMA steps per accumulator block, the
-//    fragments of the next step read during the current one; workgroup ids are
-//    XCD-remapped and grouped along M, as in the BF16 GEMM.
+//  * the GEMM is gemm_fp8.hip's.
 #include "common.h"
 #include "internal.h"
 #include "sage.h"
+#include "gemm_fp8.h"
 #include "../../include/h3_quant.h"
 #include "../../include/h3_residency.h"
 #include "../../include/h3_gpu_surface.h"
@@ -259,129 +254,6 @@ int nvfp4_pack_all(h3_gpu *g, const uint16_t *x, unsigned rows, unsigned k, unsi
     hipLaunchKernelGGL(nvfp4_pack, dim3((unsigned)((blocks + 255) / 256)), dim3(256), 0, g->compute, x, rows, k,
                        (const float *)global, codes, scales, deq);
     return h3_launch_status(g, "NVFP4 packing");
-}
-
-// ---------------------------------------------------------------- GEMM
-constexpr int TM = 256, TN = 256, TK = 128;          // TK in FP8 bytes
-constexpr int ROW = TK;                              // 128 B per LDS row
-constexpr int TILE = 256 * ROW;                      // 32 KB per operand tile
-constexpr int STAGE = 2 * TILE;
-constexpr int GROUP_M = 8;
-
-__device__ inline unsigned swz(unsigned row, unsigned ch) { return ch ^ ((row >> 1) & 7); }
-
-struct Fp8Args {
-    uint16_t *y;
-    const uint8_t *x, *w;
-    const float *sx, *sw;     // device scalars: activation and weight scales
-    unsigned m, n, k;
-};
-
-__global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2)))
-void fp8_gemm(Fp8Args a) {
-    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
-    const unsigned tid = threadIdx.x, wave = tid / 64, lane = tid % 64, n32 = lane % 32, hf = lane / 32;
-    const unsigned tiles_m = (a.m + TM - 1) / TM, tiles_n = (a.n + TN - 1) / TN;
-    const unsigned pid = xcd_remap(blockIdx.x, gridDim.x);
-    const unsigned band = pid / (GROUP_M * tiles_n), first_m = band * GROUP_M;
-    const unsigned rows_in_band = min(tiles_m - first_m, (unsigned)GROUP_M);
-    const unsigned tm = first_m + (pid % (GROUP_M * tiles_n)) % rows_in_band;
-    const unsigned tn = (pid % (GROUP_M * tiles_n)) / rows_in_band;
-    const unsigned m0 = tm * TM, n0 = tn * TN;
-    const unsigned wm = wave / 4, wn = wave % 4;   // rows m0 + wm*128, columns n0 + wn*64
-    const unsigned ksteps = a.k / TK;
-
-    f32x16 acc[2][4];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = f32x16{};
-
-    // 256 rows x 128 B of each operand: 32 groups of 8 rows, 16 B per lane.
-    auto load = [&](unsigned kt, int stage) {
-        uint8_t *xs = lds + stage * STAGE;
-#pragma unroll
-        for (unsigned b = wave; b < 32; b += 8) {
-            const unsigned row = 8 * b + lane / 8, ph = lane % 8;
-            const unsigned gm = min(m0 + row, a.m - 1);
-            const uint8_t *xsrc = a.x + (size_t)gm * a.k + kt * TK + swz(row, ph) * 16;
-            const uint8_t *wsrc = a.w + (size_t)min(n0 + row, a.n - 1) * a.k + kt * TK + swz(row, ph) * 16;
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)xsrc,
-                                             (__attribute__((address_space(3))) void *)(xs + b * 1024), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)wsrc,
-                                             (__attribute__((address_space(3))) void *)(xs + TILE + b * 1024), 16, 0, 0);
-        }
-    };
-    // MFMA step s (64 K bytes): lane half hf supplies bytes 32 hf .. 32 hf + 31,
-    // chunks 4 s + 2 hf and 4 s + 2 hf + 1 of its row.
-    auto fragment = [&](const uint8_t *tile, unsigned row, int s) -> i32x8 {
-        const unsigned c0 = 4 * s + 2 * hf;
-        const i32x4 lo = *reinterpret_cast<const i32x4 *>(tile + row * ROW + swz(row, c0) * 16);
-        const i32x4 hi = *reinterpret_cast<const i32x4 *>(tile + row * ROW + swz(row, c0 + 1) * 16);
-        return i32x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    };
-
-    load(0, 0);
-    wait_vm_loads();
-    __syncthreads();
-    for (unsigned kt = 0; kt < ksteps; kt++) {
-        const int cur = kt & 1;
-        if (kt + 1 < ksteps) load(kt + 1, cur ^ 1);
-        const uint8_t *xs = lds + cur * STAGE, *ws = xs + TILE;
-        i32x8 wf[2][2], xf[2][4];
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-#pragma unroll
-            for (int i = 0; i < 2; i++) wf[s][i] = fragment(ws, wn * 64 + i * 32 + n32, s);
-#pragma unroll
-            for (int j = 0; j < 4; j++) xf[s][j] = fragment(xs, wm * 128 + j * 32 + n32, s);
-        }
-#pragma unroll
-        for (int s = 0; s < 2; s++)
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wf[s][i], xf[s][j], acc[i][j], 0, 0,
-                                                                                0, 0, 0, 0);
-        wait_vm_loads();
-        __syncthreads();
-    }
-
-    const float scale = a.sx[0] * a.sw[0];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const unsigned row = m0 + wm * 128 + j * 32 + n32;
-        if (row >= a.m) continue;
-        uint16_t *dst = a.y + (size_t)row * a.n;
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int g4 = 0; g4 < 4; g4++) {
-                const unsigned col = n0 + wn * 64 + i * 32 + g4 * 8 + hf * 4;
-                if (col >= a.n) continue;     // N is a multiple of 128: the last tile may be half full
-                u16x4 out;
-#pragma unroll
-                for (int e = 0; e < 4; e++) out[e] = f32_to_bf16(acc[i][j][g4 * 4 + e] * scale);
-                *reinterpret_cast<u16x4 *>(dst + col) = out;
-            }
-    }
-}
-
-// Packed weights have N and K multiples of 128 (h3_gpu_quant_load); any M.
-int launch_gemm(h3_gpu *g, const Fp8Args &a) {
-    static bool configured = false;
-    if (!configured) {
-        if (!h3_hip_check(g, hipFuncSetAttribute((const void *)fp8_gemm, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 2 * STAGE), "FP8 GEMM shared memory"))
-            return 0;
-        configured = true;
-    }
-    const unsigned tiles = (a.m + TM - 1) / TM * ((a.n + TN - 1) / TN);
-    hipEvent_t timing = h3_kernel_timing_begin(g);
-    hipLaunchKernelGGL(fp8_gemm, dim3(tiles), dim3(512), 2 * STAGE, g->compute, a);
-    h3_kernel_timing_end(g, timing);
-    return h3_launch_status(g, "native fp8 projection");
 }
 
 // ---------------------------------------------------------------- host helpers
@@ -927,11 +799,11 @@ int h3_quant_gemm(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tensor *in, const 
         return 1;
     }
     if (!fp8_pack(g, (const uint16_t *)in->data, count, base, partials, global, nullptr)) return 0;
-    Fp8Args a;
+    Fp8GemmArgs a{};
     a.y = (uint16_t *)out->data; a.x = base; a.w = weight;
     a.sx = global; a.sw = (const float *)(weight + w->quant_scale);
     a.m = rows; a.n = n; a.k = k;
-    if (!launch_gemm(g, a)) return 0;
+    if (!h3_gemm_fp8(g, a)) return 0;
     g->stats.quant_projection_dispatches++;
     g->stats.linear_dispatches++;
     return 1;

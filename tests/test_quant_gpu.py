@@ -205,6 +205,32 @@ def test_strict_artifact(tmp_path):
             load(g, path, n, k)
 
 
+@pytest.mark.parametrize("m,n,k", [(300, 384, 4224), (33, 256, 2048), (70, 640, 1152)])
+def test_gemm_split_over_k(tmp_path, m, n, k):
+    """Few tiles and a long K: shares of K added by a second launch (33 K tiles in
+    uneven shares, two shares of eight, and nine K tiles unsplit), with the bound
+    of test_gemm_against_oracle."""
+    say(f"gemm split m={m} n={n} k={k}")
+    rng = np.random.default_rng(m * 7 + n)
+    w = synth.f32_to_bf16((rng.standard_normal(n * k) * 0.03).astype(np.float32))
+    x = synth.f32_to_bf16((rng.standard_normal(m * k) * 1.5).astype(np.float32))
+    path = tmp_path / "w.bin"
+    write_weight(path, w)
+    with Gpu() as g:
+        g.check(configure(g, tmp_path / "cache"), "configure")
+        weight = load(g, path, n, k)
+        x8, xg = pack_on_gpu(g, x)
+        got = linear(g, g.empty(m * n), g.from_bf16(x), weight, m, k, n)
+        w8, sw, _ = oracle.fp8_pack(w)
+        want = oracle.fp8_gemm(x8, xg[0], w8, sw, m, n, k)
+    table = oracle.e4m3_decode(np.arange(256)).astype(np.float64)
+    X, W = np.abs(table[x8]).reshape(m, k // 64, 64).max(axis=2), np.abs(table[w8]).reshape(n, k // 64, 64).max(axis=2)
+    s = float(np.float32(xg[0]) * np.float32(sw))
+    g32, w32 = synth.bf16_to_f32(got).astype(np.float64), synth.bf16_to_f32(want).astype(np.float64)
+    bound = 2.0 ** -7 * np.maximum(np.abs(g32), np.abs(w32)) + 2.0 ** -14 * s * (X @ W.T)
+    assert np.all(np.abs(g32 - w32) <= bound), np.max(np.abs(g32 - w32) - bound)
+
+
 @pytest.mark.parametrize("m,n,k", [(300, 512, 384), (1, 256, 128), (257, 768, 1024), (33, 384, 256),
                                    (1000, 1280, 640)])
 def test_gemm_against_oracle(tmp_path, m, n, k):
