@@ -5,26 +5,28 @@
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
+constexpr unsigned GEMM_Q8 = 1;
+
 struct GemmPlan {
     float us;             // modelled time
-    unsigned tm;          // row tile of gemm_mid, 0: gemm_bf16_pipe
+    unsigned tm;          // row tile of gemm_mid, 0: gemm_bf16_pipe, GEMM_Q8: gemm_q8_pipe
     unsigned split;       // K shares of each tile of the last, incomplete wave
     bool dequant;         // W8A16: convert the whole weight to BF16 first
 };
 
 // Modelled time in microseconds of tiles output tiles of `units` K units, unit_us
-// each: 2 more per workgroup, share_us per share of a split tile for its partial sums
+// each: start_us more per workgroup, share_us per share of a split tile for its partial sums
 // written and read, 3 for the reduction launch and 0.9 for each share added in turn.
 // At most `most` shares in all (128 MB), each of `least_units` or more.
 inline GemmPlan gemm_last_wave(const h3_gpu *g, unsigned tiles, unsigned units, float unit_us, float share_us, unsigned most,
-                               unsigned least_units = 1) {
+                               unsigned least_units = 1, float start_us = 2.f) {
     const unsigned rest = tiles % g->cus;
-    GemmPlan p{(float)(tiles / g->cus) * (units * unit_us + 2.f), 0, 1, false};
+    GemmPlan p{(float)(tiles / g->cus) * (units * unit_us + start_us), 0, 1, false};
     if (!rest) return p;
-    float least = units * unit_us + 2.f;
+    float least = units * unit_us + start_us;
     for (unsigned s = 2; s <= 32 && s * least_units <= units && rest * s <= most; s++) {
         const float waves = (float)((rest * s + g->cus - 1) / g->cus);
-        const float t = waves * ((units + s - 1) / s * unit_us + 2.f) + rest * s * share_us + 3.f + 0.9f * s;
+        const float t = waves * ((units + s - 1) / s * unit_us + start_us) + rest * s * share_us + 3.f + 0.9f * s;
         if (t < least) { least = t; p.split = s; }
     }
     p.us += least;
@@ -110,3 +112,7 @@ int h3_gemm_skinny(h3_gpu *g, const GemmArgs &a, bool q8);
 // shares of K.
 bool h3_gemm_mid_fits(const GemmArgs &a, bool q8);
 int h3_gemm_mid(h3_gpu *g, const GemmArgs &a, bool q8, unsigned tm, unsigned split, bool timed = true);
+
+// gemm_q8.hip: per-column W8A16 weights converted in a hand-scheduled loop, 256 x 256 tiles.
+bool h3_gemm_q8_fits(const GemmArgs &a);
+int h3_gemm_q8(h3_gpu *g, GemmArgs a, unsigned split);

@@ -15,6 +15,7 @@
 //    (in registers, 16 codes per thread), which costs about 1% of the GEMM at
 //    M = 32400 and leaves the MFMA loop free of VALU work;
 //  * gemm_mid.hip: fewer rows, any N, int8 weights converted in the kernel;
+//  * gemm_q8.hip: per-column int8 weights converted in a hand-scheduled loop;
 //  * gemm_skinny.hip: at most 16 rows;
 //  * gemm_small, here: any shape.
 // Both tiled kernels compute C^T = W . X^T, so a lane owns one output row and
@@ -375,7 +376,7 @@ int launch_pipe(h3_gpu *g, GemmArgs a, unsigned split, bool timed) {
     }
     const unsigned tiles = (a.m + TM - 1) / TM * (a.n / TN);
     unsigned rest = tiles % g->cus;
-    a.split = split;
+    a.split = split < a.k / (2 * TK) ? split : a.k / (2 * TK);   // every share has a stage pair
     if (a.split > 1 && !h3_buffer_try(g, &g->gemm_partials, (size_t)rest * a.split * TM * TN * 4)) a.split = 1;
     if (a.split == 1) rest = 0;
     a.full = tiles - rest;
@@ -537,15 +538,17 @@ int launch_small(h3_gpu *g, const GemmArgs &a, bool q8) {
 // The faster of the kernels that take this projection, by the model above with these
 // rates (microseconds per 64 values of K, one workgroup on each CU, measured at 64 to
 // 8193 rows): pipe 1.5; mid, BF16 weights 1.0 / 1.2 / 1.95 for 64 / 128 / 256 rows;
-// mid, int8 weights 1.3 / 1.25 / 2.1; converting a weight to BF16 first 0.5 per million
-// values. Measured, in microseconds, the runner-up in brackets: 63 tiles of 256
-// (729 rows, 7168 -> 5376), BF16: pipe in 4 shares 66.6 (unsplit 134.6); 336 tiles
-// (729 rows, 5376 -> 28672), BF16: pipe, the last 80 tiles in 3 shares, 201.8 (242.6);
-// 693 tiles (8193 rows, 14336 -> 5376): unsplit 998 (2 shares 1018); 729 rows,
-// 5376 -> 28672, int8: mid 256 in 3 shares 247 (pipe 287); 1200 rows, 13824 -> 5120,
-// int8: pipe in 2 shares 209 (mid 202); 2000 rows, 5120 -> 5120, int8: pipe 116 (mid
-// 140); 300 rows, 7168 -> 5376, BF16: mid 128 in 4 shares 38.7 (pipe 50.9); 8193 rows,
-// 5440 -> 5120, int8, which pipe does not take: converted first 442 (mid 475).
+// mid, int8 weights 1.3 / 1.25 / 2.1; q8 1.72, and 10 to fill its stages and to store;
+// converting a weight to BF16 first 0.5 per million values. Measured, in microseconds,
+// the runner-up in brackets: 63 tiles of 256 (729 rows, 7168 -> 5376), BF16: pipe in 4
+// shares 66.6 (unsplit 134.6); 336 tiles (729 rows, 5376 -> 28672), BF16: pipe, the last
+// 80 tiles in 3 shares, 201.8 (242.6); 693 tiles (8193 rows, 14336 -> 5376): unsplit 998
+// (2 shares 1018); 729 rows, 5376 -> 28672, int8 of group 64: mid 256 in 3 shares 247
+// (pipe 287), one scale per column: q8 in 3 shares 246 (mid 265); 1200 rows, 13824 ->
+// 5120, per column: q8 in 2 shares 197 (pipe 211); 2000 rows, 5120 -> 5120, int8: pipe
+// 117 (q8 124, mid 140); 700 rows, 1024 -> 14336, per column: mid 256 40.4 (q8 46.8);
+// 300 rows, 7168 -> 5376, BF16: mid 128 in 4 shares 38.7 (pipe 50.9); 8193 rows,
+// 5440 -> 5120, group 64, which pipe does not take: converted first 442 (mid 475).
 GemmPlan choose(const h3_gpu *g, const GemmArgs &a, bool q8) {
     static constexpr float BF16_STEP[3] = {1.0f, 1.2f, 1.95f}, Q8_STEP[3] = {1.3f, 1.25f, 2.1f};
     GemmPlan best{3.4e38f, 0, 1, false};
@@ -558,6 +561,10 @@ GemmPlan choose(const h3_gpu *g, const GemmArgs &a, bool q8) {
         if (p.us < best.us) best = p;
     };
     if (pipe) consider(gemm_last_wave(g, (a.m + TM - 1) / TM * (a.n / TN), a.k / (2 * TK), 3.0f, 0.09f, 512), 0, q8);
+    if (q8 && h3_gemm_q8_fits(a)) {
+        const unsigned tiles = (a.m + TM - 1) / TM * ((a.n + TN - 1) / TN);
+        consider(gemm_last_wave(g, tiles, a.k / TK, 1.72f, 0.04f, 256, 1, 10.f), GEMM_Q8, false);
+    }
     if (h3_gemm_mid_fits(a, q8))
         for (unsigned i = 0; i < 3; i++) {
             const unsigned tm = 64u << i, tiles = (a.m + tm - 1) / tm * ((a.n + TN - 1) / TN);
@@ -580,6 +587,7 @@ int run(h3_gpu *g, const GemmArgs &a, bool q8, int epi) {
         p.split = 1;
         p.dequant = false;
     }
+    if (p.tm == GEMM_Q8) return h3_gemm_q8(g, a, p.split);
     if (!p.dequant) return p.tm ? h3_gemm_mid(g, a, q8, p.tm, p.split) : launch_pipe_epi(g, a, epi, p.split, true);
     const size_t chunks = weights / 16;
     hipEvent_t timing = h3_kernel_timing_begin(g);

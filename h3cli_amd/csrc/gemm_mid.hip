@@ -364,7 +364,7 @@ int launch(h3_gpu *g, GemmArgs a, unsigned split, bool timed) {
     }
     const unsigned tiles = (a.m + TM - 1) / TM * ((a.n + TN - 1) / TN);
     unsigned rest = tiles % g->cus;
-    a.split = split;
+    a.split = split < a.k / TK ? split : a.k / TK;   // every share has a K step
     if (a.split > 1 && !h3_buffer_try(g, &g->gemm_partials, (size_t)rest * a.split * TM * TN * 4)) a.split = 1;
     if (a.split == 1) rest = 0;
     a.full = tiles - rest;

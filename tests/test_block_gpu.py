@@ -227,6 +227,22 @@ def test_mlp(gpu, m, k, hidden, n, group):
         gpu.free(t)
 
 
+@pytest.mark.parametrize("m,k,n,hidden,bias,gelu", [
+    (1000, 1472, 16192, 0, True, True),   # an odd K tile count, a quarter column tile
+    (500, 1792, 32768, 0, True, False),   # an even one, a row tile of 244 rows
+    (520, 4160, 8256, 0, False, True),    # 65 K tiles in two shares, 8 rows of the last row tile
+    (513, 2112, 192, 9664, False, False), # SwiGLU, one row and half a column tile past whole ones
+    (520, 4160, 128, 4128, False, False), # SwiGLU from split tiles, a quarter column tile
+])
+def test_per_channel_q8(gpu, m, k, n, hidden, bias, gelu):
+    """W8A16 with one scale per channel, at sizes that convert the codes inside the
+    hand-scheduled K loop; bounds as in test_few_rows_linear and test_mlp."""
+    if hidden:
+        test_mlp(gpu, m, k, hidden, n, k)
+    else:
+        test_few_rows_linear(gpu, m, k, n, k, bias, gelu)
+
+
 def test_bf16_linear_exact_pattern(gpu):
     """tests/quant_native.c:31-50 power-of-two pattern: the BF16 GEMM output must
     equal bf16(exact sum) bit for bit, for several row counts."""
