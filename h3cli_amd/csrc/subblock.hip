@@ -9,13 +9,15 @@
 // MI355X layout: the cell dot products of one head form a [cells x cells]
 // matrix product, so scoring runs on the matrix cores (32 x 32 cell tiles,
 // fp32 accumulation of exact BF16 products) and the two log-sum-exps fold in
-// registers. Selection writes the route bytes and, in the same pass, the
+// registers; the pools are stored in that product's fragment order. Selection finds each
+// row's threshold by bisection of its keys in registers. It writes the route bytes and, in the same pass, the
 // ordered list of kept 64-key tiles per (head, 128-query block) with one route
 // bit per 64-query half, which is what the sparse attention kernel walks.
 #include "subblock.h"
 #include "../../include/h3_policy.h"
 #include <algorithm>
 #include <cmath>
+#include <vector>
 
 namespace {
 
@@ -25,14 +27,21 @@ constexpr unsigned KEY_SPLIT = 16;         // 32-cell key tiles per score workgr
 
 // One thread per (cell, head, 8 channels): fp32 tree sum over the cell's 16
 // rows (missing rows are zero), mean * scale, rounded to BF16. 16-byte loads;
-// a workgroup covers 16 cells of one head.
+// a workgroup covers 16 cells of one head. The pools are written in the fragment
+// order of sb_score: its load of 16 channels of 32 cells is 1 KB in a row instead of
+// 32 row pieces of 32 bytes, which had kept the texture unit busy for longer than
+// everything else there (sb_score at 507 blocks and 40 heads: 207 -> 119 us).
+__host__ __device__ inline size_t pool_chunk(unsigned cell, unsigned part) {   // 8 channels from 8 * part
+    return ((size_t)(cell / 32) * 8 + part / 2) * 64 + part % 2 * 32 + cell % 32;
+}
+
 __global__ __launch_bounds__(256) void sb_pool(const uint16_t *q, const uint16_t *k, uint16_t *qpool,
                                                uint16_t *kpool, unsigned seq, unsigned heads, unsigned cells,
                                                float qscale, unsigned *fault) {
     const unsigned cell = blockIdx.x * 16 + threadIdx.x / 16, part = threadIdx.x % 16, head = blockIdx.y;
     const bool is_k = blockIdx.z != 0;
     const uint16_t *src = is_k ? k : q;
-    uint16_t *dst = (is_k ? kpool : qpool) + ((size_t)head * cells + cell) * D + part * 8;
+    uint16_t *dst = (is_k ? kpool : qpool) + (size_t)head * cells * D + pool_chunk(cell, part) * 8;
     const float scale = is_k ? 1.f : qscale;
     const unsigned start = cell * 16, count = start < seq ? min(16u, seq - start) : 0u;
     u16x8 raw[16];
@@ -59,13 +68,17 @@ __global__ __launch_bounds__(256) void sb_pool(const uint16_t *q, const uint16_t
     *reinterpret_cast<u16x8 *>(dst) = result;
 }
 
+template <int CTRL> __device__ inline float quad_move(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+constexpr int QUAD_XOR1 = 0xB1, QUAD_XOR2 = 0x4E;
 __device__ inline float quad_max(float x) {
-    x = fmaxf(x, __shfl_xor(x, 1, 64));
-    return fmaxf(x, __shfl_xor(x, 2, 64));
+    x = fmaxf(x, quad_move<QUAD_XOR1>(x));
+    return fmaxf(x, quad_move<QUAD_XOR2>(x));
 }
 __device__ inline float quad_sum(float x) {
-    x += __shfl_xor(x, 1, 64);
-    return x + __shfl_xor(x, 2, 64);
+    x += quad_move<QUAD_XOR1>(x);
+    return x + quad_move<QUAD_XOR2>(x);
 }
 
 // Scores for 32 query cells (8 query blocks) per wave against KEY_SPLIT tiles
@@ -89,7 +102,7 @@ __global__ __launch_bounds__(256) void sb_score(const uint16_t *qpool, const uin
     const uint16_t *kh = kpool + (size_t)head * cells * D;
     bf16x8 qf[8];
 #pragma unroll
-    for (int ks = 0; ks < 8; ks++) qf[ks] = *reinterpret_cast<const bf16x8 *>(qh + (size_t)qcell * D + ks * 16 + hf * 8);
+    for (int ks = 0; ks < 8; ks++) qf[ks] = *reinterpret_cast<const bf16x8 *>(qh + pool_chunk(qcell, 2 * ks + hf) * 8);
     const bool q_valid = qcell < valid;
     const unsigned ktiles = cells / 32;
     const unsigned kt0 = blockIdx.y * KEY_SPLIT, kt1 = min(ktiles, kt0 + KEY_SPLIT);
@@ -99,7 +112,7 @@ __global__ __launch_bounds__(256) void sb_score(const uint16_t *qpool, const uin
     auto load_k = [&](unsigned kt) {
 #pragma unroll
         for (int ks = 0; ks < 8; ks++)
-            kf[ks] = *reinterpret_cast<const bf16x8 *>(kh + (size_t)(kt * 32 + n) * D + ks * 16 + hf * 8);
+            kf[ks] = *reinterpret_cast<const bf16x8 *>(kh + pool_chunk(kt * 32 + n, 2 * ks + hf) * 8);
     };
     if (kt0 < kend) load_k(kt0);
     for (unsigned kt = kt0; kt < kend; kt++) {
@@ -142,79 +155,106 @@ __device__ inline uint32_t score_key(float f) {
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-// One workgroup per (query block of the slab [qb0, qb0 + qslab), head); rows
-// of scores, routes, lists and counts are slab-relative. Route rule and counters of the
-// reference's selection (cuda_subblock.cu:300-324): with
+// W waves per (query block of the slab [qb0, qb0 + qslab), head), four waves per
+// workgroup; rows of scores, routes, lists and counts are slab-relative. Route rule and
+// counters of the reference's selection (cuda_subblock.cu:300-324): with
 // rank(k) = #{j : s_j > s_k} + #{j < k : s_j == s_k}, key block k is kept
 // when rank < keep, when it is protected, when the query block is protected
-// or with force_all. rank(k) is k's position when the row is sorted by
-// descending score and ascending index, so a bitonic sort of
-// (key << 32 | ~index) in LDS gives every rank at once (P = next power of two
-// of B; padding sorts last). The kept blocks are then compacted in ascending
+// or with force_all. rank(k) < keep exactly when its key is above the keep-th largest
+// key T, or is T and fewer than keep - #{key > T} keys equal to T come before it. T is
+// found bit by bit from the top: a bit stays when at least `keep` keys reach it. Each
+// lane holds KEYS keys (wave w those from w * KEYS * 64), so a bit costs KEYS compares,
+// counted on the scalar unit. The kept blocks are compacted in ascending
 // order into the row's tile list; counts[row] is its length and
-// added_blocks[row] the protected key blocks kept beyond the top.
+// added_blocks[row] the protected key blocks kept beyond the top. One wave per row up to
+// 512 blocks, a workgroup above that (507 blocks, 40 heads, 20280 rows: 50 us, with a
+// bitonic sort of each row in LDS 229).
+template <int W, int KEYS>
 __global__ __launch_bounds__(256) void sb_select(const float *scores, uint8_t *routes, const uint8_t *q_protect,
-                                                 const uint8_t *k_protect, unsigned blocks, unsigned padded,
-                                                 unsigned keep, int force_all, unsigned qb0, unsigned qslab,
-                                                 uint32_t *lists, uint32_t *counts, uint32_t *added_blocks) {
-    extern __shared__ unsigned long long sortbuf[];   // [padded], then top flags [blocks]
-    uint8_t *top_flag = reinterpret_cast<uint8_t *>(sortbuf + padded);
-    __shared__ unsigned wave_total[4];
-    __shared__ unsigned red[4];
-    const unsigned tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-    const unsigned qb = qb0 + blockIdx.x, head = blockIdx.y;
-    const size_t row = (size_t)head * qslab + blockIdx.x;
-    const float *src = scores + row * blocks;
-    for (unsigned i = tid; i < padded; i += 256)
-        sortbuf[i] = i < blocks ? ((unsigned long long)score_key(src[i]) << 32) | (0xffffffffu - i) : 0ull;
-    __syncthreads();
-    // Descending bitonic sort.
-    for (unsigned size = 2; size <= padded; size <<= 1)
-        for (unsigned step = size >> 1; step; step >>= 1) {
-            for (unsigned t = tid; t < padded / 2; t += 256) {
-                const unsigned i = 2 * step * (t / step) + (t % step), j = i + step;
-                const unsigned long long x = sortbuf[i], y = sortbuf[j];
-                const bool descending = (i & size) == 0;
-                if (descending ? x < y : x > y) { sortbuf[i] = y; sortbuf[j] = x; }
-            }
-            __syncthreads();
-        }
-    for (unsigned i = tid; i < blocks; i += 256) top_flag[i] = 0;
-    __syncthreads();
-    for (unsigned p = tid; p < keep; p += 256) top_flag[0xffffffffu - (uint32_t)sortbuf[p]] = 1;
-    __syncthreads();
-
-    const bool pq = q_protect[qb] != 0;
-    uint32_t *list = lists + row * blocks;
-    uint8_t *route_row = routes + row * blocks;
-    unsigned offset = 0;
-    unsigned added = 0;
-    for (unsigned base = 0; base < blocks; base += 256) {
-        const unsigned k = base + tid;
-        bool retain = false;
-        if (k < blocks) {
-            const bool top = top_flag[k] != 0;
-            const bool protect = k_protect[k] != 0;
-            retain = force_all || pq || top || protect;
-            route_row[k] = (uint8_t)retain;
-            added += protect && !top && !pq && !force_all;
-        }
-        const unsigned long long mask = __ballot(retain);
-        const unsigned before = __popcll(mask & ((1ull << lane) - 1ull));
-        if (lane == 0) wave_total[wave] = __popcll(mask);
+                                                 const uint8_t *k_protect, unsigned blocks, unsigned keep,
+                                                 int force_all, unsigned qb0, unsigned qslab, uint32_t *lists,
+                                                 uint32_t *counts, uint32_t *added_blocks) {
+    __shared__ unsigned exchange[2][4];
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+    const unsigned block = blockIdx.x * (4 / W) + wave / W, part = wave % W, head = blockIdx.y;
+    if (block >= qslab) return;                       // W = 4: never, so the barriers are whole
+    const size_t row = (size_t)head * qslab + block;
+    const unsigned base = part * KEYS * 64 + lane;    // key j of this lane is block base + 64 j
+    // Sum over the row's waves; calls alternate between the two rows of `exchange`, so
+    // one barrier each is enough. `before`: the sum over the waves before this one.
+    unsigned turn = 0, before = 0;
+    auto row_sum = [&](unsigned x) {
+        if (W == 1) return x;
+        if (lane == 0) exchange[turn][part] = x;
         __syncthreads();
-        unsigned pos = offset + before;
-        for (unsigned w = 0; w < wave; w++) pos += wave_total[w];
-        if (retain) list[pos] = k;
-        offset += wave_total[0] + wave_total[1] + wave_total[2] + wave_total[3];
-        __syncthreads();
+        unsigned sum = 0;
+        before = 0;
+        for (unsigned w = 0; w < W; w++) {
+            before += w < part ? exchange[turn][w] : 0u;
+            sum += exchange[turn][w];
+        }
+        turn ^= 1;
+        return sum;
+    };
+    // Keys past the last block are 0 and never reach a candidate (all are above 0).
+    uint32_t key[KEYS];
+#pragma unroll
+    for (int j = 0; j < KEYS; j++) {
+        const unsigned k = base + j * 64;
+        key[j] = k < blocks ? score_key(scores[row * blocks + k]) : 0u;
     }
-    for (int off = 32; off; off >>= 1) added += __shfl_xor(added, off, 64);
-    if (lane == 0) red[wave] = added;
-    __syncthreads();
-    if (tid == 0) {
-        counts[row] = offset;
-        added_blocks[row] = red[0] + red[1] + red[2] + red[3];
+    uint32_t threshold = 0;
+    for (uint32_t bit = 0x80000000u; bit; bit >>= 1) {
+        const uint32_t candidate = threshold | bit;
+        unsigned reach = 0;
+#pragma unroll
+        for (int j = 0; j < KEYS; j++) reach += __popcll(__ballot(key[j] >= candidate));
+        if (row_sum(reach) >= keep) threshold = candidate;
+    }
+    unsigned above = 0, equal = 0;
+#pragma unroll
+    for (int j = 0; j < KEYS; j++) {
+        above += __popcll(__ballot(key[j] > threshold));
+        equal += __popcll(__ballot(base + j * 64 < blocks && key[j] == threshold));
+    }
+    const unsigned ties = keep - row_sum(above);      // keys equal to the threshold that are kept
+    row_sum(equal);
+    unsigned tied = before;                           // those before this wave's current 64
+
+    const bool all = force_all || q_protect[qb0 + block] != 0;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    uint8_t *route_row = routes + row * blocks;
+    uint32_t retained = 0;                            // bit j: key j is kept
+    unsigned kept = 0, added = 0;
+#pragma unroll
+    for (int j = 0; j < KEYS; j++) {
+        const unsigned k = base + j * 64;
+        const bool valid = k < blocks;
+        const unsigned long long same = __ballot(valid && key[j] == threshold);
+        const bool top = key[j] > threshold ||
+                         (valid && key[j] == threshold && tied + (unsigned)__popcll(same & below) < ties);
+        tied += __popcll(same);
+        const bool protect = valid && k_protect[k] != 0;
+        const bool retain = valid && (all || top || protect);
+        if (valid) route_row[k] = (uint8_t)retain;
+        retained |= (uint32_t)retain << j;
+        kept += __popcll(__ballot(retain));
+        added += __popcll(__ballot(protect && !top && !all));
+    }
+    kept = row_sum(kept);
+    unsigned pos = before;
+    uint32_t *list = lists + row * blocks;
+#pragma unroll
+    for (int j = 0; j < KEYS; j++) {
+        const bool retain = retained >> j & 1;
+        const unsigned long long mask = __ballot(retain);
+        if (retain) list[pos + (unsigned)__popcll(mask & below)] = base + j * 64;
+        pos += __popcll(mask);
+    }
+    added = row_sum(added);
+    if (part == 0 && lane == 0) {
+        counts[row] = kept;
+        added_blocks[row] = added;
     }
 }
 
@@ -246,7 +286,7 @@ int h3_subblock_bind(h3_gpu *g, h3_subblock_router *r, const h3_sol_layout *layo
         return h3_set_error(g, "SubBlock: missing layout");
     if (r->bound) return h3_set_error(g, "SubBlock: layout is already configured");
     const uint32_t seq = layout->sequence, blocks = (seq + 63) / 64;
-    // Selection sorts a row of 8-byte keys in LDS: at most 8192 blocks.
+    // Selection holds a row of keys in the registers of a workgroup: at most 8192 blocks.
     if (blocks > 8192) return h3_set_error(g, "SubBlock: sequence %u exceeds the router's limit", seq);
     if (layout->query_blocks != blocks || layout->key_blocks != blocks)
         return h3_set_error(g, "SubBlock: layout geometry differs from Q64/K64");
@@ -353,18 +393,9 @@ int h3_subblock_route(h3_gpu *g, h3_subblock_router *r, const uint16_t *q, const
     hipLaunchKernelGGL(sb_score, dim3((qslab * 4 + CELL_TILE - 1) / CELL_TILE, (ktiles + KEY_SPLIT - 1) / KEY_SPLIT, group),
                        dim3(256), 0, g->compute, qpool, kpool, scores, seq, cells, blocks, qb0, qslab, g->fault);
     if (!h3_launch_status(g, "SubBlock score")) return 0;
-    unsigned padded = 1;
-    while (padded < blocks) padded <<= 1;
-    const size_t shared = (size_t)padded * 8 + blocks;
-    static bool configured = false;
-    if (!configured) {
-        if (!h3_hip_check(g, hipFuncSetAttribute((const void *)sb_select, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 (int)(8192 * 8 + 8192)), "SubBlock select shared memory"))
-            return 0;
-        configured = true;
-    }
-    hipLaunchKernelGGL(sb_select, dim3(qslab, group), dim3(256), shared, g->compute, scores, base + r->off_routes,
-                       meta, meta + blocks, blocks, padded, keep, force_all ? 1 : 0, qb0, qslab,
+    const auto select = blocks <= 512 ? sb_select<1, 8> : blocks <= 2048 ? sb_select<4, 8> : sb_select<4, 32>;
+    hipLaunchKernelGGL(select, dim3(blocks <= 512 ? (qslab + 3) / 4 : qslab, group), dim3(256), 0, g->compute, scores,
+                       base + r->off_routes, meta, meta + blocks, blocks, keep, force_all ? 1 : 0, qb0, qslab,
                        (uint32_t *)(base + r->off_list), (uint32_t *)(base + r->off_count),
                        (uint32_t *)(base + r->off_added));
     if (!h3_launch_status(g, "SubBlock select")) return 0;
@@ -425,9 +456,13 @@ extern "C" int h3_hip_subblock_routes(h3_gpu *g, uint8_t *routes, float *scores,
         uint16_t *dst = which ? k_pool : q_pool;
         if (!dst) continue;
         const auto *src = (const uint16_t *)(base + (which ? r->off_kpool : r->off_qpool));
-        if (!h3_hip_check(g, hipMemcpy2D(dst, cells * D * 2, src, (size_t)r->cells * D * 2, cells * D * 2, r->heads,
-                                         hipMemcpyDeviceToHost), "pooled cells"))
-            return 0;
+        std::vector<uint16_t> pool((size_t)r->heads * r->cells * D);
+        if (!h3_hip_check(g, hipMemcpy(pool.data(), src, pool.size() * 2, hipMemcpyDeviceToHost), "pooled cells")) return 0;
+        for (size_t head = 0; head < r->heads; head++)
+            for (unsigned cell = 0; cell < cells; cell++)
+                for (unsigned part = 0; part < D / 8; part++)
+                    std::copy_n(&pool[head * r->cells * D + pool_chunk(cell, part) * 8], 8,
+                                dst + (head * cells + cell) * D + part * 8);
     }
     return 1;
 }

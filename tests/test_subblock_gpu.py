@@ -204,6 +204,39 @@ def test_constant_value_and_ties():
         g.close()
 
 
+@pytest.mark.parametrize("seq,period", [
+    (64 * 512, 0),        # the most blocks of one wave per row
+    (64 * 512 + 1, 37),   # the fewest of four waves, ties across all of them
+    (64 * 2048 + 30, 37), # the fewest of 32 keys per lane
+    (64 * 65, 7),         # two keys per lane, the second in one lane only
+])
+def test_selection_of_many_blocks(seq, period):
+    """Routes and counters equal a stable sort of the returned scores. With a
+    period the key blocks repeat, so that ties straddle the threshold."""
+    print(f"[subblock select] seq={seq} period={period}", flush=True)
+    rng = np.random.default_rng(seq)
+    blocks = (seq + 63) // 64
+    q = synth.f32_to_bf16(rng.standard_normal(seq * 128).astype(np.float32))
+    rows = np.arange(seq) % (64 * period) if period else np.arange(seq)
+    k = synth.f32_to_bf16(rng.standard_normal((seq, 128)).astype(np.float32) * 4)[rows].reshape(-1)
+    protect = np.zeros(blocks, np.uint8)
+    protect[[blocks // 2, blocks - 1]] = 1
+    g = make_router(seq, np.zeros(blocks, np.uint8), protect)
+    try:
+        sdpa(g, q, k, q, seq, 1, scale=SCALE, step=STEP, block=BLOCK)
+        routes, scores, _, _ = capture(g, seq, 1)
+        order = np.argsort(-scores[0], axis=1, kind="stable")
+        want = np.zeros((blocks, blocks), np.uint8)
+        np.put_along_axis(want, order[:, :keep_of(g, blocks)], 1, axis=1)
+        if period:
+            assert (np.sort(scores[0], axis=1)[:, 1:] == np.sort(scores[0], axis=1)[:, :-1]).any()
+        want[:, protect != 0] = 1
+        assert np.array_equal(routes[0], want)
+        assert stats(g).subblock_selected == int(want.sum())
+    finally:
+        g.close()
+
+
 def test_large_values_kind3():
     """Q = 100, K = +-100 by channel parity: every pooled dot is exactly 0, so
     the ranking is decided by index alone, and outputs are V means."""
