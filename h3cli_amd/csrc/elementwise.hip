@@ -33,20 +33,29 @@ struct AdaLNArgs {
     float eps;
 };
 
-// One wave per row. MODE 0: AdaLN. MODE 1 (gate_adaln): the row is first gated (residual + branch * gate,
+// One wave (W 1) or one workgroup (W 4) per row. MODE 0: AdaLN. MODE 1 (gate_adaln): the row is first gated (residual + branch * gate,
 // rounded to BF16 and stored) and the AdaLN then normalizes that BF16 row, as the
 // reference's two-kernel composition does (src/cuda/gpu_cuda.cu:1118-1120).
 // MODE 2: plain RMSNorm y = bf16(x * rsqrt(mean x^2 + eps) * w), no modulation
 // (src/cuda/cuda_kernels.cuh:805-833).
 enum { ADALN = 0, GATE_ADALN = 1, RMS_NORM = 2 };
-// CH: 16-byte chunks per lane (width <= 512 * CH); the row stays in registers
+// CH: 16-byte chunks per lane (width <= 512 * W * CH); the row stays in registers
 // as packed BF16 between the reduction and the output pass (exact: the value
 // normalized is the BF16 input, or the BF16-rounded gated row).
-template <int MODE, int CH>
+//
+// Latency-bound below a few thousand rows: a wave's chunks are one long chain of loads, and
+// 729 rows at four per workgroup leave a quarter of the CUs idle. With a workgroup per row
+// at width 5376, AdaLN / gate + AdaLN in microseconds: 32 rows 6.3 -> 4.2 / 8.7 -> 4.5, 729
+// rows 7.4 -> 5.5 / 11.1 -> 7.2, 2048 rows 11.1 -> 9.7 / 18.0 -> 15.5. Not at 3000 rows
+// (14.5, 14.7 / 21.8, 21.7), where bandwidth bounds both, nor at width 2048, a chunk per
+// lane (729 rows 4.6, 5.0 / 5.8, 5.1).
+constexpr unsigned ADALN_ROWS = 2048, ADALN_WIDTH = 4096;
+template <int MODE, int CH, int W>
 __global__ __launch_bounds__(256) void adaln_kernel(AdaLNArgs a) {
     constexpr bool GATE = MODE == GATE_ADALN;
-    const unsigned wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-    const unsigned row = blockIdx.x * 4 + wave;
+    constexpr unsigned STRIDE = 64 * W;
+    const unsigned wave = threadIdx.x / 64, lane = threadIdx.x % STRIDE;
+    const unsigned row = W == 4 ? blockIdx.x : blockIdx.x * 4 + wave;
     if (row >= a.rows) return;
     const unsigned chunks = a.width / 8;
     const size_t base = (size_t)row * a.width;
@@ -55,13 +64,13 @@ __global__ __launch_bounds__(256) void adaln_kernel(AdaLNArgs a) {
     float sumsq = 0.f;
 #pragma unroll
     for (int i = 0; i < CH; i++) {
-        const unsigned c = lane + 64 * i;
+        const unsigned c = lane + STRIDE * i;
         if (c >= chunks) break;
         raw[i] = *reinterpret_cast<const u16x8 *>(a.x + base + c * 8);
     }
 #pragma unroll
     for (int i = 0; i < CH; i++) {
-        const unsigned c = lane + 64 * i;
+        const unsigned c = lane + STRIDE * i;
         if (c >= chunks) break;
         if constexpr (GATE) {
             u16x8 br = *reinterpret_cast<const u16x8 *>(a.branch + base + c * 8);
@@ -77,10 +86,17 @@ __global__ __launch_bounds__(256) void adaln_kernel(AdaLNArgs a) {
             sumsq = fmaf(v, v, sumsq);
         }
     }
-    const float inv = rsqrtf(wave_sum(sumsq) / (float)a.width + a.eps);
+    sumsq = wave_sum(sumsq);
+    if constexpr (W == 4) {
+        __shared__ float part[4];
+        if (threadIdx.x % 64 == 0) part[wave] = sumsq;
+        __syncthreads();
+        sumsq = part[0] + part[1] + part[2] + part[3];
+    }
+    const float inv = rsqrtf(sumsq / (float)a.width + a.eps);
 #pragma unroll
     for (int i = 0; i < CH; i++) {
-        const unsigned c = lane + 64 * i;
+        const unsigned c = lane + STRIDE * i;
         if (c >= chunks) break;
         u16x8 wr = *reinterpret_cast<const u16x8 *>(a.weight + c * 8);
         u16x8 o;
@@ -103,9 +119,18 @@ __global__ __launch_bounds__(256) void adaln_kernel(AdaLNArgs a) {
 // Launch with the smallest chunk count that covers the row.
 template <int MODE>
 void launch_adaln(h3_gpu *g, const AdaLNArgs &a) {
+    const dim3 block(256);
+    if (a.width >= ADALN_WIDTH && a.rows <= ADALN_ROWS) {
+        switch ((a.width / 8 + 255) / 256) {
+#define H3_ADALN_CASE(n) case n: hipLaunchKernelGGL((adaln_kernel<MODE, n, 4>), dim3(a.rows), block, 0, g->compute, a); break;
+            H3_ADALN_CASE(2) H3_ADALN_CASE(3) default: H3_ADALN_CASE(4)
+#undef H3_ADALN_CASE
+        }
+        return;
+    }
     const unsigned per_lane = (a.width / 8 + 63) / 64;
-    const dim3 grid((a.rows + 3) / 4), block(256);
-#define H3_ADALN_CASE(n) case n: hipLaunchKernelGGL((adaln_kernel<MODE, n>), grid, block, 0, g->compute, a); break;
+    const dim3 grid((a.rows + 3) / 4);
+#define H3_ADALN_CASE(n) case n: hipLaunchKernelGGL((adaln_kernel<MODE, n, 1>), grid, block, 0, g->compute, a); break;
     switch (per_lane) {
         H3_ADALN_CASE(1) H3_ADALN_CASE(2) H3_ADALN_CASE(3) H3_ADALN_CASE(4) H3_ADALN_CASE(5) H3_ADALN_CASE(6)
         H3_ADALN_CASE(7) H3_ADALN_CASE(8) H3_ADALN_CASE(9) H3_ADALN_CASE(10) H3_ADALN_CASE(11) H3_ADALN_CASE(12)

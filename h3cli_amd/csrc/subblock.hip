@@ -10,9 +10,9 @@
 // matrix product, so scoring runs on the matrix cores (32 x 32 cell tiles,
 // fp32 accumulation of exact BF16 products) and the two log-sum-exps fold in
 // registers; the pools are stored in that product's fragment order. Selection finds each
-// row's threshold by bisection of its keys in registers. It writes the route bytes and, in the same pass, the
-// ordered list of kept 64-key tiles per (head, 128-query block) with one route
-// bit per 64-query half, which is what the sparse attention kernel walks.
+// row's threshold by bisection of its keys in registers. It writes the route bytes and, in
+// the same pass, the ordered list of kept 64-key tiles per (head, 64-query block), which is
+// what the sparse attention kernel walks.
 #include "subblock.h"
 #include "../../include/h3_policy.h"
 #include <algorithm>

@@ -366,6 +366,14 @@ def test_adaln(gpu, rows, width):
     assert d.max() <= 1 and d.mean() < 0.02
 
 
+@pytest.mark.parametrize("rows,width", [
+    (1, 4096), (2048, 4104), (3, 6152),   # a workgroup per row: whole chunks, one left over
+    (2049, 5376), (3, 4088),              # a wave per row: one row more, one chunk less
+])
+def test_adaln_row_split(gpu, rows, width):
+    test_adaln(gpu, rows, width)
+
+
 def test_gate_and_gate_adaln(gpu):
     rows, width = 129, 5120
     res = synth.normal_bf16(1, rows * width)
