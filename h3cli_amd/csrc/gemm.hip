@@ -323,7 +323,10 @@ void gemm_bf16_pipe(GemmArgs a) {
         for (int j = 0; j < 8; j++) {
             if (m0 + wm * 128 + j * 16 >= a.m) break;
 #pragma unroll
-            for (int i = 0; i < 8; i++) dst[(8 * j + i) * 256] = c[i][j];
+            for (int i = 0; i < 8; i++) {
+                hold(c[i][j]);
+                dst[(8 * j + i) * 256] = c[i][j];
+            }
         }
         return;
     }
@@ -335,7 +338,10 @@ void gemm_bf16_pipe(GemmArgs a) {
         if (row >= a.m) continue;
         f32x4 block[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) block[i] = c[i][j];
+        for (int i = 0; i < 8; i++) {
+            hold(c[i][j]);
+            block[i] = c[i][j];
+        }
         pipe_store<EPI>(a, row, n0 + wn * 128, q4, block);
     }
 }

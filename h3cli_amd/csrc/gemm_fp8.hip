@@ -208,11 +208,13 @@ void fp8_gemm_pipe(Fp8GemmArgs a) {
         for (int j = 0; j < 4; j++) {
             if (m0 + wm * 128 + j * 32 >= a.m) break;
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+            for (int i = 0; i < 4; i++) {
+                hold(c[i][j]);
 #pragma unroll
                 for (int g = 0; g < 4; g++)
                     dst[((j * 4 + i) * 4 + g) * 256] =
                         f32x4{c[i][j][4 * g], c[i][j][4 * g + 1], c[i][j][4 * g + 2], c[i][j][4 * g + 3]};
+            }
         }
         return;
     }
@@ -222,6 +224,7 @@ void fp8_gemm_pipe(Fp8GemmArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             f32x4 block[4];
+            hold(c[i][j]);
 #pragma unroll
             for (int g = 0; g < 4; g++)
                 block[g] = f32x4{c[i][j][4 * g], c[i][j][4 * g + 1], c[i][j][4 * g + 2], c[i][j][4 * g + 3]};

@@ -296,11 +296,13 @@ void gemm_q8_pipe(GemmArgs a) {
         for (int j = 0; j < 4; j++) {
             if (m0 + wm * 128 + j * 32 >= a.m) break;
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+            for (int i = 0; i < 4; i++) {
+                hold(c[i][j]);
 #pragma unroll
                 for (int r = 0; r < 4; r++)
                     dst[((j * 4 + i) * 4 + r) * 256] =
                         f32x4{c[i][j][4 * r], c[i][j][4 * r + 1], c[i][j][4 * r + 2], c[i][j][4 * r + 3]};
+            }
         }
         return;
     }
@@ -311,12 +313,13 @@ void gemm_q8_pipe(GemmArgs a) {
         for (int ip = 0; ip < 2; ip++) {
             f32x4 block[2][4];
 #pragma unroll
-            for (int h = 0; h < 2; h++)
+            for (int h = 0; h < 2; h++) {
+                f32x16 &x = c[2 * ip + h][j];
+                hold(x);
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const f32x16 &x = c[2 * ip + h][j];
+                for (int r = 0; r < 4; r++)
                     block[h][r] = f32x4{x[4 * r], x[4 * r + 1], x[4 * r + 2], x[4 * r + 3]};
-                }
+            }
             if (row < a.m) q8_store(a, row, n0 + wn * 128 + ip * 64, hf, block);
         }
     }

@@ -2,6 +2,8 @@
 its host-side logic (no GPU calls) matches the oracle."""
 import ctypes as C
 import re
+import struct
+import subprocess
 from pathlib import Path
 
 import numpy as np
@@ -108,3 +110,42 @@ def test_device_configure_validation(monkeypatch):
     finally:  # the C-level environment is not restored by monkeypatch
         libc.unsetenv(b"H3_CUDA_DEVICE")
         libc.unsetenv(b"H3_CUDA_WEIGHT_MODE")
+
+
+def device_kernels(tmp_path):
+    """(name, scratch bytes per lane, spilled vector registers) of every gfx950 kernel of
+    the library, from the metadata of its code objects."""
+    tools = Path("/opt/rocm/llvm/bin")
+    section = tmp_path / "fatbin"
+    subprocess.run([tools / "llvm-objcopy", f"--dump-section=.hip_fatbin={section}", _lib.LIB_PATH, tmp_path / "copy"],
+                   check=True)
+    data, magic, out = section.read_bytes(), b"__CLANG_OFFLOAD_BUNDLE__", []
+    at = data.find(magic)
+    while at >= 0:
+        count, = struct.unpack_from("<Q", data, at + 24)
+        p = at + 32
+        for _ in range(count):
+            offset, size, length = struct.unpack_from("<QQQ", data, p)
+            name = data[p + 24:p + 24 + length]
+            p += 24 + length
+            if b"gfx950" in name:
+                elf = tmp_path / "code.o"
+                elf.write_bytes(data[at + offset:at + offset + size])
+                notes = subprocess.run([tools / "llvm-readelf", "--notes", elf], check=True, capture_output=True,
+                                       text=True).stdout
+                for kernel in notes.split("- .agpr_count")[1:]:
+                    field = {k: re.search(rf"\.{k}:\s+(\S+)", kernel).group(1)
+                             for k in ("symbol", "private_segment_fixed_size", "vgpr_spill_count")}
+                    out.append((field["symbol"], int(field["private_segment_fixed_size"]),
+                                int(field["vgpr_spill_count"])))
+        at = data.find(magic, at + 24)
+    return out
+
+
+def test_hand_scheduled_projections_do_not_spill(tmp_path):
+    """Their accumulators fill the AGPRs; a register spilled around the K loop costs
+    every output tile several microseconds."""
+    kernels = [k for k in device_kernels(tmp_path)
+               if any(n in k[0] for n in ("gemm_bf16_pipe", "gemm_q8_pipe", "fp8_gemm_pipe", "8gemm_mid"))]
+    assert len(kernels) >= 24
+    assert not [k for k in kernels if k[1] or k[2]]
