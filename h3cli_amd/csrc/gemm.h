@@ -2,6 +2,7 @@
 // the launchers that h3_gemm chooses between.
 #pragma once
 #include "common.h"
+#include "internal.h"
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
@@ -33,6 +34,13 @@ inline GemmPlan gemm_last_wave(const h3_gpu *g, unsigned tiles, unsigned units, 
     return p;
 }
 
+// Split tiles of a launch. Tiles [0, full) are whole; each later one is taken by `split`
+// workgroups, whose FP32 partial sums go to part.
+struct TileSplit {
+    unsigned tiles, full, split;
+    float *part;
+};
+
 // Epilogue of h3_gemm after the bias. SwiGLU (no bias): the weight holds hidden gate
 // rows, then hidden up rows, n = 2 * hidden, and y is [m, hidden]; only where
 // h3_gemm_swiglu_fits.
@@ -47,10 +55,7 @@ struct GemmArgs {
     const float *alpha;       // EPI bit 2: device scalar multiplying the accumulator
     unsigned m, n, k, group, groups;
     int gelu;                 // H3_GEMM_PLAIN, _GELU or (pipe and mid kernels) _SWIGLU
-    // gemm_bf16_pipe and gemm_mid: tiles [0, full) are whole; each later one is split over K
-    // into `split` workgroups, whose FP32 partial sums go to part.
-    unsigned full, split;
-    float *part;
+    TileSplit tile;           // all kernels but gemm_skinny and gemm_small
 };
 
 __device__ inline float gelu_tanh(float v) {
@@ -74,6 +79,37 @@ __device__ inline float swiglu_fast(float gate, float up) {
 // front of the branch and spills 8 to 32 registers of the kernel (729 rows, 5376 -> 28672,
 // int8 of one scale per column: 246 us, without spills 213).
 template <class V> __device__ inline void hold(V &acc) { asm volatile("" : "+a"(acc)); }
+
+// The output tile (pid) of this workgroup, its place among the split ones (tile) and its
+// share of the K units: `ksteps` of them from `first` on (on entry those of a whole tile).
+// Behind whole waves tiles keep the places that they have in an unsplit launch, so that the
+// whole tiles of an XCD meet in its L2 as they do there, and the split ones are its last
+// (10000 rows, 5376 -> 28672, 17.5 waves: 2273 us unsplit; in two shares, whole and split
+// tiles placed each among themselves, 2394). Without whole waves the shares of one K range
+// are neighbours.
+struct TileShare {
+    unsigned pid, tile, share, first;
+    bool partial;
+};
+__device__ inline unsigned split_tile(const TileSplit &s, unsigned tile) {
+    return s.full ? xcd_remap(s.full + tile, s.tiles) : tile;
+}
+__device__ inline TileShare tile_share(const TileSplit &s, unsigned &ksteps) {
+    if (blockIdx.x < s.full) return {xcd_remap(blockIdx.x, s.tiles), 0, 0, 0, false};
+    const unsigned rest = s.tiles - s.full, at = s.full ? blockIdx.x - s.full : xcd_remap(blockIdx.x, gridDim.x);
+    const unsigned tile = at % rest, share = at / rest;
+    const unsigned first = share * ksteps / s.split;
+    ksteps = (share + 1) * ksteps / s.split - first;
+    return {split_tile(s, tile), tile, share, first, true};
+}
+// The tiles of a last, incomplete wave in `split` shares of their K units (each share has
+// one or more) of `values` partial sums, or whole where there is no memory for those.
+inline TileSplit split_last_wave(h3_gpu *g, unsigned tiles, unsigned split, unsigned units, size_t values) {
+    const unsigned rest = tiles % g->cus, shares = split < units ? split : units;
+    if (!rest || shares <= 1 || !h3_buffer_try(g, &g->gemm_partials, (size_t)rest * shares * values * 4))
+        return {tiles, tiles, 1, nullptr};
+    return {tiles, tiles - rest, shares, (float *)g->gemm_partials.ptr};
+}
 
 // Tile (row, column) of workgroup pid: bands of at most `rows` row tiles sweep the
 // columns together, so that the workgroups an XCD runs at a time share both operands in

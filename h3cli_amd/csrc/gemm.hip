@@ -223,23 +223,14 @@ void gemm_bf16_pipe(GemmArgs a) {
     const unsigned tid = threadIdx.x, lane = tid % 64, n16 = lane % 16, q4 = lane / 16;
     const unsigned wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const unsigned wm = wave / 2, wn = wave % 2;
-    // Whole tiles first; a split tile's workgroups take the K stage pairs in
-    // `split` consecutive shares. Neighbouring workgroups share a K range.
-    unsigned pid, share = 0, k0 = 0, ksteps = a.k / TK;
-    const bool partial = SPLIT && blockIdx.x >= a.full;
-    if (!partial) {
-        pid = xcd_remap(blockIdx.x, SPLIT ? a.full : gridDim.x);
-    } else {
-        const unsigned count = gridDim.x - a.full, rest = count / a.split;
-        const unsigned id = xcd_remap(blockIdx.x - a.full, count);
-        share = id / rest;
-        pid = a.full + id % rest;
-        const unsigned pairs = ksteps / 2, p0 = share * pairs / a.split, p1 = (share + 1) * pairs / a.split;
-        k0 = p0 * 2 * TK;
-        ksteps = (p1 - p0) * 2;
-    }
+    // K units: stage pairs.
+    unsigned units = a.k / (2 * TK);
+    TileShare t{};
+    if constexpr (SPLIT) t = tile_share(a.tile, units);
+    else t.pid = xcd_remap(blockIdx.x, gridDim.x);
+    const unsigned k0 = t.first * 2 * TK, ksteps = units * 2;
     unsigned m0, n0;
-    pipe_tile(a, pid, m0, n0);
+    pipe_tile(a, t.pid, m0, n0);
 
     const uint64_t xbase = (uint64_t)(a.x + (size_t)m0 * a.k + k0);
     const unsigned wrow = EPI & 8 ? n0 / 2 : n0, wrows = EPI & 8 ? a.n / 2 + TN / 2 : TN;
@@ -315,10 +306,11 @@ void gemm_bf16_pipe(GemmArgs a) {
           [mb] "s"(mb), [kmax] "s"(kmax), [pw0] "v"(pw[0]), [pw1] "v"(pw[1]), [px0] "v"(px[0]), [px1] "v"(px[1])
         : "m0", "scc", "memory");
 
-    if (partial) {
+    if (SPLIT && t.partial) {
         // Partial sums of (split tile, share): element (i, j) of thread t at
         // ((8 j + i) * 256 + t), so that every store instruction is contiguous.
-        f32x4 *dst = reinterpret_cast<f32x4 *>(a.part) + ((size_t)(pid - a.full) * a.split + share) * (TM * TN / 4) + tid;
+        f32x4 *dst = reinterpret_cast<f32x4 *>(a.tile.part) +
+                     ((size_t)t.tile * a.tile.split + t.share) * (TM * TN / 4) + tid;
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             if (m0 + wm * 128 + j * 16 >= a.m) break;
@@ -353,15 +345,15 @@ __global__ __launch_bounds__(256) void gemm_pipe_reduce(GemmArgs a) {
     const unsigned tile = blockIdx.x / 8, j = blockIdx.x % 8, tid = threadIdx.x;
     const unsigned lane = tid % 64, wave = tid / 64, n16 = lane % 16, q4 = lane / 16;
     unsigned m0, n0;
-    pipe_tile(a, a.full + tile, m0, n0);
+    pipe_tile(a, split_tile(a.tile, tile), m0, n0);
     const unsigned row = m0 + (wave / 2) * 128 + j * 16 + n16;
     if (row >= a.m) return;
-    const f32x4 *src = reinterpret_cast<const f32x4 *>(a.part) + (size_t)tile * a.split * (TM * TN / 4) + 8 * j * 256 + tid;
+    const f32x4 *src = reinterpret_cast<const f32x4 *>(a.tile.part) + (size_t)tile * a.tile.split * (TM * TN / 4) + 8 * j * 256 + tid;
     f32x4 block[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) block[i] = src[i * 256];
 #pragma unroll 4
-    for (unsigned s = 1; s < a.split; s++) {
+    for (unsigned s = 1; s < a.tile.split; s++) {
         src += TM * TN / 4;
 #pragma unroll
         for (int i = 0; i < 8; i++) block[i] += src[i * 256];
@@ -381,17 +373,13 @@ int launch_pipe(h3_gpu *g, GemmArgs a, unsigned split, bool timed) {
         configured = true;
     }
     const unsigned tiles = (a.m + TM - 1) / TM * (a.n / TN);
-    unsigned rest = tiles % g->cus;
-    a.split = split < a.k / (2 * TK) ? split : a.k / (2 * TK);   // every share has a stage pair
-    if (a.split > 1 && !h3_buffer_try(g, &g->gemm_partials, (size_t)rest * a.split * TM * TN * 4)) a.split = 1;
-    if (a.split == 1) rest = 0;
-    a.full = tiles - rest;
-    a.part = (float *)g->gemm_partials.ptr;
+    a.tile = split_last_wave(g, tiles, split, a.k / (2 * TK), TM * TN);
+    const unsigned rest = tiles - a.tile.full;
     hipEvent_t timing = timed ? h3_kernel_timing_begin(g) : nullptr;
     if (!rest) {
         hipLaunchKernelGGL((gemm_bf16_pipe<EPI, false>), dim3(tiles), dim3(256), shared, g->compute, a);
     } else {
-        hipLaunchKernelGGL((gemm_bf16_pipe<EPI, true>), dim3(a.full + rest * a.split), dim3(256), shared, g->compute, a);
+        hipLaunchKernelGGL((gemm_bf16_pipe<EPI, true>), dim3(a.tile.full + rest * a.tile.split), dim3(256), shared, g->compute, a);
         if (h3_launch_status(g, "BF16 GEMM"))
             hipLaunchKernelGGL(gemm_pipe_reduce<EPI>, dim3(rest * 8), dim3(256), 0, g->compute, a);
     }

@@ -119,21 +119,13 @@ void fp8_gemm_pipe(Fp8GemmArgs a) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     const unsigned tid = threadIdx.x, lane = tid % 64, n32 = lane % 32, hf = lane / 32;
     const unsigned wave = __builtin_amdgcn_readfirstlane(tid / 64), wm = wave / 2, wn = wave % 2;
-    unsigned pid, share = 0, k0 = 0, ksteps = a.k / TK;
-    const bool partial = SPLIT && blockIdx.x >= a.full;
-    if (!partial) {
-        pid = xcd_remap(blockIdx.x, SPLIT ? a.full : gridDim.x);
-    } else {
-        const unsigned count = gridDim.x - a.full, rest = count / a.split;
-        const unsigned id = xcd_remap(blockIdx.x - a.full, count);
-        share = id / rest;
-        pid = a.full + id % rest;
-        const unsigned s0 = share * ksteps / a.split, s1 = (share + 1) * ksteps / a.split;
-        k0 = s0 * TK;
-        ksteps = s1 - s0;
-    }
+    unsigned ksteps = a.k / TK;
+    TileShare t{};
+    if constexpr (SPLIT) t = tile_share(a.tile, ksteps);
+    else t.pid = xcd_remap(blockIdx.x, gridDim.x);
+    const unsigned k0 = t.first * TK;
     unsigned m0, n0;
-    fp8_tile(a, pid, m0, n0);
+    fp8_tile(a, t.pid, m0, n0);
     const uint64_t xbase = (uint64_t)(a.x + (size_t)m0 * a.k + k0), wbase = (uint64_t)(a.w + (size_t)n0 * a.k + k0);
     const unsigned xrows = min(a.m - m0, (unsigned)TM), wrows = min(a.n - n0, (unsigned)TN);
     // Rows past M or N are past the resources' size and load zeros.
@@ -202,8 +194,9 @@ void fp8_gemm_pipe(Fp8GemmArgs a) {
 
     // Block (i, j): lane holds output row m0 + 128 wm + 32 j + n32.
     const float scale = a.sx[0] * a.sw[0];
-    if (partial) {
-        f32x4 *dst = reinterpret_cast<f32x4 *>(a.part) + ((size_t)(pid - a.full) * a.split + share) * (TM * TN / 4) + tid;
+    if (SPLIT && t.partial) {
+        f32x4 *dst = reinterpret_cast<f32x4 *>(a.tile.part) +
+                     ((size_t)t.tile * a.tile.split + t.share) * (TM * TN / 4) + tid;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             if (m0 + wm * 128 + j * 32 >= a.m) break;
@@ -239,16 +232,16 @@ __global__ __launch_bounds__(256) void fp8_gemm_reduce(Fp8GemmArgs a) {
     const unsigned tile = blockIdx.x / 16, j = blockIdx.x % 16 / 4, i = blockIdx.x % 4;
     const unsigned tid = threadIdx.x, wave = tid / 64, lane = tid % 64, n32 = lane % 32, hf = lane / 32;
     unsigned m0, n0;
-    fp8_tile(a, a.full + tile, m0, n0);
+    fp8_tile(a, split_tile(a.tile, tile), m0, n0);
     const unsigned row = m0 + wave / 2 * 128 + j * 32 + n32;
     if (row >= a.m) return;
-    const f32x4 *src = reinterpret_cast<const f32x4 *>(a.part) + (size_t)tile * a.split * (TM * TN / 4) +
+    const f32x4 *src = reinterpret_cast<const f32x4 *>(a.tile.part) + (size_t)tile * a.tile.split * (TM * TN / 4) +
                        (j * 4 + i) * 4 * 256 + tid;
     f32x4 block[4];
 #pragma unroll
     for (int g = 0; g < 4; g++) block[g] = src[g * 256];
 #pragma unroll 4
-    for (unsigned s = 1; s < a.split; s++) {
+    for (unsigned s = 1; s < a.tile.split; s++) {
         src += TM * TN / 4;
 #pragma unroll
         for (int g = 0; g < 4; g++) block[g] += src[g * 256];
@@ -269,20 +262,17 @@ int h3_gemm_fp8(h3_gpu *g, Fp8GemmArgs a) {
         configured = true;
     }
     const unsigned tiles = (a.m + TM - 1) / TM * ((a.n + TN - 1) / TN);
-    unsigned rest = tiles % g->cus;
     // Shared over K where all tiles are less than one wave, at 1.5 us per K tile, in
     // shares of eight K tiles or more, so that short sums keep one order. Behind whole
     // waves it does not pay (8193 rows, 5376 -> 28672: 1092 us, split 1125).
-    a.split = tiles < g->cus ? gemm_last_wave(g, tiles, a.k / TK, 1.5f, 0.09f, 512, 8).split : 1;
-    if (a.split > 1 && !h3_buffer_try(g, &g->gemm_partials, (size_t)rest * a.split * TM * TN * 4)) a.split = 1;
-    if (a.split == 1) rest = 0;
-    a.full = tiles - rest;
-    a.part = (float *)g->gemm_partials.ptr;
+    const unsigned split = tiles < g->cus ? gemm_last_wave(g, tiles, a.k / TK, 1.5f, 0.09f, 512, 8).split : 1;
+    a.tile = split_last_wave(g, tiles, split, a.k / TK, TM * TN);
+    const unsigned rest = tiles - a.tile.full;
     hipEvent_t timing = h3_kernel_timing_begin(g);
     if (!rest) {
         hipLaunchKernelGGL(fp8_gemm_pipe<false>, dim3(tiles), dim3(256), LDS, g->compute, a);
     } else {
-        hipLaunchKernelGGL(fp8_gemm_pipe<true>, dim3(a.full + rest * a.split), dim3(256), LDS, g->compute, a);
+        hipLaunchKernelGGL(fp8_gemm_pipe<true>, dim3(a.tile.full + rest * a.tile.split), dim3(256), LDS, g->compute, a);
         if (h3_launch_status(g, "native fp8 projection"))
             hipLaunchKernelGGL(fp8_gemm_reduce, dim3(rest * 16), dim3(256), 0, g->compute, a);
     }

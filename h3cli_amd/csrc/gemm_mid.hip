@@ -137,23 +137,12 @@ void gemm_mid(GemmArgs a) {
     uint8_t *const ws_deq = scs + D * scale_bytes<W, TM>();
     const unsigned tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
     const unsigned n32 = lane % 32, hf = lane / 32, wm = wave / 4, wn = wave % 4;
-    unsigned pid, share = 0, k0 = 0, ksteps = a.k / TK;
-    const bool partial = blockIdx.x >= a.full;
-    if (!partial) {
-        pid = xcd_remap(blockIdx.x, a.full);
-    } else {
-        const unsigned count = gridDim.x - a.full, rest = count / a.split;
-        const unsigned id = xcd_remap(blockIdx.x - a.full, count);
-        share = id / rest;
-        pid = a.full + id % rest;
-        const unsigned s0 = share * ksteps / a.split, s1 = (share + 1) * ksteps / a.split;
-        k0 = s0 * TK;
-        ksteps = s1 - s0;
-    }
-    k0 = __builtin_amdgcn_readfirstlane(k0);
+    unsigned ksteps = a.k / TK;
+    const TileShare t = tile_share(a.tile, ksteps);
+    const unsigned k0 = __builtin_amdgcn_readfirstlane(t.first * TK);
     ksteps = __builtin_amdgcn_readfirstlane(ksteps);
     unsigned m0, n0;
-    mid_tile<TM>(a, pid, m0, n0);
+    mid_tile<TM>(a, t.pid, m0, n0);
 
     // Rows past M or N are past the resources' size and load zeros (SwiGLU: up rows
     // past the end; gate rows past it are up rows, whose columns are not stored).
@@ -308,8 +297,9 @@ void gemm_mid(GemmArgs a) {
     auto part4 = [&](int i, int j, int g) {
         return f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
     };
-    if (partial) {
-        f32x4 *dst = reinterpret_cast<f32x4 *>(a.part) + ((size_t)(pid - a.full) * a.split + share) * (TM * TN / 4) + tid;
+    if (t.partial) {
+        f32x4 *dst = reinterpret_cast<f32x4 *>(a.tile.part) +
+                     ((size_t)t.tile * a.tile.split + t.share) * (TM * TN / 4) + tid;
 #pragma unroll
         for (int j = 0; j < NBM; j++) {
             if (m0 + wm * (TM / 2) + j * 32 >= a.m) break;
@@ -336,13 +326,14 @@ __global__ __launch_bounds__(T) void gemm_mid_reduce(GemmArgs a) {
     const unsigned tile = blockIdx.x / BLOCKS, j = blockIdx.x % BLOCKS / 4, g = blockIdx.x % 4;
     const unsigned tid = threadIdx.x, wave = tid / 64, lane = tid % 64, n32 = lane % 32, hf = lane / 32;
     unsigned m0, n0;
-    mid_tile<TM>(a, a.full + tile, m0, n0);
+    mid_tile<TM>(a, split_tile(a.tile, tile), m0, n0);
     const unsigned row = m0 + wave / 4 * (TM / 2) + j * 32 + n32;
     if (row >= a.m) return;
-    const f32x4 *src = reinterpret_cast<const f32x4 *>(a.part) + (size_t)tile * a.split * (TM * TN / 4) + (j * 8 + g) * T + tid;
+    const f32x4 *src = reinterpret_cast<const f32x4 *>(a.tile.part) +
+                       (size_t)tile * a.tile.split * (TM * TN / 4) + (j * 8 + g) * T + tid;
     f32x4 v0 = src[0], v1 = src[4 * T];
 #pragma unroll 4
-    for (unsigned s = 1; s < a.split; s++) {
+    for (unsigned s = 1; s < a.tile.split; s++) {
         src += TM * TN / 4;
         v0 += src[0];
         v1 += src[4 * T];
@@ -363,14 +354,10 @@ int launch(h3_gpu *g, GemmArgs a, unsigned split, bool timed) {
         configured = true;
     }
     const unsigned tiles = (a.m + TM - 1) / TM * ((a.n + TN - 1) / TN);
-    unsigned rest = tiles % g->cus;
-    a.split = split < a.k / TK ? split : a.k / TK;   // every share has a K step
-    if (a.split > 1 && !h3_buffer_try(g, &g->gemm_partials, (size_t)rest * a.split * TM * TN * 4)) a.split = 1;
-    if (a.split == 1) rest = 0;
-    a.full = tiles - rest;
-    a.part = (float *)g->gemm_partials.ptr;
+    a.tile = split_last_wave(g, tiles, split, a.k / TK, TM * TN);
+    const unsigned rest = tiles - a.tile.full;
     hipEvent_t timing = timed ? h3_kernel_timing_begin(g) : nullptr;
-    hipLaunchKernelGGL(kernel, dim3(a.full + rest * a.split), dim3(T), shared, g->compute, a);
+    hipLaunchKernelGGL(kernel, dim3(a.tile.full + rest * a.tile.split), dim3(T), shared, g->compute, a);
     if (rest && h3_launch_status(g, "GEMM"))
         hipLaunchKernelGGL(gemm_mid_reduce<TM>, dim3(rest * (TM / 64) * 4), dim3(T), 0, g->compute, a);
     h3_kernel_timing_end(g, timing);

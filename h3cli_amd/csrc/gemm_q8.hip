@@ -179,21 +179,11 @@ void gemm_q8_pipe(GemmArgs a) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     const unsigned tid = threadIdx.x, lane = tid % 64, n32 = lane % 32, hf = lane / 32;
     const unsigned wave = __builtin_amdgcn_readfirstlane(tid / 64), wm = wave / 2, wn = wave % 2;
-    unsigned pid, share = 0, k0 = 0, ksteps = a.k / TK;
-    const bool partial = blockIdx.x >= a.full;
-    if (!partial) {
-        pid = xcd_remap(blockIdx.x, a.full);
-    } else {
-        const unsigned count = gridDim.x - a.full, rest = count / a.split;
-        const unsigned id = xcd_remap(blockIdx.x - a.full, count);
-        share = id / rest;
-        pid = a.full + id % rest;
-        const unsigned s0 = share * ksteps / a.split, s1 = (share + 1) * ksteps / a.split;
-        k0 = s0 * TK;
-        ksteps = s1 - s0;
-    }
+    unsigned ksteps = a.k / TK;
+    const TileShare t = tile_share(a.tile, ksteps);
+    const unsigned k0 = t.first * TK;
     unsigned m0, n0;
-    q8_tile(a, pid, m0, n0);
+    q8_tile(a, t.pid, m0, n0);
     const unsigned first = a.gelu == H3_GEMM_SWIGLU ? n0 / 2 : n0;
     const unsigned wrows = a.gelu == H3_GEMM_SWIGLU ? a.n - first : min(a.n - n0, (unsigned)TN);
     const uint64_t xbase = (uint64_t)(a.x + (size_t)m0 * a.k + k0);
@@ -290,8 +280,9 @@ void gemm_q8_pipe(GemmArgs a) {
           "memory");
 
     // Block (i, j): lane holds output row m0 + 128 wm + 32 j + n32.
-    if (partial) {
-        f32x4 *dst = reinterpret_cast<f32x4 *>(a.part) + ((size_t)(pid - a.full) * a.split + share) * (TM * TN / 4) + tid;
+    if (t.partial) {
+        f32x4 *dst = reinterpret_cast<f32x4 *>(a.tile.part) +
+                     ((size_t)t.tile * a.tile.split + t.share) * (TM * TN / 4) + tid;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             if (m0 + wm * 128 + j * 32 >= a.m) break;
@@ -331,16 +322,16 @@ __global__ __launch_bounds__(256) void gemm_q8_reduce(GemmArgs a) {
     const unsigned tile = blockIdx.x / 8, j = blockIdx.x % 8 / 2, ip = blockIdx.x % 2;
     const unsigned tid = threadIdx.x, wave = tid / 64, lane = tid % 64, n32 = lane % 32, hf = lane / 32;
     unsigned m0, n0;
-    q8_tile(a, a.full + tile, m0, n0);
+    q8_tile(a, split_tile(a.tile, tile), m0, n0);
     const unsigned row = m0 + wave / 2 * 128 + j * 32 + n32;
     if (row >= a.m) return;
-    const f32x4 *src = reinterpret_cast<const f32x4 *>(a.part) + (size_t)tile * a.split * (TM * TN / 4) +
+    const f32x4 *src = reinterpret_cast<const f32x4 *>(a.tile.part) + (size_t)tile * a.tile.split * (TM * TN / 4) +
                        (j * 4 + 2 * ip) * 4 * 256 + tid;
     f32x4 block[2][4];
 #pragma unroll
     for (int r = 0; r < 8; r++) block[r / 4][r % 4] = src[r * 256];
 #pragma unroll 2
-    for (unsigned s = 1; s < a.split; s++) {
+    for (unsigned s = 1; s < a.tile.split; s++) {
         src += TM * TN / 4;
 #pragma unroll
         for (int r = 0; r < 8; r++) block[r / 4][r % 4] += src[r * 256];
@@ -366,14 +357,10 @@ int h3_gemm_q8(h3_gpu *g, GemmArgs a, unsigned split) {
         configured = true;
     }
     const unsigned tiles = (a.m + TM - 1) / TM * ((a.n + TN - 1) / TN);
-    unsigned rest = tiles % g->cus;
-    a.split = split < a.k / TK ? split : a.k / TK;   // every share has a K tile
-    if (a.split > 1 && !h3_buffer_try(g, &g->gemm_partials, (size_t)rest * a.split * TM * TN * 4)) a.split = 1;
-    if (a.split == 1) rest = 0;
-    a.full = tiles - rest;
-    a.part = (float *)g->gemm_partials.ptr;
+    a.tile = split_last_wave(g, tiles, split, a.k / TK, TM * TN);
+    const unsigned rest = tiles - a.tile.full;
     hipEvent_t timing = h3_kernel_timing_begin(g);
-    hipLaunchKernelGGL(gemm_q8_pipe, dim3(a.full + rest * a.split), dim3(256), LDS, g->compute, a);
+    hipLaunchKernelGGL(gemm_q8_pipe, dim3(a.tile.full + rest * a.tile.split), dim3(256), LDS, g->compute, a);
     if (rest && h3_launch_status(g, "W8A16 GEMM"))
         hipLaunchKernelGGL(gemm_q8_reduce, dim3(rest * 8), dim3(256), 0, g->compute, a);
     h3_kernel_timing_end(g, timing);
