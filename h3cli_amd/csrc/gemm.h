@@ -15,22 +15,37 @@ struct GemmPlan {
     bool dequant;         // W8A16: convert the whole weight to BF16 first
 };
 
-// Modelled time in microseconds of tiles output tiles of `units` K units, unit_us
-// each: start_us more per workgroup, share_us per share of a split tile for its partial sums
-// written and read, 3 for the reduction launch and 0.9 for each share added in turn.
-// At most `most` shares in all (128 MB), each of `least_units` or more.
-inline GemmPlan gemm_last_wave(const h3_gpu *g, unsigned tiles, unsigned units, float unit_us, float share_us, unsigned most,
-                               unsigned least_units = 1, float start_us = 2.f) {
-    const unsigned rest = tiles % g->cus;
-    GemmPlan p{(float)(tiles / g->cus) * (units * unit_us + start_us), 0, 1, false};
-    if (!rest) return p;
-    float least = units * unit_us + start_us;
-    for (unsigned s = 2; s <= 32 && s * least_units <= units && rest * s <= most; s++) {
-        const float waves = (float)((rest * s + g->cus - 1) / g->cus);
-        const float t = waves * ((units + s - 1) / s * unit_us + start_us) + rest * s * share_us + 3.f + 0.9f * s;
-        if (t < least) { least = t; p.split = s; }
+// Measured rates of a kernel in microseconds, one workgroup on each CU: a K unit of a tile in
+// a whole wave (full); in a wave that occupies a part f of the CUs, part + rise * max(0, f -
+// knee), because fewer busy CUs draw less power and clock higher (7168 -> 5376, BF16, 84 /
+// 168 / 252 tiles: 114 / 128 / 153); start per round of workgroups; and for split tiles
+// their second launch (fixed), each share's 256 x 256 partial sums (sum) and each share added
+// in turn (turn).
+struct GemmRates {
+    float full, part, rise, knee, start, fixed, sum, turn;
+};
+
+// The modelled time of `tiles` output tiles of `units` K units, `size` times 256 x 256 each, and
+// the number of shares of the tiles of the last wave that it is least for. Shares run in one
+// round of the CUs: half of a wave or more stays whole (7168 -> 5376, BF16: 84 tiles in 3
+// shares 72 us (whole 114), in 4, so two rounds, 96; 168 tiles whole 128, in 3 shares 146).
+// Behind one whole wave also two rounds (14336 -> 5376, 420 tiles: 3 shares 621, whole 658),
+// behind eight or more none: what is left to gain is within the noise (5376 -> 28672, 8193
+// rows, 14.4 waves: 1788 either way).
+inline GemmPlan gemm_last_wave(const h3_gpu *g, unsigned tiles, unsigned units, const GemmRates &r, float size = 1.f,
+                               unsigned least_units = 1) {
+    const unsigned rest = tiles % g->cus, waves = tiles / g->cus, rounds_max = waves == 1 ? 2 : 1;
+    auto unit = [&](float busy) { return r.part + r.rise * (busy > r.knee ? busy - r.knee : 0.f); };
+    const float before = (float)waves * units * r.full + r.start;
+    GemmPlan p{before + (rest ? units * unit((float)rest / g->cus) : 0.f), 0, 1, false};
+    if (!rest || waves >= 8) return p;
+    for (unsigned s = 2; s <= 32 && s * least_units <= units && rest * s <= rounds_max * g->cus; s++) {
+        const unsigned rounds = (rest * s + g->cus - 1) / g->cus;
+        const float busy = (float)(rest * s) / (rounds * g->cus);
+        const float t = before + rounds * ((units + s - 1) / s * unit(busy) + r.start) - r.start + r.fixed +
+                        rest * s * size * r.sum + s * r.turn;
+        if (t < p.us) { p.us = t; p.split = s; }
     }
-    p.us += least;
     return p;
 }
 

@@ -529,42 +529,48 @@ int launch_small(h3_gpu *g, const GemmArgs &a, bool q8) {
 }
 
 // ------------------------------------------------------------ choice of the kernel
-// The faster of the kernels that take this projection, by the model above with these
-// rates (microseconds per 64 values of K, one workgroup on each CU, measured at 64 to
-// 8193 rows): pipe 1.5; mid, BF16 weights 1.0 / 1.2 / 1.95 for 64 / 128 / 256 rows;
-// mid, int8 weights 1.3 / 1.25 / 2.1; q8 1.72, and 10 to fill its stages and to store;
-// converting a weight to BF16 first 0.5 per million values. Measured, in microseconds,
-// the runner-up in brackets: 63 tiles of 256 (729 rows, 7168 -> 5376), BF16: pipe in 4
-// shares 66.6 (unsplit 134.6); 336 tiles (729 rows, 5376 -> 28672), BF16: pipe, the last
-// 80 tiles in 3 shares, 201.8 (242.6); 693 tiles (8193 rows, 14336 -> 5376): unsplit 998
-// (2 shares 1018); 729 rows, 5376 -> 28672, int8 of group 64: mid 256 in 3 shares 247
-// (pipe 287), one scale per column: q8 in 3 shares 246 (mid 265); 1200 rows, 13824 ->
-// 5120, per column: q8 in 2 shares 197 (pipe 211); 2000 rows, 5120 -> 5120, int8: pipe
-// 117 (q8 124, mid 140); 700 rows, 1024 -> 14336, per column: mid 256 40.4 (q8 46.8);
-// 300 rows, 7168 -> 5376, BF16: mid 128 in 4 shares 38.7 (pipe 50.9); 8193 rows,
-// 5440 -> 5120, group 64, which pipe does not take: converted first 442 (mid 475).
+// The fastest of the kernels that take this projection, by gemm_last_wave with rates fitted
+// to the measured times of all plans of eight projections (K, N 5120 to 28672) of 33 to 24000
+// rows, BF16, int8 with one scale per column and int8 of group 64: the plan taken is 0.5%
+// slower than the best one in the mean, 13% at most, and never 2% slower than whole tiles of
+// the pipe kernel. Converting a weight to BF16 first takes 0.4 to 1.2 us per million values,
+// most for a long K, whose rows share the cache with the weight. What is not the pipe kernel
+// on whole tiles must promise 2%. Measured, in microseconds, the runner-up in brackets: 729
+// rows, 7168 -> 5376, BF16: pipe in 4 shares 61 (whole 113); 729 rows, 5376 -> 28672, int8 of
+// group 64: mid 256 in 3 shares 260 (pipe in 3 281), per column: q8 in 3 shares 213 (mid 240);
+// 729 rows, 5120 -> 13824, group 64: pipe 122 (mid 151); 1800 rows, 14336 -> 5376, per column:
+// q8 292 (pipe 315); 64 rows, 5376 -> 28672, BF16: mid 64 in 2 shares 61 (pipe 114).
 GemmPlan choose(const h3_gpu *g, const GemmArgs &a, bool q8) {
-    static constexpr float BF16_STEP[3] = {1.0f, 1.2f, 1.95f}, Q8_STEP[3] = {1.3f, 1.25f, 2.1f};
+    static constexpr GemmRates PIPE{2.89f, 1.96f, 1.72f, .65f, 6.4f, .6f, .044f, .41f};      // per 128 values of K
+    static constexpr GemmRates CODES{1.73f, 1.22f, .93f, .57f, 8.5f, 1.3f, .03f, .95f};      // gemm_q8; per 64, as all below
+    static constexpr GemmRates MID_BF16[3] = {{.61f, .5f, .58f, .74f, 4.1f, 1.4f, .085f, .39f},
+                                              {.98f, .75f, .65f, .66f, 3.8f, .7f, .083f, .02f},
+                                              {1.95f, 1.5f, .8f, .55f, 3.f, 5.f, .04f, 0.f}};
+    static constexpr GemmRates MID_COLUMN[3] = {{.88f, .74f, .22f, .47f, 4.7f, 5.f, .042f, .11f},
+                                                {1.17f, 1.03f, .19f, .2f, 2.5f, 5.f, .057f, 0.f},
+                                                {1.94f, 1.4f, .6f, .2f, 3.4f, 8.3f, .03f, 0.f}};
+    static constexpr GemmRates MID_GROUP[3] = {{1.08f, 1.f, .22f, .47f, 5.f, 4.7f, .045f, .08f},
+                                               {1.38f, 1.24f, .25f, .2f, 2.f, 6.f, .054f, 0.f},
+                                               {2.01f, 1.66f, .63f, .54f, 2.f, 8.6f, .042f, 0.f}};
     GemmPlan best{3.4e38f, 0, 1, false};
-    const bool pipe = pipe_fits(a);
-    const float convert = q8 ? (float)a.n * a.k * 0.5e-6f + 4.f : 0.f;
+    const float convert = q8 ? (float)a.n * a.k * (.4e-6f + 3e-11f * a.k) + 4.f : 0.f;
     auto consider = [&](GemmPlan p, unsigned tm, bool dequant) {
         p.tm = tm;
         p.dequant = dequant;
         if (dequant) p.us += convert;
+        if (tm || p.split > 1) p.us *= 1.02f;
         if (p.us < best.us) best = p;
     };
-    if (pipe) consider(gemm_last_wave(g, (a.m + TM - 1) / TM * (a.n / TN), a.k / (2 * TK), 3.0f, 0.09f, 512), 0, q8);
-    if (q8 && h3_gemm_q8_fits(a)) {
-        const unsigned tiles = (a.m + TM - 1) / TM * ((a.n + TN - 1) / TN);
-        consider(gemm_last_wave(g, tiles, a.k / TK, 1.72f, 0.04f, 256, 1, 10.f), GEMM_Q8, false);
-    }
+    auto tiles = [&](unsigned rows) { return (a.m + rows - 1) / rows * ((a.n + TN - 1) / TN); };
+    const bool pipe = pipe_fits(a);
+    if (pipe) consider(gemm_last_wave(g, tiles(TM), a.k / (2 * TK), PIPE), 0, q8);
+    if (q8 && h3_gemm_q8_fits(a)) consider(gemm_last_wave(g, tiles(TM), a.k / TK, CODES), GEMM_Q8, false);
     if (h3_gemm_mid_fits(a, q8))
         for (unsigned i = 0; i < 3; i++) {
-            const unsigned tm = 64u << i, tiles = (a.m + tm - 1) / tm * ((a.n + TN - 1) / TN);
-            const float share = 0.09f * tm / 256;
-            if (q8) consider(gemm_last_wave(g, tiles, a.k / TK, Q8_STEP[i], share, 512 * 256 / tm), tm, false);
-            if (i < 2 || !pipe) consider(gemm_last_wave(g, tiles, a.k / TK, BF16_STEP[i], share, 512 * 256 / tm), tm, q8);
+            const unsigned tm = 64u << i;
+            const GemmRates &codes = a.group == a.k ? MID_COLUMN[i] : MID_GROUP[i];
+            if (q8) consider(gemm_last_wave(g, tiles(tm), a.k / TK, codes, tm / 256.f), tm, false);
+            if (i < 2 || !pipe) consider(gemm_last_wave(g, tiles(tm), a.k / TK, MID_BF16[i], tm / 256.f), tm, q8);
         }
     return best;
 }
