@@ -177,6 +177,7 @@ _SIGNATURES.update({
     "h3_gpu_profile_mark": (None, [_p, C.c_char_p]),
     "h3_device_query": (_i, [_p, C.c_char_p, _sz]),
     "h3_hip_kernel_timing": (_i, [_p, _i]),
+    "h3_hip_last_kernel": (C.c_char_p, [_p]),
     "h3_hip_kernel_timing_read": (_i, [_p, C.POINTER(C.c_double), C.POINTER(C.c_uint64)]),
     "h3_device_configure": (_i, [C.c_char_p, C.c_char_p, C.c_char_p, _sz]),
     "h3_device_memory_fits": (_i, [C.c_uint64]),

@@ -158,7 +158,14 @@ struct h3_gpu {
     h3_device_buffer gemm_partials; // FP32 partial sums of the tiles split over K
     h3_device_buffer mlp_workspace; // h3_gpu_mlp_bf16: activated rows (and the fused product)
     unsigned cus;                   // compute units of the device
+    // What the last projection or attention launched (h3_hip_last_kernel).
+    struct { const char *name; unsigned rows, shares; bool converted; } last;
+    char last_text[96];
 };
+
+inline void h3_note_kernel(h3_gpu *g, const char *name, unsigned rows = 0, unsigned shares = 1) {
+    g->last = {name, rows, shares, false};
+}
 
 // ---------------------------------------------------------------- helpers
 int h3_set_error(h3_gpu *g, const char *fmt, ...) __attribute__((format(printf, 2, 3)));

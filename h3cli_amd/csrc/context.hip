@@ -677,13 +677,16 @@ int h3_buffer_reserve(h3_gpu *g, h3_device_buffer *b, size_t bytes, const char *
     return 1;
 }
 
-bool h3_buffer_try(h3_gpu *g, h3_device_buffer *b, size_t bytes) {
-    if (b->bytes >= bytes) return true;
+bool h3_capturing(h3_gpu *g) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(g->compute, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return false;
-    }
+    if (hipStreamIsCapturing(g->compute, &capture) == hipSuccess) return capture != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
+bool h3_buffer_try(h3_gpu *g, h3_device_buffer *b, size_t bytes) {
+    if (h3_capturing(g)) return false;
+    if (b->bytes >= bytes) return true;
     if (b->ptr && hipStreamSynchronize(g->compute) != hipSuccess) return false;
     h3_buffer_free(b);
     if (hipMalloc(&b->ptr, bytes) != hipSuccess) {
@@ -722,6 +725,15 @@ static void kernel_events_clear(h3_gpu *g) {
     if (!g->kernel_events) return;
     for (auto &p : *g->kernel_events) { hipEventDestroy(p.first); hipEventDestroy(p.second); }
     g->kernel_events->clear();
+}
+
+extern "C" const char *h3_hip_last_kernel(h3_gpu *g) {
+    if (!g || !g->last.name) return "";
+    int n = snprintf(g->last_text, sizeof(g->last_text), "%s", g->last.name);
+    if (g->last.rows) n += snprintf(g->last_text + n, sizeof(g->last_text) - n, " rows=%u", g->last.rows);
+    if (g->last.shares > 1) n += snprintf(g->last_text + n, sizeof(g->last_text) - n, " shares=%u", g->last.shares);
+    if (g->last.converted) snprintf(g->last_text + n, sizeof(g->last_text) - n, " converted");
+    return g->last_text;
 }
 
 extern "C" int h3_hip_kernel_timing(h3_gpu *g, int enable) {

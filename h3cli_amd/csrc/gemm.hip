@@ -375,6 +375,7 @@ int launch_pipe(h3_gpu *g, GemmArgs a, unsigned split, bool timed) {
     const unsigned tiles = (a.m + TM - 1) / TM * (a.n / TN);
     a.tile = split_last_wave(g, tiles, split, a.k / (2 * TK), TM * TN);
     const unsigned rest = tiles - a.tile.full;
+    h3_note_kernel(g, "gemm_bf16_pipe", 0, a.tile.split);
     hipEvent_t timing = timed ? h3_kernel_timing_begin(g) : nullptr;
     if (!rest) {
         hipLaunchKernelGGL((gemm_bf16_pipe<EPI, false>), dim3(tiles), dim3(256), shared, g->compute, a);
@@ -520,6 +521,7 @@ __global__ __launch_bounds__(256) void gemm_small(GemmArgs a) {
 
 int launch_small(h3_gpu *g, const GemmArgs &a, bool q8) {
     const bool vec = a.k % 8 == 0 && (!q8 || a.group % 8 == 0);
+    h3_note_kernel(g, "gemm_small");
     const dim3 grid((a.m + 4 * SMALL_R - 1) / (4 * SMALL_R), (a.n + 63) / 64);
     if (q8 && vec) hipLaunchKernelGGL((gemm_small<true, true>), grid, dim3(256), 0, g->compute, a);
     else if (q8) hipLaunchKernelGGL((gemm_small<true, false>), grid, dim3(256), 0, g->compute, a);
@@ -540,7 +542,7 @@ int launch_small(h3_gpu *g, const GemmArgs &a, bool q8) {
 // group 64: mid 256 in 3 shares 260 (pipe in 3 281), per column: q8 in 3 shares 213 (mid 240);
 // 729 rows, 5120 -> 13824, group 64: pipe 122 (mid 151); 1800 rows, 14336 -> 5376, per column:
 // q8 292 (pipe 315); 64 rows, 5376 -> 28672, BF16: mid 64 in 2 shares 61 (pipe 114).
-GemmPlan choose(const h3_gpu *g, const GemmArgs &a, bool q8) {
+GemmPlan choose(const h3_gpu *g, const GemmArgs &a, bool q8, bool may_convert) {
     static constexpr GemmRates PIPE{2.89f, 1.96f, 1.72f, .65f, 6.4f, .6f, .044f, .41f};      // per 128 values of K
     static constexpr GemmRates CODES{1.73f, 1.22f, .93f, .57f, 8.5f, 1.3f, .03f, .95f};      // gemm_q8; per 64, as all below
     static constexpr GemmRates MID_BF16[3] = {{.61f, .5f, .58f, .74f, 4.1f, 1.4f, .085f, .39f},
@@ -563,14 +565,15 @@ GemmPlan choose(const h3_gpu *g, const GemmArgs &a, bool q8) {
     };
     auto tiles = [&](unsigned rows) { return (a.m + rows - 1) / rows * ((a.n + TN - 1) / TN); };
     const bool pipe = pipe_fits(a);
-    if (pipe) consider(gemm_last_wave(g, tiles(TM), a.k / (2 * TK), PIPE), 0, q8);
+    if (pipe && (!q8 || may_convert)) consider(gemm_last_wave(g, tiles(TM), a.k / (2 * TK), PIPE), 0, q8);
     if (q8 && h3_gemm_q8_fits(a)) consider(gemm_last_wave(g, tiles(TM), a.k / TK, CODES), GEMM_Q8, false);
     if (h3_gemm_mid_fits(a, q8))
         for (unsigned i = 0; i < 3; i++) {
             const unsigned tm = 64u << i;
             const GemmRates &codes = a.group == a.k ? MID_COLUMN[i] : MID_GROUP[i];
             if (q8) consider(gemm_last_wave(g, tiles(tm), a.k / TK, codes, tm / 256.f), tm, false);
-            if (i < 2 || !pipe) consider(gemm_last_wave(g, tiles(tm), a.k / TK, MID_BF16[i], tm / 256.f), tm, q8);
+            if ((i < 2 || !pipe) && (!q8 || may_convert))
+                consider(gemm_last_wave(g, tiles(tm), a.k / TK, MID_BF16[i], tm / 256.f), tm, q8);
         }
     return best;
 }
@@ -578,15 +581,10 @@ GemmPlan choose(const h3_gpu *g, const GemmArgs &a, bool q8) {
 // Runs a projection that pipe or mid takes. Both kernels of a converted projection are
 // inside one kernel-timing window.
 int run(h3_gpu *g, const GemmArgs &a, bool q8, int epi) {
-    GemmPlan p = choose(g, a, q8);
+    GemmPlan p = choose(g, a, q8, true);
     const size_t weights = (size_t)a.n * a.k;
-    if (p.dequant && !h3_buffer_try(g, &g->gemm_weights, weights * 2)) {
-        // No room for the converted weight: the same tiles on the codes.
-        if (!h3_gemm_mid_fits(a, true)) return h3_set_error(g, "GEMM weight buffer: out of device memory");
-        p.tm = 256;
-        p.split = 1;
-        p.dequant = false;
-    }
+    // No room for the converted weight: a kernel that reads the codes (gemm_mid takes all).
+    if (p.dequant && !h3_buffer_try(g, &g->gemm_weights, weights * 2)) p = choose(g, a, q8, false);
     if (p.tm == GEMM_Q8) return h3_gemm_q8(g, a, p.split);
     if (!p.dequant) return p.tm ? h3_gemm_mid(g, a, q8, p.tm, p.split) : launch_pipe_epi(g, a, epi, p.split, true);
     const size_t chunks = weights / 16;
@@ -598,6 +596,7 @@ int run(h3_gpu *g, const GemmArgs &a, bool q8, int epi) {
     const int ok = h3_launch_status(g, "W8A16 dequantization") &&
                    (p.tm ? h3_gemm_mid(g, b, false, p.tm, p.split, false) : launch_pipe_epi(g, b, epi, p.split, false));
     h3_kernel_timing_end(g, timing);
+    g->last.converted = true;
     return ok;
 }
 

@@ -269,6 +269,7 @@ int h3_gemm_fp8(h3_gpu *g, Fp8GemmArgs a) {
     const unsigned split = tiles < g->cus ? gemm_last_wave(g, tiles, a.k / TK, RATES, 1.f, 8).split : 1;
     a.tile = split_last_wave(g, tiles, split, a.k / TK, TM * TN);
     const unsigned rest = tiles - a.tile.full;
+    h3_note_kernel(g, "fp8_gemm_pipe", 0, a.tile.split);
     hipEvent_t timing = h3_kernel_timing_begin(g);
     if (!rest) {
         hipLaunchKernelGGL(fp8_gemm_pipe<false>, dim3(tiles), dim3(256), LDS, g->compute, a);

@@ -356,6 +356,7 @@ int launch(h3_gpu *g, GemmArgs a, unsigned split, bool timed) {
     const unsigned tiles = (a.m + TM - 1) / TM * ((a.n + TN - 1) / TN);
     a.tile = split_last_wave(g, tiles, split, a.k / TK, TM * TN);
     const unsigned rest = tiles - a.tile.full;
+    h3_note_kernel(g, "gemm_mid", TM, a.tile.split);
     hipEvent_t timing = timed ? h3_kernel_timing_begin(g) : nullptr;
     hipLaunchKernelGGL(kernel, dim3(a.tile.full + rest * a.tile.split), dim3(T), shared, g->compute, a);
     if (rest && h3_launch_status(g, "GEMM"))

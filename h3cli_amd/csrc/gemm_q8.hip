@@ -359,6 +359,7 @@ int h3_gemm_q8(h3_gpu *g, GemmArgs a, unsigned split) {
     const unsigned tiles = (a.m + TM - 1) / TM * ((a.n + TN - 1) / TN);
     a.tile = split_last_wave(g, tiles, split, a.k / TK, TM * TN);
     const unsigned rest = tiles - a.tile.full;
+    h3_note_kernel(g, "gemm_q8_pipe", 0, a.tile.split);
     hipEvent_t timing = h3_kernel_timing_begin(g);
     hipLaunchKernelGGL(gemm_q8_pipe, dim3(a.tile.full + rest * a.tile.split), dim3(256), LDS, g->compute, a);
     if (rest && h3_launch_status(g, "W8A16 GEMM"))

@@ -100,6 +100,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_skinny(GemmArgs a) {
 
 template <bool Q8, int NB, int WAVES>
 int launch(h3_gpu *g, const GemmArgs &a) {
+    h3_note_kernel(g, "gemm_skinny");
     hipLaunchKernelGGL((gemm_skinny<Q8, NB, WAVES>), dim3((a.n + 16 * NB - 1) / (16 * NB)), dim3(64 * WAVES), 0,
                        g->compute, a);
     return h3_launch_status(g, "skinny GEMM");

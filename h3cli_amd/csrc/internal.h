@@ -64,9 +64,12 @@ int h3_gemm_bf16_alpha(h3_gpu *g, uint16_t *y, const uint16_t *x, const uint16_t
                        uint32_t k, uint32_t n);
 
 int h3_buffer_reserve(h3_gpu *g, h3_device_buffer *b, size_t bytes, const char *what);
-// As h3_buffer_reserve for a workspace that the caller can do without: false,
-// with no error left behind, when memory is short or the compute stream is being
-// captured (nothing may be allocated then).
+// Whether the compute stream is being captured into a graph.
+bool h3_capturing(h3_gpu *g);
+// As h3_buffer_reserve for a workspace that the caller can do without: false, with no error
+// left behind, when memory is short, and always while the compute stream is being captured:
+// a graph keeps the address for its replays, while other calls use the buffer and, where they
+// grow it, free it.
 bool h3_buffer_try(h3_gpu *g, h3_device_buffer *b, size_t bytes);
 void h3_buffer_free(h3_device_buffer *b);
 

@@ -76,6 +76,8 @@ static h3_gpu_tensor workspace_tensor(h3_gpu *g, void *data, size_t elements) {
 extern "C" int h3_gpu_mlp_bf16(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tensor *in, const h3_gpu_tensor *w1,
                                const h3_gpu_tensor *w2, uint32_t rows, uint32_t width, uint32_t hidden, uint32_t output_dim) {
     if (!g) return 0;
+    // Its intermediates cannot be allocated for a graph, nor may a graph keep the workspace.
+    if (h3_capturing(g)) return h3_set_error(g, "MLP: the compute stream is being captured");
     const size_t n = (size_t)rows * hidden;
     const bool fused = n && w1 && w1->owner == g && !w1->quant_mode && h3_gemm_swiglu_fits(w1, rows, width, hidden);
     // Each part with the slack of h3_gpu_tensor_alloc behind it.

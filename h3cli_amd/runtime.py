@@ -116,6 +116,10 @@ class Gpu:
         if t in self.tensors:
             self.tensors.remove(t)
 
+    def last_kernel(self):
+        """The kernel that the last projection or attention launched (h3_hip_last_kernel)."""
+        return self.lib.h3_hip_last_kernel(self.handle).decode()
+
     # -- timing
     def timing_event(self):
         e = self.lib.h3_hip_timing_event_new(self.handle)

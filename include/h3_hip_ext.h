@@ -199,6 +199,11 @@ int h3_hip_event_elapsed_ms(h3_gpu *gpu, h3_gpu_event *start, h3_gpu_event *end,
  * the number of timed launches, and clears them. Enabling or disabling also clears. */
 int h3_hip_kernel_timing(h3_gpu *gpu, int enable);
 int h3_hip_kernel_timing_read(h3_gpu *gpu, double *ms_total, uint64_t *launches);
+/* The kernel that the last projection or attention of this context launched, for tests that
+ * are about one: its name, then where they apply " rows=<row tile>", " shares=<K shares of a
+ * split tile>", " converted" (an int8 weight written as BF16 first). "" before the first.
+ * Valid until the next call. */
+const char *h3_hip_last_kernel(h3_gpu *gpu);
 
 #ifdef __cplusplus
 }
