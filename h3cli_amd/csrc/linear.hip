@@ -3,6 +3,7 @@
 #include "common.h"
 #include "internal.h"
 #include "gemm.h"
+#include <algorithm>
 #include <cerrno>
 #include <cmath>
 #include <fcntl.h>
@@ -58,8 +59,8 @@ extern "C" int h3_gpu_grouped_qkv_linear_rope_bf16(h3_gpu *g, h3_gpu_tensor *q, 
 
 // The MLP's intermediates stay in a grow-only workspace of the context: allocating
 // and freeing them in each call waits for the GPU (8193 rows, 5376 -> 14336 -> 5376,
-// alone: 20.0 ms a call, of which 3.4 ms computing). Larger ones than this are
-// allocated per call, so the context keeps no more.
+// alone: 20.0 ms a call, of which 3.4 ms computing). The context keeps no more than this;
+// calls with more rows than it holds run in parts of the rows.
 constexpr size_t MLP_WORKSPACE = (size_t)1 << 30;
 
 // A BF16 tensor over workspace memory, for the operators of one call.
@@ -70,6 +71,18 @@ static h3_gpu_tensor workspace_tensor(h3_gpu *g, void *data, size_t elements) {
     return t;
 }
 
+// Workspace of `rows` rows: the activated rows and, where SwiGLU is not fc1's epilogue, the
+// 2 * hidden wide product, each with the slack of h3_gpu_tensor_alloc behind it.
+struct MlpPart {
+    bool fused;
+    size_t act, both;
+};
+static MlpPart mlp_part(const h3_gpu_tensor *w1, size_t rows, uint32_t width, uint32_t hidden) {
+    const bool fused = w1 && !w1->quant_mode && h3_gemm_swiglu_fits(w1, (uint32_t)rows, width, hidden);
+    const auto slack = [](size_t bytes) { return (bytes + 511) & ~(size_t)255; };
+    return {fused, slack(rows * hidden * 2), fused ? 0 : slack(rows * hidden * 4)};
+}
+
 // fc1 (2*hidden, gate rows then up rows) -> SwiGLU -> fc2, as src/cuda/gpu_cuda.cu:1108-1112.
 // Where the projection kernel takes it, SwiGLU is fc1's epilogue and the 2 * hidden
 // wide product is never written.
@@ -78,25 +91,43 @@ extern "C" int h3_gpu_mlp_bf16(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tenso
     if (!g) return 0;
     // Its intermediates cannot be allocated for a graph, nor may a graph keep the workspace.
     if (h3_capturing(g)) return h3_set_error(g, "MLP: the compute stream is being captured");
-    const size_t n = (size_t)rows * hidden;
-    const bool fused = n && w1 && w1->owner == g && !w1->quant_mode && h3_gemm_swiglu_fits(w1, rows, width, hidden);
-    // Each part with the slack of h3_gpu_tensor_alloc behind it.
-    const size_t part = (n * 2 + 511) & ~(size_t)255, product = fused ? 0 : (n * 4 + 511) & ~(size_t)255;
-    if (n && n <= MLP_WORKSPACE && part + product <= MLP_WORKSPACE && h3_buffer_try(g, &g->mlp_workspace, part + product)) {
-        h3_gpu_tensor act = workspace_tensor(g, g->mlp_workspace.ptr, n);
-        h3_gpu_tensor both = workspace_tensor(g, (char *)g->mlp_workspace.ptr + part, fused ? 0 : n * 2);
-        const int ok = fused ? linear(g, &act, in, w1, nullptr, rows, width, hidden * 2, H3_GEMM_SWIGLU)
-                             : h3_gpu_linear_bf16(g, &both, in, w1, nullptr, rows, width, hidden * 2) &&
-                                   h3_gpu_swiglu_bf16(g, &act, &both, rows, hidden);
-        return ok && h3_gpu_linear_bf16(g, out, &act, w2, nullptr, rows, hidden, output_dim);
+    if (!rows || !hidden || hidden > UINT32_MAX / 2 ||
+        !h3_require(g, in, H3_GPU_BF16, (size_t)rows * width, "MLP input") ||
+        !h3_require(g, out, H3_GPU_BF16, (size_t)rows * output_dim, "MLP output"))
+        return rows && hidden && hidden <= UINT32_MAX / 2 ? 0 : h3_set_error(g, "MLP: invalid shape %ux%u", rows, hidden);
+    // Parts of whole 256-row tiles, even ones. A packed weight sees all rows at once: the
+    // scale of its quantized activations is the tensor's.
+    size_t most = rows;
+    if (!(w1 && w1->quant_mode) && !(w2 && w2->quant_mode)) {
+        const size_t row_bytes = (size_t)hidden * (mlp_part(w1, rows, width, hidden).fused ? 2 : 6);
+        most = std::max(MLP_WORKSPACE / row_bytes / 256, (size_t)1) * 256;
     }
-    h3_gpu_tensor *both = h3_gpu_tensor_new_bf16(g, n * 2);
-    h3_gpu_tensor *act = h3_gpu_tensor_new_bf16(g, n);
-    int ok = both && act && h3_gpu_linear_bf16(g, both, in, w1, nullptr, rows, width, hidden * 2) &&
-             h3_gpu_swiglu_bf16(g, act, both, rows, hidden) &&
-             h3_gpu_linear_bf16(g, out, act, w2, nullptr, rows, hidden, output_dim);
-    h3_gpu_tensor_free(both);
-    h3_gpu_tensor_free(act);
+    const size_t parts = (rows + most - 1) / most;
+    const size_t step = parts == 1 ? rows : ((rows + parts - 1) / parts + 255) / 256 * 256;
+    const size_t last = rows - (rows - 1) / step * step;
+    const MlpPart a = mlp_part(w1, step, width, hidden), b = mlp_part(w1, last, width, hidden);
+    const size_t bytes = std::max(a.act + a.both, b.act + b.both);
+    h3_gpu_tensor *own = nullptr;
+    char *workspace = nullptr;
+    if (bytes <= MLP_WORKSPACE + 1024 && h3_buffer_try(g, &g->mlp_workspace, bytes)) workspace = (char *)g->mlp_workspace.ptr;
+    else if ((own = h3_gpu_tensor_new_bf16(g, bytes / 2))) workspace = (char *)own->data;
+    int ok = workspace != nullptr;
+    // Last part first where the output of a part could reach the input of a later one.
+    const bool backward = out->data == in->data && output_dim > width;
+    const size_t count = (rows + step - 1) / step;
+    for (size_t i = 0; ok && i < count; i++) {
+        const size_t first = (backward ? count - 1 - i : i) * step, m = std::min(step, rows - first);
+        const MlpPart p = m == step ? a : b;
+        h3_gpu_tensor act = workspace_tensor(g, workspace, m * hidden);
+        h3_gpu_tensor both = workspace_tensor(g, workspace + p.act, p.fused ? 0 : m * hidden * 2);
+        h3_gpu_tensor x = workspace_tensor(g, (uint16_t *)in->data + first * width, m * width);
+        h3_gpu_tensor y = workspace_tensor(g, (uint16_t *)out->data + first * output_dim, m * output_dim);
+        ok = p.fused ? linear(g, &act, &x, w1, nullptr, (uint32_t)m, width, hidden * 2, H3_GEMM_SWIGLU)
+                     : linear(g, &both, &x, w1, nullptr, (uint32_t)m, width, hidden * 2, H3_GEMM_PLAIN) &&
+                           h3_gpu_swiglu_bf16(g, &act, &both, (uint32_t)m, hidden);
+        ok = ok && linear(g, &y, &act, w2, nullptr, (uint32_t)m, hidden, output_dim, H3_GEMM_PLAIN);
+    }
+    h3_gpu_tensor_free(own);
     return ok;
 }
 

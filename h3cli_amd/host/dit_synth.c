@@ -350,11 +350,16 @@ h3_hip_dit_synth *h3_hip_dit_synth_create(h3_gpu *g, const h3_hip_dit_synth_conf
         m->qkv = bf16_buffer(g, R * I * 3);
         m->q = bf16_buffer(g, R * I); m->k = bf16_buffer(g, R * I); m->v = bf16_buffer(g, R * I);
         m->attn = bf16_buffer(g, R * I); m->o = bf16_buffer(g, R * H);
-        m->h = bf16_buffer(g, R * c->mlp * (c->swiglu ? 2 : 1)); m->f = bf16_buffer(g, R * H);
-        m->act = c->swiglu || c->projection_quant ? bf16_buffer(g, R * c->mlp) : NULL;
+        /* The SwiGLU MLP is one call with a workspace of its own; its stages are
+         * separate only for packed weights and, beside it, for the trace. */
+        const int stages = c->projection_quant || !c->swiglu || c->trace_block;
+        const int act = c->projection_quant || (c->swiglu && c->trace_block);
+        m->h = stages ? bf16_buffer(g, R * c->mlp * (c->swiglu ? 2 : 1)) : NULL;
+        m->f = bf16_buffer(g, R * H);
+        m->act = act ? bf16_buffer(g, R * c->mlp) : NULL;
         m->vel = bf16_buffer(g, R * c->latent);
         if (!m->row_map || !m->latent || !m->latent_bf16 || !m->x || !m->xn || !m->qkv || !m->q || !m->k || !m->v ||
-            !m->attn || !m->o || !m->h || !m->f || !m->vel || ((c->swiglu || c->projection_quant) && !m->act)) {
+            !m->attn || !m->o || (stages && !m->h) || !m->f || !m->vel || (act && !m->act)) {
             fail(error, size, "activations: %s", h3_gpu_error(g));
             h3_gpu_cancel(g);
             goto bad;

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from h3cli_amd import synth
+from h3cli_amd._lib import GpuStats
 from h3cli_amd.runtime import Gpu
 from oracle import oracle
 from tests.helpers import GEMM_REL_L2, bf16, metrics
@@ -225,6 +226,47 @@ def test_mlp(gpu, m, k, hidden, n, group):
     assert met["rel_l2"] <= 4 * 2.0 ** -9, met
     for t in (tx, out, *ws):
         gpu.free(t)
+
+
+def test_mlp_in_parts():
+    """More rows than the kept workspace holds (1 GiB of activated rows): parts of the
+    rows, bit for bit what a call on a part's rows gives, with no tensor allocated in any
+    call, and in place in both directions."""
+    m, k, hidden, n, part = 16640, 64, 32768, 128, 8448
+    print(f"[mlp parts] m={m} k={k} hidden={hidden} n={n}", flush=True)
+    x = synth.normal_bf16(1, m * k)
+    bits = [synth.normal_bf16(2, 2 * hidden * k, scale=1 / math.sqrt(k)),
+            synth.normal_bf16(3, n * hidden, scale=1 / math.sqrt(hidden)),
+            synth.normal_bf16(4, k // 2 * hidden, scale=1 / math.sqrt(hidden))]
+    with Gpu() as gpu:
+        tx, out, few = gpu.from_bf16(x), gpu.empty(m * n), gpu.empty(part * n)
+        w1, w2, narrow = (gpu.from_bf16(b) for b in bits)
+        place = gpu.empty(m * n)
+        before, after = GpuStats(), GpuStats()
+        gpu.lib.h3_gpu_get_stats(gpu.handle, C.byref(before))
+        run(gpu, gpu.lib.h3_gpu_mlp_bf16, out.handle, tx.handle, w1.handle, w2.handle, m, k, hidden, n)
+        got = out.read().reshape(m, n)
+        for first in (0, part):
+            rows = min(part, m - first)
+            tp = gpu.from_bf16(x.reshape(m, k)[first:first + rows])
+            run(gpu, gpu.lib.h3_gpu_mlp_bf16, few.handle, tp.handle, w1.handle, w2.handle, rows, k, hidden, n)
+            assert np.array_equal(few.read(rows * n).reshape(rows, n), got[first:first + rows])
+        rows = np.r_[0:m:997, part - 1, part, m - 1]
+        xv, wv = bf16(x).reshape(m, k)[rows].astype(np.float64), [bf16(b).astype(np.float64) for b in bits]
+        both = xv @ wv[0].reshape(-1, k).T
+        want = (both[:, :hidden] / (1 + np.exp(-both[:, :hidden])) * both[:, hidden:]) @ wv[1].reshape(n, hidden).T
+        met = metrics(bf16(got[rows]), want)
+        assert met["rel_l2"] <= 4 * 2.0 ** -9, met
+        # In place: wider output (last part first) and narrower output.
+        for w, width in ((w2, n), (narrow, k // 2)):
+            run(gpu, gpu.lib.h3_gpu_mlp_bf16, out.handle, tx.handle, w1.handle, w.handle, m, k, hidden, width)
+            place_rows = np.zeros(m * n, np.uint16)
+            place_rows[:m * k] = x
+            gpu.check(gpu.lib.h3_gpu_tensor_write_bf16(place.handle, place_rows.ctypes.data, m * n), "write")
+            run(gpu, gpu.lib.h3_gpu_mlp_bf16, place.handle, place.handle, w1.handle, w.handle, m, k, hidden, width)
+            assert np.array_equal(place.read(m * width), out.read(m * width))
+        gpu.lib.h3_gpu_get_stats(gpu.handle, C.byref(after))
+        assert after.tensor_allocations - before.tensor_allocations == 2    # tp, twice
 
 
 @pytest.mark.parametrize("m,k,n,hidden,bias,gelu", [
