@@ -490,8 +490,12 @@ int h3_hip_dit_synth_step(h3_hip_dit_synth *m, int step, float dt) {
              h3_gpu_gate_adaln_bf16(g, m->x, m->xn, m->x, m->o, m->norm2[b], m->mod[b], m->mod[b], m->row_map, R, H,
                                     SLOTS, 2, 3, 4, c->eps) &&
              (!tr || (keep(m, T_X1, m->x) && keep(m, T_XN2, m->xn)));
-        if (c->swiglu && !c->projection_quant && !tr) {
-            ok = ok && h3_gpu_mlp_bf16(g, m->f, m->xn, w[2], w[3], R, H, c->mlp, H);
+        if (c->swiglu && !c->projection_quant) {
+            /* The traced block runs the same MLP; its product and activation, which that
+             * call does not write, are computed beside it. */
+            ok = ok && (!tr || (h3_gpu_linear_bf16(g, m->h, m->xn, w[2], NULL, R, H, 2 * c->mlp) &&
+                                h3_gpu_swiglu_bf16(g, m->act, m->h, R, c->mlp))) &&
+                 h3_gpu_mlp_bf16(g, m->f, m->xn, w[2], w[3], R, H, c->mlp, H);
         } else if (c->swiglu) {
             ok = ok && h3_gpu_linear_bf16(g, m->h, m->xn, w[2], NULL, R, H, 2 * c->mlp) &&
                  h3_gpu_swiglu_bf16(g, m->act, m->h, R, c->mlp) &&

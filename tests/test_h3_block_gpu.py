@@ -127,3 +127,33 @@ def test_h3_geometry_step_small():
     assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
     assert np.array_equal(outs[0][0], outs[2][0])
     assert not np.array_equal(outs[0][1], outs[3][1])     # Sage differs from BF16
+
+
+def test_h3_geometry_traced_step_is_the_step():
+    """Tracing a block changes no bit of the step, and the traced MLP output is that of
+    the MLP which the step runs, held to the traced stages before it: gate, up, the
+    activation and the result are rounded to BF16 once each."""
+    from h3cli_amd.runtime import DitSynth
+    small = dict(blocks=2, hidden=512, heads=3, mlp=768, frames=3, height=8, width=200, latent=256, seed=4,
+                 streamed_first=2)
+    print(f"[h3 traced step] {small}", flush=True)
+    outs = []
+    for block in (0, 1, 2):
+        with DitSynth(geometry="h3", trace_block=block, **small) as m:
+            rows = m.rows
+            if block:
+                fc1, fc2 = (m.read_q8(f"blocks.{block - 1}.mlp.{n}.weight", *s)
+                            for n, s in (("fc1", (2 * 768, 512)), ("fc2", (512, 768))))
+            m.step(step=12, dt=-0.1)
+            outs.append((m.read("latent"), m.read("hidden")))
+            if block:
+                h, act, f, xn2 = (m.read(f"trace.{s}") for s in ("h", "act", "f", "xn2"))
+                w = [bf16(synth.f32_to_bf16(c.reshape(-1, k).astype(np.float32) * s[:, None])).astype(np.float64)
+                     for (c, s), k in ((fc1, 512), (fc2, 768))]
+                both = bf16(xn2).reshape(rows, 512).astype(np.float64) @ w[0].T
+                assert metrics(bf16(h).reshape(rows, -1), both)["rel_l2"] < 0.006
+                want = both[:, :768] / (1 + np.exp(-both[:, :768])) * both[:, 768:]
+                assert metrics(bf16(act).reshape(rows, -1), want)["rel_l2"] <= 3 * 2.0 ** -9
+                assert metrics(bf16(f).reshape(rows, -1), want @ w[1].T)["rel_l2"] <= 4 * 2.0 ** -9
+    for lat, hid in outs[1:]:
+        assert np.array_equal(lat, outs[0][0]) and np.array_equal(hid, outs[0][1])
