@@ -445,7 +445,8 @@ __global__ __launch_bounds__(256) void gemm_small(GemmArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t ws[64 * SMALL_ROW];
     __shared__ __attribute__((aligned(16))) float xs[4 * SMALL_R][SMALL_K];
     const unsigned tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-    const unsigned n0 = blockIdx.y * 64, m0 = blockIdx.x * 4 * SMALL_R, col = n0 + lane;
+    const unsigned row_blocks = (a.m + 4 * SMALL_R - 1) / (4 * SMALL_R);
+    const unsigned n0 = blockIdx.x / row_blocks * 64, m0 = blockIdx.x % row_blocks * 4 * SMALL_R, col = n0 + lane;
     float acc[SMALL_R] = {};
     for (unsigned k0 = 0; k0 < a.k; k0 += SMALL_K) {
         const unsigned kn = min(SMALL_K, a.k - k0);
@@ -522,7 +523,8 @@ __global__ __launch_bounds__(256) void gemm_small(GemmArgs a) {
 int launch_small(h3_gpu *g, const GemmArgs &a, bool q8) {
     const bool vec = a.k % 8 == 0 && (!q8 || a.group % 8 == 0);
     h3_note_kernel(g, "gemm_small");
-    const dim3 grid((a.m + 4 * SMALL_R - 1) / (4 * SMALL_R), (a.n + 63) / 64);
+    // One grid dimension, rows first: the others end at 65535 blocks (4.19 million columns).
+    const dim3 grid((a.m + 4 * SMALL_R - 1) / (4 * SMALL_R) * ((a.n + 63) / 64));
     if (q8 && vec) hipLaunchKernelGGL((gemm_small<true, true>), grid, dim3(256), 0, g->compute, a);
     else if (q8) hipLaunchKernelGGL((gemm_small<true, false>), grid, dim3(256), 0, g->compute, a);
     else if (vec) hipLaunchKernelGGL((gemm_small<false, true>), grid, dim3(256), 0, g->compute, a);

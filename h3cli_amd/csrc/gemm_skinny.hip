@@ -120,7 +120,8 @@ int choose(h3_gpu *g, const GemmArgs &a) {
 }  // namespace
 
 bool h3_gemm_skinny_fits(const GemmArgs &a, bool q8) {
-    return a.m <= 16 && a.k > H3_GEMM_SHORT_K && a.k % STEP == 0 && (!q8 || a.group % 16 == 0);
+    // Up to 32 threads a column, less than 2^32 in all.
+    return a.m <= 16 && a.k > H3_GEMM_SHORT_K && a.k % STEP == 0 && (!q8 || a.group % 16 == 0) && a.n < (1u << 27);
 }
 
 int h3_gemm_skinny(h3_gpu *g, const GemmArgs &a, bool q8) { return q8 ? choose<true>(g, a) : choose<false>(g, a); }

@@ -171,6 +171,24 @@ def test_linear_split_over_k(gpu, m, k, n, q8, bias, gelu):
         gpu.free(t)
 
 
+@pytest.mark.parametrize("m,k", [(2, 8), (20, 4)])
+def test_any_shape_linear_of_many_columns(gpu, m, k):
+    """More blocks of columns than the second and third grid dimensions hold (65535)."""
+    n = 64 * 65536 + 33
+    print(f"[many columns] m={m} k={k} n={n}", flush=True)
+    x, w = synth.normal_bf16(m, m * k), synth.normal_bf16(m + 1, n * k)
+    tx, tw, out = gpu.from_bf16(x), gpu.from_bf16(w), gpu.empty(m * n)
+    run(gpu, gpu.lib.h3_gpu_linear_bf16, out.handle, tx.handle, tw.handle, None, m, k, n)
+    assert gpu.last_kernel() == "gemm_small"
+    cols = np.r_[0:n:9973, n - 70:n]
+    xv, wv = bf16(x).reshape(m, k).astype(np.float64), bf16(w).reshape(n, k)[cols].astype(np.float64)
+    want = xv @ wv.T
+    bound = 2.0 ** -8 * np.abs(want) + k * 2.0 ** -24 * (np.abs(xv) @ np.abs(wv).T)
+    assert np.all(np.abs(bf16(out.read()).reshape(m, n)[:, cols] - want) <= bound)
+    for t in (tx, tw, out):
+        gpu.free(t)
+
+
 @pytest.mark.parametrize("m,k,n,group,bias,gelu", [
     (17, 64, 30, 0, False, False),        # one K step, a ragged column tile of odd width
     (64, 1088, 256, 0, True, False),      # 17 steps, split
