@@ -583,8 +583,10 @@ GemmPlan choose(const h3_gpu *g, const GemmArgs &a, bool q8, bool may_convert) {
 // Runs a projection that pipe or mid takes. Both kernels of a converted projection are
 // inside one kernel-timing window.
 int run(h3_gpu *g, const GemmArgs &a, bool q8, int epi) {
-    GemmPlan p = choose(g, a, q8, true);
+    // The context keeps the converted weight: none of 2 GiB or more, which the pipe kernel's
+    // 32-bit offsets do not take either.
     const size_t weights = (size_t)a.n * a.k;
+    GemmPlan p = choose(g, a, q8, weights * 2 < (1ull << 31));
     // No room for the converted weight: a kernel that reads the codes (gemm_mid takes all).
     if (p.dequant && !h3_buffer_try(g, &g->gemm_weights, weights * 2)) p = choose(g, a, q8, false);
     if (p.tm == GEMM_Q8) return h3_gemm_q8(g, a, p.split);

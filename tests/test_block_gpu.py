@@ -189,6 +189,34 @@ def test_any_shape_linear_of_many_columns(gpu, m, k):
         gpu.free(t)
 
 
+def test_large_q8_weight_is_not_converted(gpu):
+    """A weight of 2 GiB or more in BF16 is multiplied from its codes, however many rows
+    would pay for the conversion: the context keeps no buffer of that size."""
+    m, k, n, group = 12288, 8256, 131072, 64
+    print(f"[large q8] m={m} k={k} n={n}", flush=True)
+    tx, out = gpu.empty(m * k), gpu.empty(m * n)
+    w = gpu.lib.h3_hip_q8_new(gpu.handle, n, k, group)
+    run(gpu, gpu.lib.h3_hip_fill_normal_bf16, tx.handle, 3, C.c_float(1.0), m * k)
+    run(gpu, gpu.lib.h3_hip_fill_q8_random, w, 5, C.c_float(1e-4), C.c_float(3e-4))
+    run(gpu, gpu.lib.h3_gpu_linear_bf16, out.handle, tx.handle, w, None, m, k, n)
+    assert gpu.last_kernel().startswith("gemm_mid rows=256") and "converted" not in gpu.last_kernel()
+    cols = np.r_[0:n:16381, n - 2:n].astype(np.uint64)
+    base, kk = np.uint64(5 << 40), np.arange(k, dtype=np.uint64)
+    codes = (synth.splitmix64(base + cols[:, None] * np.uint64(k) + kk) % np.uint64(255)).astype(np.float32) - 127
+    at = cols[:, None] * np.uint64(k // group) + np.arange(k // group, dtype=np.uint64)
+    unit = (synth.splitmix64(base + np.uint64(1 << 39) + at) >> np.uint64(11)).astype(np.float64) * 2.0 ** -53
+    scales = (1e-4 + 2e-4 * unit).astype(np.float32)
+    wv = bf16(synth.f32_to_bf16((codes * np.repeat(scales, group, axis=1)).reshape(-1))).reshape(len(cols), k)
+    xv = bf16(tx.read(k)).astype(np.float64)
+    want = wv.astype(np.float64) @ xv
+    # One BF16 rounding, the FP32 sum, and weights whose scale differs in the last place.
+    bound = 2.0 ** -8 * np.abs(want) + k * 2.0 ** -24 * (np.abs(wv) @ np.abs(xv)) + 2.0 ** -8 * np.sqrt((wv ** 2) @ (xv ** 2))
+    assert np.all(np.abs(bf16(out.read(n))[cols.astype(np.int64)] - want) <= bound)
+    gpu.lib.h3_gpu_tensor_free(w)
+    for t in (tx, out):
+        gpu.free(t)
+
+
 @pytest.mark.parametrize("m,k,n,group,bias,gelu", [
     (17, 64, 30, 0, False, False),        # one K step, a ragged column tile of odd width
     (64, 1088, 256, 0, True, False),      # 17 steps, split
