@@ -17,7 +17,8 @@
 #include "../../include/h3_policy.h"
 #include <algorithm>
 #include <cmath>
-#include <vector>
+#include <memory>
+#include <new>
 
 namespace {
 
@@ -456,8 +457,10 @@ extern "C" int h3_hip_subblock_routes(h3_gpu *g, uint8_t *routes, float *scores,
         uint16_t *dst = which ? k_pool : q_pool;
         if (!dst) continue;
         const auto *src = (const uint16_t *)(base + (which ? r->off_kpool : r->off_qpool));
-        std::vector<uint16_t> pool((size_t)r->heads * r->cells * D);
-        if (!h3_hip_check(g, hipMemcpy(pool.data(), src, pool.size() * 2, hipMemcpyDeviceToHost), "pooled cells")) return 0;
+        const size_t count = (size_t)r->heads * r->cells * D;
+        const std::unique_ptr<uint16_t[]> pool(new (std::nothrow) uint16_t[count]);
+        if (!pool) return h3_set_error(g, "SubBlock capture: out of host memory");
+        if (!h3_hip_check(g, hipMemcpy(pool.get(), src, count * 2, hipMemcpyDeviceToHost), "pooled cells")) return 0;
         for (size_t head = 0; head < r->heads; head++)
             for (unsigned cell = 0; cell < cells; cell++)
                 for (unsigned part = 0; part < D / 8; part++)
