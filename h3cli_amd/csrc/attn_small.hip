@@ -15,7 +15,8 @@
 //    row-major V tile by transposing LDS reads (ds_read_b64_tr_b16), in the key order
 //    that P has;
 //  * a running max per tile, raised when a tile's max passes it by more than 8 (log2
-//    units; P stays below 256).
+//    units). P is taken 8 below it, so that P <= 1 in every wave, whichever key it has seen
+//    first, and a partial O is at most the keys' sum of |V|.
 #include "common.h"
 #include "internal.h"
 #include "attn_common.h"
@@ -186,7 +187,7 @@ void attn_small(SmallArgs a) {
 #pragma unroll
                 for (int md = 0; md < 4; md++) o[b][md] *= alpha;
             }
-            const float neg = -m[b];
+            const float neg = -m[b] - RESCALE_SLACK;
             float sum = 0.f;
 #pragma unroll
             for (int mb = 0; mb < 2; mb++)

@@ -212,6 +212,20 @@ def test_few_rows_nonfinite(gpu, which, value, row):
         sdpa(g, *bits, seq, heads)
 
 
+@pytest.mark.parametrize("seq,heads", [(700, 3), (2048, 8)])
+def test_few_rows_large_values(gpu, seq, heads):
+    """|V| = 1e35 and, in a tile whose wave has not seen the row's largest score, 64 keys
+    that its own running max lags by 7.5 log2 units: P near 2^7.5 would carry the wave's
+    partial O past FP32. With constant V the output is V, as from the tile kernels."""
+    k = np.zeros((seq, heads, 128), np.float32)
+    k[0] = 1.2266           # 20 log2 units: the first wave's first tile
+    k[320:384] = 0.459      # 7.5: the second wave's second tile, after one of zeros
+    big = float(synth.bf16_to_f32(synth.f32_to_bf16(np.float32(1e35))))
+    q, k, v = (synth.f32_to_bf16(x.reshape(-1)) for x in (np.ones_like(k), k, np.full_like(k, big)))
+    out = bf16(sdpa(gpu, q, k, v, seq, heads))
+    assert np.max(np.abs(out / big - 1)) < 2e-2
+
+
 def test_large_values_after_score_jump(gpu):
     """A 41-log2-unit score jump with |V| near 1e26: P that large must not
     reach O unscaled (it would overflow FP32). The rows go to the
