@@ -379,6 +379,7 @@ int launch(h3_gpu *g, const Args &a, unsigned groups) {
             return 0;
         configured = true;
     }
+    h3_note_kernel(g, SPARSE ? "attn_bf16_kernel (lists)" : "attn_bf16_kernel");
     hipEvent_t timing = h3_kernel_timing_begin(g);
     hipLaunchKernelGGL(kernel, dim3(groups), dim3(64 * WAVES), shared, g->compute, a);
     h3_kernel_timing_end(g, timing);
@@ -748,6 +749,7 @@ int launch_wide(h3_gpu *g, const Args &a, unsigned groups) {
     constexpr size_t shared = 2 * KT * STAGE_BYTES;
     if (!configure_wide<KT, SPARSE, MSUM, false, WAVES>(g)) return 0;
     if (NOMAX && !configure_wide<KT, SPARSE, MSUM, true, WAVES>(g)) return 0;
+    h3_note_kernel(g, a.buffered ? "attn_bf16_wide" : "attn_bf16_wide (global loads)");
     hipEvent_t timing = h3_kernel_timing_begin(g);
     hipLaunchKernelGGL((attn_bf16_wide<KT, SPARSE, MSUM, NOMAX, WAVES>), dim3(groups), dim3(64 * WAVES), shared,
                        g->compute, a);
@@ -1249,6 +1251,7 @@ int launch_pipe_attention(h3_gpu *g, const Args &a) {
     }
     if (!configure_wide<2, false, false, false, 8>(g)) return 0;
     const unsigned groups = (a.seq + 255) / 256 * a.heads;
+    h3_note_kernel(g, "attn_bf16_pipe");
     hipEvent_t timing = h3_kernel_timing_begin(g);
     hipLaunchKernelGGL(attn_bf16_pipe, dim3(groups), dim3(256), shared, g->compute, a);
     if (!h3_launch_status(g, "BF16 attention")) {
@@ -1526,6 +1529,7 @@ int launch_pingpong(h3_gpu *g, const Args &a, unsigned groups) {
         configured = true;
     }
     if (!configure_wide<2, false, false, false>(g)) return 0;
+    h3_note_kernel(g, "attn_bf16_pingpong");
     hipEvent_t timing = h3_kernel_timing_begin(g);
     hipLaunchKernelGGL(attn_bf16_pingpong<KT>, dim3(groups), dim3(512), shared, g->compute, a);
     if (!h3_launch_status(g, "BF16 attention")) return 0;
@@ -1910,6 +1914,7 @@ int launch_listed(h3_gpu *g, const Args &a, unsigned groups) {
             return 0;
         configured = true;
     }
+    h3_note_kernel(g, "attn_bf16_listed");
     hipEvent_t timing = h3_kernel_timing_begin(g);
     hipLaunchKernelGGL(kernel, dim3(groups), dim3(64 * QW), shared, g->compute, a);
     h3_kernel_timing_end(g, timing);
@@ -1939,9 +1944,8 @@ int h3_launch_attention_bf16(h3_gpu *g, void *workspace, uint16_t *out, const ui
     a.fault = g->fault;
     // Variant 13: the global-load path that tensors of 4 GiB and more take.
     a.buffered = fits_buffer(a) && g->attention_variant != 13;
-    // Few query rows. Variants 3, 13 and 14 choose among the tile kernels only.
-    const int variant = g->attention_variant;
-    if (!kv_list && (variant == 0 || variant == 3 || variant == 13 || variant == 14)) {
+    // Few query rows. Every other variant is one of the tile kernels (15: the default one).
+    if (!kv_list && g->attention_variant == 0) {
         const int blocks = h3_attention_small_blocks(g, seq, heads);
         if (blocks) return h3_launch_attention_small(g, blocks, out, q, k, v, seq, heads, scale, head_major);
     }

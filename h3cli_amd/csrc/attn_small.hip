@@ -292,6 +292,7 @@ int launch(h3_gpu *g, const SmallArgs &a) {
             return 0;
         configured = true;
     }
+    h3_note_kernel(g, "attn_small", 32 * NQ);
     hipEvent_t timing = h3_kernel_timing_begin(g);
     hipLaunchKernelGGL(attn_small<NQ>, dim3((a.seq + 32 * NQ - 1) / (32 * NQ) * a.heads), dim3(64 * WAVES), shared,
                        g->compute, a);

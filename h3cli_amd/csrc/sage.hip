@@ -1004,6 +1004,7 @@ int launch_sage_pipe(h3_gpu *g, const SArgs &a) {
             return 0;
         configured = true;
     }
+    h3_note_kernel(g, "sage_pipe");
     hipEvent_t timing = h3_kernel_timing_begin(g);
     hipLaunchKernelGGL(sage_pipe, dim3((a.seq + 255) / 256 * a.heads), dim3(256), SP_LDS, g->compute, a);
     if (!h3_launch_status(g, "Sage attention")) {
@@ -1021,6 +1022,7 @@ int launch_sage_pipe(h3_gpu *g, const SArgs &a) {
 template <int WAVES, int OCC, bool SPARSE>
 int launch_sage(h3_gpu *g, const SArgs &a, unsigned groups) {
     constexpr size_t shared = 2 * SAGE_TILE;
+    h3_note_kernel(g, SPARSE ? "sage_attn_kernel (lists)" : "sage_attn_kernel");
     hipEvent_t timing = h3_kernel_timing_begin(g);
     hipLaunchKernelGGL((sage_attn_kernel<WAVES, OCC, SPARSE>), dim3(groups), dim3(64 * WAVES), shared, g->compute, a);
     if (!h3_launch_status(g, "Sage attention")) {

@@ -1,6 +1,7 @@
 """BF16 DiT attention on the GPU vs the CPU oracle (reference
 src/cuda/cuda_attention.cuh:7-51 restated in oracle/attention.c), through the C ABI."""
 import math
+import os
 
 import numpy as np
 import pytest
@@ -13,16 +14,52 @@ from tests.helpers import ATTN_COSINE, ATTN_MAX_ABS, bf16, metrics, scale_bf16, 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module")
-def gpu():
-    g = Gpu()
+def context(variant):
+    """A context of attention variant `variant` (H3_HIP_ATTENTION_VARIANT, read when it is
+    created). 15 takes the kernels of 256-query tiles also for few query rows."""
+    before = os.environ.get("H3_HIP_ATTENTION_VARIANT")
+    os.environ["H3_HIP_ATTENTION_VARIANT"] = variant
+    try:
+        g = Gpu()
+    finally:
+        os.environ.pop("H3_HIP_ATTENTION_VARIANT")
+        if before is not None:
+            os.environ["H3_HIP_ATTENTION_VARIANT"] = before
+    g.variant = variant
+    return g
+
+
+@pytest.fixture(scope="module", params=["0", "15"], ids=["default", "tiles"])
+def gpu(request):
+    """The default choice, which takes attn_small for every shape of these tests that does
+    not say otherwise, and the tile kernels on the same shapes."""
+    g = context(request.param)
     yield g
     g.close()
+
+
+@pytest.fixture(scope="module")
+def default():
+    g = context("0")
+    yield g
+    g.close()
+
+
+@pytest.fixture(scope="module")
+def tiles():
+    g = context("15")
+    yield g
+    g.close()
+
+
+def tile_kernel(seq):
+    return "attn_bf16_pipe" if seq > 256 else "attn_bf16_wide"
 
 
 def _check(gpu, q, k, v, seq, heads, head_major=False, dit=True, rows=None):
     print(f"[attention] seq={seq} heads={heads} head_major={head_major} dit={dit}", flush=True)
     out = sdpa(gpu, q, k, v, seq, heads, head_major=head_major, dit=dit)
+    assert gpu.last_kernel().startswith(tile_kernel(seq) if gpu.variant == "15" else "attn_small"), gpu.last_kernel()
     scale = scale_bf16(1 / math.sqrt(128))
     r0, r1 = rows if rows else (0, seq)
     ref = oracle.attention(bf16(q), bf16(k), bf16(v), seq, heads, scale, tile=64, rows=(r0, r1))
@@ -95,7 +132,7 @@ def test_score_growth(gpu, pattern):
         assert m["max_abs"] <= ATTN_MAX_ABS and m["cosine"] >= ATTN_COSINE, m
 
 
-def test_recomputation_launch_matches_tile_max_kernel(gpu, monkeypatch):
+def test_recomputation_launch_matches_tile_max_kernel(tiles):
     """A 130-log2-unit spike overflows P in every workgroup of the default
     kernel, so the recomputation launch redoes all rows with the per-tile-max
     kernel (attention variant 3): the two outputs agree bit for bit. A rising
@@ -103,37 +140,39 @@ def test_recomputation_launch_matches_tile_max_kernel(gpu, monkeypatch):
     of variant 3."""
     seq, heads = 1500, 2
     q, k, v = _growth_inputs(seq, heads, "spike")
-    fast = sdpa(gpu, q, k, v, seq, heads)
-    monkeypatch.setenv("H3_HIP_ATTENTION_VARIANT", "3")
-    g3 = Gpu()
+    fast = sdpa(tiles, q, k, v, seq, heads)
+    assert tiles.last_kernel() == "attn_bf16_pipe"
+    g3 = context("3")
     try:
         assert np.array_equal(sdpa(g3, q, k, v, seq, heads), fast)
+        assert g3.last_kernel() == "attn_bf16_wide"
         q, k, v = _growth_inputs(seq, heads, "rise")
-        m = metrics(bf16(sdpa(gpu, q, k, v, seq, heads)), bf16(sdpa(g3, q, k, v, seq, heads)))
+        m = metrics(bf16(sdpa(tiles, q, k, v, seq, heads)), bf16(sdpa(g3, q, k, v, seq, heads)))
         assert m["max_abs"] <= ATTN_MAX_ABS and m["cosine"] >= ATTN_COSINE, m
     finally:
         g3.close()
 
 
 @pytest.mark.parametrize("seq,heads", [(4200, 2), (65, 3), (1, 1)])
-def test_global_load_path_matches_buffer_path(gpu, monkeypatch, seq, heads):
+def test_global_load_path_matches_buffer_path(tiles, seq, heads):
     """K and V^T below 4 GiB load their tiles with buffer loads (keys past the
     sequence read as zeros); larger tensors take the global-load path (rows
     clamped to the last key), forced here with attention variant 13. Both
     mask the same keys, so the outputs agree bit for bit, ragged tails
     included."""
     q, k, v = synth.attention_inputs(seq, heads, seed=31, scale=0.5)
-    buffered = sdpa(gpu, q, k, v, seq, heads)
-    monkeypatch.setenv("H3_HIP_ATTENTION_VARIANT", "13")
-    g13 = Gpu()
+    buffered = sdpa(tiles, q, k, v, seq, heads)
+    assert tiles.last_kernel() == tile_kernel(seq)
+    g13 = context("13")
     try:
         assert np.array_equal(sdpa(g13, q, k, v, seq, heads), buffered)
+        assert g13.last_kernel() == "attn_bf16_wide (global loads)"
     finally:
         g13.close()
 
 
 @pytest.mark.parametrize("case", ["257x3", "300x40", "4200x2", "8191x2", "rise", "fall", "spike"])
-def test_scheduled_kernel_matches_wide_kernel(gpu, monkeypatch, case):
+def test_scheduled_kernel_matches_wide_kernel(tiles, case):
     """Sequences above 256 keys run the hand-scheduled kernel (four waves of
     64 queries); attention variant 14 forces the compiler-scheduled wide
     kernel (eight waves of 32). Both compute the same products, sums and
@@ -147,24 +186,25 @@ def test_scheduled_kernel_matches_wide_kernel(gpu, monkeypatch, case):
         seq, heads = 1500, 2
         q, k, v = _growth_inputs(seq, heads, case)
     print(f"[attention] scheduled vs wide {case}", flush=True)
-    pipe = sdpa(gpu, q, k, v, seq, heads)
-    monkeypatch.setenv("H3_HIP_ATTENTION_VARIANT", "14")
-    g14 = Gpu()
+    pipe = sdpa(tiles, q, k, v, seq, heads)
+    assert tiles.last_kernel() == "attn_bf16_pipe"
+    g14 = context("14")
     try:
         assert np.array_equal(sdpa(g14, q, k, v, seq, heads), pipe)
+        assert g14.last_kernel() == "attn_bf16_wide"
     finally:
         g14.close()
 
 
 @pytest.mark.parametrize("variant,kind", [("14", "rise"), ("14", "fall"), ("14", "spike"), ("3", "spike")])
-def test_tile_kernels_agree_at_many_heads(gpu, monkeypatch, variant, kind):
-    """As the two tests above, with enough query rows that the 256-query tile
-    kernels run (few rows take a kernel of their own under every variant)."""
+def test_tile_kernels_agree_at_many_heads(default, variant, kind):
+    """As the two tests above, with enough query rows that the default choice
+    is the 256-query tile kernel."""
     seq, heads = 1500, 42
     q, k, v = (np.tile(x.reshape(seq, 2, 128), (1, 21, 1)).reshape(-1) for x in _growth_inputs(seq, 2, kind))
-    fast = sdpa(gpu, q, k, v, seq, heads)
-    monkeypatch.setenv("H3_HIP_ATTENTION_VARIANT", variant)
-    g = Gpu()
+    fast = sdpa(default, q, k, v, seq, heads)
+    assert default.last_kernel() == "attn_bf16_pipe"
+    g = context(variant)
     try:
         assert np.array_equal(sdpa(g, q, k, v, seq, heads), fast)
     finally:
@@ -172,21 +212,23 @@ def test_tile_kernels_agree_at_many_heads(gpu, monkeypatch, variant, kind):
 
 
 @pytest.mark.parametrize("head_major", [False, True])
-@pytest.mark.parametrize("seq,heads", [
-    (31, 2),      # part of one query block, one wave's tile
-    (33, 1),      # two query blocks
-    (64, 3),      # one whole tile
-    (257, 3),     # five tiles: one wave takes two
-    (1024, 8),    # the most rows of one block per workgroup
-    (2050, 8),    # two blocks per workgroup, ragged
+@pytest.mark.parametrize("seq,heads,rows", [
+    (31, 2, 32),      # part of one query block, one wave's tile
+    (33, 1, 32),      # two query blocks
+    (64, 3, 32),      # one whole tile
+    (257, 3, 32),     # five tiles: one wave takes two
+    (1024, 8, 32),    # the most rows of one block per workgroup
+    (300, 40, 64),    # two blocks per workgroup
+    (2047, 8, 64),    # the same, ragged, every workgroup on a CU of its own
 ])
-def test_few_rows_every_element(gpu, seq, heads, head_major):
+def test_few_rows_every_element(default, seq, heads, rows, head_major):
     """Few query rows (a kernel of their own) against FP64 on every element:
     P and the output are rounded to BF16 (2^-9 relative), so an output is
     within 2^-8 sum p |v| of the exact one."""
     print(f"[attention] few rows seq={seq} heads={heads} head_major={head_major}", flush=True)
     q, k, v = synth.attention_inputs(seq, heads, seed=seq, scale=1.0)
-    got = bf16(sdpa(gpu, q, k, v, seq, heads, head_major=head_major)).reshape(seq, heads, 128)
+    got = bf16(sdpa(default, q, k, v, seq, heads, head_major=head_major)).reshape(seq, heads, 128)
+    assert default.last_kernel() == f"attn_small rows={rows}"
     scale = scale_bf16(1 / math.sqrt(128))
     qf, kf, vf = (bf16(x).reshape(seq, heads, 128).astype(np.float64) for x in (q, k, v))
     for h in range(heads):
@@ -197,19 +239,24 @@ def test_few_rows_every_element(gpu, seq, heads, head_major):
         assert np.all(np.abs(got[:, h] - p @ vf[:, h]) <= bound), h
 
 
-@pytest.mark.parametrize("row", [0, 200, 383, 699])
+@pytest.mark.parametrize("seq,heads,row", [(700, 3, 0), (700, 3, 200), (700, 3, 383), (700, 3, 699),
+                                           (300, 40, 0), (300, 40, 130), (300, 40, 299)])
 @pytest.mark.parametrize("which,value", [(0, np.inf), (1, -np.inf), (1, np.nan), (2, np.inf)])
-def test_few_rows_nonfinite(gpu, which, value, row):
+@pytest.mark.parametrize("variant", ["0", "15"])
+def test_few_rows_nonfinite(variant, which, value, seq, heads, row):
     """One Inf or NaN anywhere in Q, K or V is reported, also where its scores
-    are all -Inf and the output stays finite."""
-    seq, heads = 700, 3
+    are all -Inf and the output stays finite: one block per workgroup, two, and
+    the tile kernel."""
     x = [synth.bf16_to_f32(t).reshape(seq, heads, 128).copy() for t in synth.attention_inputs(seq, heads, seed=3)]
     if which == 1 and value == -np.inf:
         x[0] = np.abs(x[0])      # -Inf times positive queries: every score -Inf
     x[which][row, 1, 77] = value
     bits = [synth.f32_to_bf16(t.reshape(-1)) for t in x]
-    with Gpu() as g, pytest.raises(Exception, match="nonfinite"):
-        sdpa(g, *bits, seq, heads)
+    with context(variant) as g:
+        with pytest.raises(Exception, match="nonfinite"):
+            sdpa(g, *bits, seq, heads)
+        kernel = {"15": "attn_bf16_pipe", "0": f"attn_small rows={32 if heads == 3 else 64}"}[variant]
+        assert g.last_kernel() == kernel
 
 
 @pytest.mark.parametrize("seq,heads", [(700, 3), (2048, 8)])
