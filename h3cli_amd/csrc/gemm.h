@@ -18,11 +18,10 @@ struct GemmPlan {
 // Measured rates of a kernel in microseconds, one workgroup on each CU: a K unit of a tile in
 // a whole wave (full); in a wave that occupies a part f of the CUs, part + rise * max(0, f -
 // knee), because fewer busy CUs draw less power and clock higher (7168 -> 5376, BF16, 84 /
-// 168 / 252 tiles: 114 / 128 / 153); start per round of workgroups; and for split tiles
-// their second launch (fixed), each share's 256 x 256 partial sums (sum) and each share added
-// in turn (turn).
+// 168 / 252 tiles: 114 / 128 / 153); start per wave of workgroups; and for split tiles each
+// share's 256 x 256 partial sums, written and read (sum), and each share added in turn (turn).
 struct GemmRates {
-    float full, part, rise, knee, start, fixed, sum, turn;
+    float full, part, rise, knee, start, sum, turn;
 };
 
 // The modelled time of `tiles` output tiles of `units` K units, `size` times 256 x 256 each, and
@@ -36,14 +35,15 @@ inline GemmPlan gemm_last_wave(const h3_gpu *g, unsigned tiles, unsigned units, 
                                unsigned least_units = 1) {
     const unsigned rest = tiles % g->cus, waves = tiles / g->cus, rounds_max = waves == 1 ? 2 : 1;
     auto unit = [&](float busy) { return r.part + r.rise * (busy > r.knee ? busy - r.knee : 0.f); };
-    const float before = (float)waves * units * r.full + r.start;
-    GemmPlan p{before + (rest ? units * unit((float)rest / g->cus) : 0.f), 0, 1, false};
-    if (!rest || waves >= 8) return p;
+    GemmPlan p{(float)waves * (units * r.full + r.start), 0, 1, false};
+    if (!rest) return p;
+    const float before = p.us;
+    p.us += units * unit((float)rest / g->cus) + r.start;
+    if (waves >= 8) return p;
     for (unsigned s = 2; s <= 32 && s * least_units <= units && rest * s <= rounds_max * g->cus; s++) {
         const unsigned rounds = (rest * s + g->cus - 1) / g->cus;
         const float busy = (float)(rest * s) / (rounds * g->cus);
-        const float t = before + rounds * ((units + s - 1) / s * unit(busy) + r.start) - r.start + r.fixed +
-                        rest * s * size * r.sum + s * r.turn;
+        const float t = before + rounds * ((units + s - 1) / s * unit(busy) + r.start) + rest * s * size * r.sum + s * r.turn;
         if (t < p.us) { p.us = t; p.split = s; }
     }
     return p;

@@ -535,29 +535,31 @@ int launch_small(h3_gpu *g, const GemmArgs &a, bool q8) {
 // ------------------------------------------------------------ choice of the kernel
 // The fastest of the kernels that take this projection, by gemm_last_wave with rates fitted
 // to the measured times of all plans of eight projections (K, N 5120 to 28672) of 33 to 24000
-// rows, BF16, int8 with one scale per column and int8 of group 64: the plan taken is 0.5%
-// slower than the best one in the mean, 13% at most, and never 2% slower than whole tiles of
-// the pipe kernel. Converting a weight to BF16 first takes 0.4 to 1.2 us per million values,
-// most for a long K, whose rows share the cache with the weight. What is not the pipe kernel
-// on whole tiles must promise 2%. Measured, in microseconds, the runner-up in brackets: 729
-// rows, 7168 -> 5376, BF16: pipe in 4 shares 61 (whole 113); 729 rows, 5376 -> 28672, int8 of
-// group 64: mid 256 in 3 shares 260 (pipe in 3 281), per column: q8 in 3 shares 213 (mid 240);
-// 729 rows, 5120 -> 13824, group 64: pipe 122 (mid 151); 1800 rows, 14336 -> 5376, per column:
-// q8 292 (pipe 315); 64 rows, 5376 -> 28672, BF16: mid 64 in 2 shares 61 (pipe 114).
+// rows and of ten narrow or short ones (K 256 to 5376, N 64 to 5376) of 33 to 24000 rows: BF16,
+// int8 with one scale per column and int8 of group 64. The plan taken is 0.5% (narrow: 1.6%)
+// slower than the best one in the mean, and never 2% slower than whole tiles of the pipe
+// kernel for the wide ones. Converting a weight to BF16 first takes 0.4 to 1.2 us per million
+// values, most for a long K, whose rows share the cache with the weight. What is not the pipe
+// kernel on whole tiles must promise 2%. Measured, in microseconds, the runner-up in brackets:
+// 729 rows, 7168 -> 5376, BF16: pipe in 4 shares 61 (whole 113); 729 rows, 5376 -> 28672, int8
+// of group 64: mid 256 in 3 shares 260 (pipe in 3 281), per column: q8 in 3 shares 213 (mid
+// 240); 729 rows, 5120 -> 13824, group 64: pipe 122 (mid 151); 1800 rows, 14336 -> 5376, per
+// column: q8 292 (pipe 315); 64 rows, 5376 -> 28672, BF16: mid 64 in 2 shares 61 (pipe 114); 256
+// rows, 5376 -> 64, BF16: mid 64 in 10 shares 12.5 (mid 128 in 16 14.7).
 GemmPlan choose(const h3_gpu *g, const GemmArgs &a, bool q8, bool may_convert) {
-    static constexpr GemmRates PIPE{2.89f, 1.96f, 1.72f, .65f, 6.4f, .6f, .044f, .41f};      // per 128 values of K
-    static constexpr GemmRates CODES{1.73f, 1.22f, .93f, .57f, 8.5f, 1.3f, .03f, .95f};      // gemm_q8; per 64, as all below
-    static constexpr GemmRates MID_BF16[3] = {{.61f, .5f, .58f, .74f, 4.1f, 1.4f, .085f, .39f},
-                                              {.98f, .75f, .65f, .66f, 3.8f, .7f, .083f, .02f},
-                                              {1.95f, 1.5f, .8f, .55f, 3.f, 5.f, .04f, 0.f}};
-    static constexpr GemmRates MID_COLUMN[3] = {{.88f, .74f, .22f, .47f, 4.7f, 5.f, .042f, .11f},
-                                                {1.17f, 1.03f, .19f, .2f, 2.5f, 5.f, .057f, 0.f},
-                                                {1.94f, 1.4f, .6f, .2f, 3.4f, 8.3f, .03f, 0.f}};
-    static constexpr GemmRates MID_GROUP[3] = {{1.08f, 1.f, .22f, .47f, 5.f, 4.7f, .045f, .08f},
-                                               {1.38f, 1.24f, .25f, .2f, 2.f, 6.f, .054f, 0.f},
-                                               {2.01f, 1.66f, .63f, .54f, 2.f, 8.6f, .042f, 0.f}};
+    static constexpr GemmRates PIPE{2.68f, 1.93f, 1.61f, .58f, 8.7f, .048f, .33f};       // per 128 values of K
+    static constexpr GemmRates CODES{1.55f, 1.1f, .93f, .51f, 15.9f, .018f, .83f};       // gemm_q8; per 64, as all below
+    static constexpr GemmRates MID_BF16[3] = {{.6f, .41f, .19f, .15f, 5.5f, .104f, .16f},
+                                              {.9f, .68f, .48f, .6f, 7.f, .088f, .09f},
+                                              {1.73f, 1.02f, .61f, .15f, 7.9f, .06f, .02f}};
+    static constexpr GemmRates MID_COLUMN[3] = {{.85f, .72f, .06f, .15f, 7.2f, .113f, .15f},
+                                                {1.08f, .95f, .05f, .15f, 8.4f, .094f, .09f},
+                                                {1.82f, 1.4f, .46f, .15f, 11.5f, .06f, .02f}};
+    static constexpr GemmRates MID_GROUP[3] = {{1.07f, .91f, .11f, .15f, 7.3f, .108f, .15f},
+                                               {1.23f, 1.06f, .18f, .15f, 8.3f, .091f, .09f},
+                                               {1.91f, 1.48f, .45f, .15f, 11.5f, .059f, .03f}};
     GemmPlan best{3.4e38f, 0, 1, false};
-    const float convert = q8 ? (float)a.n * a.k * (.4e-6f + 3e-11f * a.k) + 4.f : 0.f;
+    const float convert = q8 ? (float)a.n * a.k * (.4e-6f + 3e-11f * a.k) + 3.f : 0.f;
     auto consider = [&](GemmPlan p, unsigned tm, bool dequant) {
         p.tm = tm;
         p.dequant = dequant;

@@ -265,7 +265,7 @@ int h3_gemm_fp8(h3_gpu *g, Fp8GemmArgs a) {
     // Shared over K where all tiles are at most half a wave, in shares of eight K tiles or
     // more, so that short sums keep one order (14336 -> 5376: 1024 rows, 84 tiles: 3 shares
     // 94 us, whole 136; 2048 rows, 168 tiles: whole 156, 3 shares 199).
-    static constexpr GemmRates RATES{1.5f, 1.5f, 0.f, 1.f, 2.f, 3.f, .09f, .9f};
+    static constexpr GemmRates RATES{1.5f, 1.5f, 0.f, 1.f, 2.f, .09f, .9f};
     const unsigned split = tiles < g->cus ? gemm_last_wave(g, tiles, a.k / TK, RATES, 1.f, 8).split : 1;
     a.tile = split_last_wave(g, tiles, split, a.k / TK, TM * TN);
     const unsigned rest = tiles - a.tile.full;
