@@ -200,7 +200,8 @@ static int dispatch(h3_gpu *g, h3_gpu_tensor *out, const h3_gpu_tensor *q, const
                                (const uint16_t *)v->data, seq, heads, scale, head_major, list, cnt, stride);
         if (ok) g->stats.sage2_attention_dispatches++;
     } else {
-        ok = h3_buffer_reserve(g, &s->bf16_ws, h3_attention_bf16_workspace(seq, heads), "attention workspace") &&
+        const bool small = !list && h3_attention_small_blocks(g, seq, heads);
+        ok = (small || h3_buffer_reserve(g, &s->bf16_ws, h3_attention_bf16_workspace(seq, heads), "attention workspace")) &&
              h3_launch_attention_bf16(g, s->bf16_ws.ptr, (uint16_t *)out->data, (const uint16_t *)q->data, (const uint16_t *)k->data,
                                       (const uint16_t *)v->data, seq, heads, scale, head_major, list, cnt, stride);
     }

@@ -1944,11 +1944,8 @@ int h3_launch_attention_bf16(h3_gpu *g, void *workspace, uint16_t *out, const ui
     a.fault = g->fault;
     // Variant 13: the global-load path that tensors of 4 GiB and more take.
     a.buffered = fits_buffer(a) && g->attention_variant != 13;
-    // Few query rows. Every other variant is one of the tile kernels (15: the default one).
-    if (!kv_list && g->attention_variant == 0) {
-        const int blocks = h3_attention_small_blocks(g, seq, heads);
-        if (blocks) return h3_launch_attention_small(g, blocks, out, q, k, v, seq, heads, scale, head_major);
-    }
+    if (const int blocks = kv_list ? 0 : h3_attention_small_blocks(g, seq, heads))
+        return h3_launch_attention_small(g, blocks, out, q, k, v, seq, heads, scale, head_major);
     hipLaunchKernelGGL(transpose_v, dim3(a.padded / BN, heads), dim3(256), 0, g->compute, v, k, (uint16_t *)workspace,
                        seq, heads, a.padded, g->fault);
     if (!h3_launch_status(g, "V transpose")) return 0;

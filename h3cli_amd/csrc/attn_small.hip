@@ -308,7 +308,8 @@ int launch(h3_gpu *g, const SmallArgs &a) {
 // block 17.0, two 24.5 (35.2); 300 x 4: 12.1, 18.6 (23.1); 2048 x 8: 41.8, 35.5 (53.1);
 // 4200 x 2: 73.8, 59.1 (86.4); 1024 x 24: 41.4, 47.0 (41.0).
 int h3_attention_small_blocks(const h3_gpu *g, uint32_t seq, uint32_t heads) {
-    if ((size_t)seq * heads * D * 2 >= (1ull << 32)) return 0;          // 32-bit buffer offsets
+    // Every other variant is one of the tile kernels (15: the default one).
+    if (g->attention_variant || (size_t)seq * heads * D * 2 >= (1ull << 32)) return 0;   // 32-bit buffer offsets
     const float tiles = (float)((seq + BN * WAVES - 1) / (BN * WAVES));   // of the busiest wave
     auto rounds = [&](uint32_t queries) {
         return (float)(((uint64_t)((seq + queries - 1) / queries) * heads + g->cus - 1) / g->cus);

@@ -14,6 +14,8 @@ int h3_tensor_acquire(h3_gpu *g, const h3_gpu_tensor *t);
 int h3_tensor_release(h3_gpu *g, const h3_gpu_tensor *t);
 
 // Launch helpers of the kernel translation units (all enqueue on g->compute).
+// The workspace of the tile kernels; a dense call that h3_attention_small_blocks takes
+// needs none.
 size_t h3_attention_bf16_workspace(uint32_t seq, uint32_t heads);
 int h3_launch_attention_bf16(h3_gpu *g, void *workspace, uint16_t *out, const uint16_t *q, const uint16_t *k,
                              const uint16_t *v, uint32_t seq, uint32_t heads, float scale,
@@ -21,7 +23,7 @@ int h3_launch_attention_bf16(h3_gpu *g, void *workspace, uint16_t *out, const ui
                              uint32_t list_stride);
 // attn_small.hip: dense attention of few query rows, in one launch with no workspace.
 // The 32-query blocks per workgroup it takes for this shape (1 or 2), 0 where the
-// 256-query tiles are faster.
+// 256-query tiles are faster or the variant selector asks for one of their kernels.
 int h3_attention_small_blocks(const h3_gpu *g, uint32_t seq, uint32_t heads);
 int h3_launch_attention_small(h3_gpu *g, int blocks, uint16_t *out, const uint16_t *q, const uint16_t *k,
                               const uint16_t *v, uint32_t seq, uint32_t heads, float scale, bool head_major);

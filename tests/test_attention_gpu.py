@@ -1,5 +1,6 @@
 """BF16 DiT attention on the GPU vs the CPU oracle (reference
 src/cuda/cuda_attention.cuh:7-51 restated in oracle/attention.c), through the C ABI."""
+import ctypes as C
 import math
 import os
 
@@ -7,6 +8,7 @@ import numpy as np
 import pytest
 
 from h3cli_amd import synth
+from h3cli_amd._lib import GpuStats
 from h3cli_amd.runtime import Gpu
 from oracle import oracle
 from tests.helpers import ATTN_COSINE, ATTN_MAX_ABS, bf16, metrics, scale_bf16, sdpa
@@ -257,6 +259,18 @@ def test_few_rows_nonfinite(variant, which, value, seq, heads, row):
             sdpa(g, *bits, seq, heads)
         kernel = {"15": "attn_bf16_pipe", "0": f"attn_small rows={32 if heads == 3 else 64}"}[variant]
         assert g.last_kernel() == kernel
+
+
+def test_few_rows_need_no_workspace():
+    """The kernel of few query rows reads V as it is: no transposed copy is allocated for it."""
+    seq, heads = 700, 3
+    q, k, v = synth.attention_inputs(seq, heads, seed=5)
+    for variant, held in (("0", False), ("15", True)):
+        g, s = context(variant), GpuStats()
+        sdpa(g, q, k, v, seq, heads)
+        g.lib.h3_gpu_get_stats(g.handle, C.byref(s))
+        assert (s.attention_workspace_bytes > 0) == held
+        g.close()
 
 
 @pytest.mark.parametrize("seq,heads", [(700, 3), (2048, 8)])
