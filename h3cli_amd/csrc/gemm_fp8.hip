@@ -27,6 +27,7 @@
 #include "internal.h"
 #include "gemm.h"
 #include "gemm_fp8.h"
+#include <algorithm>
 
 namespace {
 
@@ -136,9 +137,10 @@ void fp8_gemm_pipe(Fp8GemmArgs a) {
                       (int)__builtin_amdgcn_readfirstlane((unsigned)(wbase >> 32)),
                       (int)__builtin_amdgcn_readfirstlane(wrows * a.k - k0), 0x00020000};
     const unsigned lrow = 8 * wave + lane / 8;
-    unsigned o[8];
+    unsigned o[8];     // offsets of 4 GiB and more belong to rows past M and N (h3_gemm_fp8): BUFFER_OOB
 #pragma unroll
-    for (int t = 0; t < 8; t++) o[t] = (lrow + 32 * t) * a.k + swz(lrow, lane % 8) * 16;
+    for (int t = 0; t < 8; t++)
+        o[t] = __umulhi(lrow + 32 * t, a.k) ? BUFFER_OOB : (lrow + 32 * t) * a.k + swz(lrow, lane % 8) * 16;
     const unsigned mb = __builtin_amdgcn_readfirstlane(wave * 1024);
     const unsigned kmax = __builtin_amdgcn_readfirstlane((ksteps - 1) * TK);
     const unsigned kone = min(kmax, (unsigned)TK);
@@ -260,6 +262,18 @@ int h3_gemm_fp8(h3_gpu *g, Fp8GemmArgs a) {
                               "FP8 GEMM shared memory"))
                 return 0;
         configured = true;
+    }
+    // Offsets inside a tile's rows have 32 bits. N * K has no more (h3_gpu_quant_load), so from
+    // K = 2^24 on the weight has 128 rows, and those of x are taken 128 at a time.
+    if ((uint64_t)TM * a.k > UINT32_MAX && a.m > TM / 2) {
+        Fp8GemmArgs part = a;
+        for (unsigned row = 0; row < a.m; row += TM / 2) {
+            part.x = a.x + (size_t)row * a.k;
+            part.y = a.y + (size_t)row * a.n;
+            part.m = std::min(a.m - row, TM / 2u);
+            if (!h3_gemm_fp8(g, part)) return 0;
+        }
+        return 1;
     }
     const unsigned tiles = (a.m + TM - 1) / TM * ((a.n + TN - 1) / TN);
     // Shared over K where all tiles are at most half a wave, in shares of eight K tiles or

@@ -337,6 +337,43 @@ def test_errors_and_nonfinite(tmp_path):
             load(g, tmp_path / "bad.bin", n, k)
 
 
+def normal_row(seed, row, k):
+    """Row `row` of a [rows, k] tensor that h3_hip_fill_normal_bf16 fills (k even), in 64 bits."""
+    at = np.uint64(seed << 40) + np.uint64(row * k) + np.arange(0, k, 2, dtype=np.uint64)
+    u = [(synth.splitmix64(at + np.uint64(i)) >> np.uint64(11)).astype(np.float64) for i in (0, 1)]
+    r, turn = np.sqrt(-2 * np.log((u[0] + 1) * 2.0 ** -53)), 2 * np.pi * 2.0 ** -53 * u[1]
+    return np.stack([r * np.cos(turn), r * np.sin(turn)], 1).reshape(-1)
+
+
+def test_tile_rows_of_4_gib(tmp_path):
+    """256 rows of K = 2^24 codes are 4 GiB, more than the kernel's 32-bit offsets reach.
+    Against the unquantized product: a code is off by at most 2^-4 of its value, 0.036 in the
+    2-norm, so the 32 results, each from two such operands, by 0.051 and by chance 0.08."""
+    m, n, k = 256, 128, 1 << 24
+    say(f"fp8 gemm m={m} n={n} k={k}")
+    with Gpu() as g:
+        g.check(configure(g, tmp_path / "cache"), "configure")
+        x, w, out = g.empty(m * k), g.empty(n * k), g.empty(m * n)
+        g.begin()
+        g.check(g.lib.h3_hip_fill_normal_bf16(g.handle, x.handle, 3, C.c_float(1.0), m * k), "fill")
+        g.check(g.lib.h3_hip_fill_normal_bf16(g.handle, w.handle, 4, C.c_float(1.0), n * k), "fill")
+        g.submit()
+        packed = g._track(g.lib.h3_hip_quant_weight_from_bf16(g.handle, w.handle, n, k), packed_size(n, k)[2], _lib.I8)
+        g.begin()
+        g.check(g.lib.h3_gpu_linear_bf16(g.handle, out.handle, x.handle, packed.handle, None, m, k, n), "linear")
+        g.submit()
+        rows, cols = [0, 127, 128, 255], [0, 1, 31, 32, 63, 64, 126, 127]
+        got = synth.bf16_to_f32(out.read()).reshape(m, n)[np.ix_(rows, cols)]
+    say("reference")
+    xv = [normal_row(3, r, k) for r in rows]
+    want = np.zeros((len(rows), len(cols)))
+    for j, c in enumerate(cols):
+        wv = normal_row(4, c, k)
+        want[:, j] = [row @ wv for row in xv]
+    off = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert off <= 0.08, off
+
+
 @pytest.mark.parametrize("m,n,k", [(300, 512, 384), (7, 256, 256), (257, 768, 1024)])
 def test_nvfp4_gemm_against_oracle(tmp_path, m, n, k):
     """NVFP4 projections: the activation packs exactly as the oracle does
