@@ -70,8 +70,8 @@ def synthetic_q8(seed, n, k, group):
     (513, 1024, 512, 64, True, False),      # reference q8 recipe (group 64) + bias
     (256, 768, 768, 768, False, True),      # fused GELU-tanh epilogue
     (33, 256, 256, 256, False, False),      # M smaller than a tile
-    (300, 1024, 512, 1024, True, False),    # hand-scheduled GEMM, bias epilogue
-    (300, 1024, 512, 1024, True, True),     # hand-scheduled GEMM, bias + GELU-tanh epilogue
+    (300, 1024, 512, 1024, True, False),    # split tiles, bias epilogue
+    (300, 1024, 512, 1024, True, True),     # split tiles, bias + GELU-tanh epilogue
     (50, 100, 30, 100, True, False),        # unaligned shape: small-GEMM path
 ])
 def test_w8a16_linear(gpu, m, k, n, group, bias, gelu):
@@ -231,6 +231,101 @@ def test_mid_rows_linear(gpu, m, k, n, group, bias, gelu):
     """Row tiles of 64 to 256 and their remainders against FP64, bound as in
     test_few_rows_linear."""
     test_few_rows_linear(gpu, m, k, n, group, bias, gelu)
+
+
+PIPE_WHOLE, PIPE_SPLIT = (2255, 128, 3840), (1690, 256, 9472)     # 135 and 256 + 3 tiles, ragged rows
+
+
+@pytest.mark.parametrize("m,k,n,group,bias,gelu,kernel", [
+    *[(*shape, 0, bias, gelu, kernel)
+      for shape, kernel in ((PIPE_WHOLE, "gemm_bf16_pipe"), (PIPE_SPLIT, "gemm_bf16_pipe shares=2"))
+      for bias in (False, True) for gelu in (False, True)],
+    (600, 7168, 5376, 0, True, True, "gemm_bf16_pipe shares=4"),              # no whole wave
+    (1163, 128, 8192, 64, True, True, "gemm_bf16_pipe converted"),
+    (2786, 512, 6144, 64, True, False, "gemm_bf16_pipe shares=4 converted"),
+    (1076, 128, 7424, 128, False, True, "gemm_bf16_pipe converted"),
+    (3316, 256, 4928, 0, True, True, "gemm_mid rows=256 shares=4"),
+    (8571, 64, 817, 0, True, False, "gemm_mid rows=256"),                     # odd width, one K step
+    (960, 6080, 2578, 6080, False, True, "gemm_mid rows=256 shares=5"),
+    (303, 192, 30464, 192, True, False, "gemm_mid rows=256"),
+    (748, 5824, 2825, 64, True, True, "gemm_mid rows=256 shares=7"),          # odd width
+    (309, 192, 32256, 64, False, False, "gemm_mid rows=256"),
+    (1458, 64, 5478, 64, True, True, "gemm_mid rows=256 converted"),
+    (729, 5376, 28672, 64, False, False, "gemm_mid rows=256 shares=3"),
+    (1275, 4096, 1545, 0, True, False, "gemm_mid rows=128 shares=3"),
+    (2976, 64, 1408, 0, False, True, "gemm_mid rows=128"),
+    (589, 3968, 2176, 3968, True, True, "gemm_mid rows=128 shares=5"),
+    (1244, 64, 3254, 64, True, False, "gemm_mid rows=128"),
+    (210, 2240, 5632, 64, False, False, "gemm_mid rows=128 shares=5"),
+    (1242, 128, 3324, 64, True, True, "gemm_mid rows=128"),
+    (81, 192, 64, 0, True, True, "gemm_mid rows=64 shares=3"),
+    (179, 64, 30, 0, True, False, "gemm_mid rows=64"),
+    (296, 128, 43, 128, True, False, "gemm_mid rows=64 shares=2"),
+    (51, 320, 62, 64, False, True, "gemm_mid rows=64 shares=5"),
+    (75, 128, 5720, 64, True, True, "gemm_mid rows=64"),
+    (755, 2304, 5504, 2304, True, True, "gemm_q8_pipe shares=3"),
+    (653, 960, 11264, 960, False, False, "gemm_q8_pipe"),
+])
+def test_linear_plans(gpu, m, k, n, group, bias, gelu, kernel):
+    """Each kernel of many rows with whole and split tiles, each weight format and epilogue,
+    and that it is the one that ran; bound as in test_few_rows_linear, rows at the edges of
+    tiles and between."""
+    print(f"[plans] m={m} k={k} n={n} group={group} bias={bias} gelu={gelu} {kernel}", flush=True)
+    x = synth.normal_bf16(m + 3, m * k)
+    b = synth.normal_bf16(7, n, scale=0.1) if bias else None
+    if group:
+        codes, scales = synthetic_q8(m + n, n, k, group)
+        w = q8_weight(gpu, codes, scales, n, k, group)
+    else:
+        bits = synth.normal_bf16(m + 4, n * k, scale=1 / math.sqrt(k))
+        w = gpu.from_bf16(bits)
+    tx, tb, out = gpu.from_bf16(x), gpu.from_bf16(b) if bias else None, gpu.empty(m * n)
+    fn = gpu.lib.h3_hip_linear_gelu_bf16 if gelu else gpu.lib.h3_gpu_linear_bf16
+    run(gpu, fn, out.handle, tx.handle, w.handle, tb.handle if bias else None, m, k, n)
+    assert gpu.last_kernel() == kernel
+    edges = np.arange(64, m, 64)
+    rows = np.unique(np.r_[0:m:max(1, m // 16), edges[:8], edges[:8] - 1, edges[-2:], edges[-2:] - 1, m - 1])
+    got = bf16(out.read()).reshape(m, n)[rows]
+    xv = bf16(x).reshape(m, k)[rows].astype(np.float64)
+    for at in range(0, n, 4096):
+        cols = slice(at, min(at + 4096, n))
+        if group:
+            wide = np.repeat(scales.reshape(n, -1)[cols], group, axis=1)[:, :k]
+            wt = bf16(synth.f32_to_bf16(codes.reshape(n, k)[cols].astype(np.float32) * wide)).astype(np.float64)
+        else:
+            wt = bf16(bits.reshape(n, k)[cols]).astype(np.float64)
+        want = xv @ wt.T + (bf16(b)[cols].astype(np.float64) if bias else 0.0)
+        bound = 2.0 ** -8 * np.abs(want) + k * 2.0 ** -24 * (np.abs(xv) @ np.abs(wt).T)
+        if gelu:
+            want = 0.5 * want * (1 + np.tanh(math.sqrt(2 / math.pi) * (want + 0.044715 * want ** 3)))
+            bound = 1.13 * bound + 2.0 ** -8 * np.abs(want) + 2.0 ** -20
+        assert np.all(np.abs(got[:, cols] - want) <= bound), float(np.max(np.abs(got[:, cols] - want) / bound))
+    for t in (tx, out, w) + ((tb,) if bias else ()):
+        gpu.free(t)
+
+
+@pytest.mark.parametrize("m,k,hidden,group,kernel", [
+    (2255, 128, 1920, 0, "gemm_bf16_pipe"),
+    (1690, 256, 4736, 0, "gemm_bf16_pipe shares=2"),
+    (1163, 128, 4096, 64, "gemm_bf16_pipe converted"),
+    (3316, 256, 2464, 0, "gemm_mid rows=256 shares=4"),          # gate and up rows ragged
+    (309, 192, 16128, 64, "gemm_mid rows=256"),
+    (1242, 128, 1662, 64, "gemm_mid rows=128"),                  # an even hidden width, not a multiple of four
+    (653, 960, 5632, 960, "gemm_q8_pipe"),
+    (755, 2304, 2752, 2304, "gemm_q8_pipe shares=3"),
+])
+def test_mlp_plans(gpu, m, k, hidden, group, kernel):
+    """SwiGLU in the epilogue of each kernel, as test_mlp. The kernel of fc1, chosen by its
+    sizes, is that of a projection of the same sizes."""
+    tx, out = gpu.empty(m * k), gpu.empty(m * 2 * hidden)
+    w = q8_weight(gpu, *synthetic_q8(1, 2 * hidden, k, group), 2 * hidden, k, group) if group else gpu.empty(2 * hidden * k)
+    for t in (tx,) if group else (tx, w):
+        run(gpu, gpu.lib.h3_hip_fill_normal_bf16, t.handle, 3, C.c_float(1.0), t.elements)
+    run(gpu, gpu.lib.h3_gpu_linear_bf16, out.handle, tx.handle, w.handle, None, m, k, 2 * hidden)
+    assert gpu.last_kernel() == kernel
+    for t in (tx, out, w):
+        gpu.free(t)
+    test_mlp(gpu, m, k, hidden, 64, group)
 
 
 @pytest.mark.parametrize("m,k,hidden,n,group", [
