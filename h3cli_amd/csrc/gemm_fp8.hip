@@ -137,10 +137,12 @@ void fp8_gemm_pipe(Fp8GemmArgs a) {
                       (int)__builtin_amdgcn_readfirstlane((unsigned)(wbase >> 32)),
                       (int)__builtin_amdgcn_readfirstlane(wrows * a.k - k0), 0x00020000};
     const unsigned lrow = 8 * wave + lane / 8;
-    unsigned o[8];     // offsets of 4 GiB and more belong to rows past M and N (h3_gemm_fp8): BUFFER_OOB
+    // From K = 2^24 on, rows of 128 and more are past M and N (h3_gemm_fp8) and their offsets
+    // would wrap: out of range instead.
+    const unsigned past = a.k >> 24 ? BUFFER_OOB : 0u;
+    unsigned o[8];
 #pragma unroll
-    for (int t = 0; t < 8; t++)
-        o[t] = __umulhi(lrow + 32 * t, a.k) ? BUFFER_OOB : (lrow + 32 * t) * a.k + swz(lrow, lane % 8) * 16;
+    for (int t = 0; t < 8; t++) o[t] = (lrow + 32 * t) * a.k + swz(lrow, lane % 8) * 16 | (t < 4 ? 0u : past);
     const unsigned mb = __builtin_amdgcn_readfirstlane(wave * 1024);
     const unsigned kmax = __builtin_amdgcn_readfirstlane((ksteps - 1) * TK);
     const unsigned kone = min(kmax, (unsigned)TK);
