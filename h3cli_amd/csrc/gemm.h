@@ -84,9 +84,11 @@ __device__ inline float gelu_tanh(float v) {
 }
 
 // silu(gate) * up with the hardware exp and reciprocal, as gelu_tanh: large |gate|
-// saturate through exp to gate * up or a signed zero.
+// saturate through exp to gate * up or a signed zero. The reciprocal flushes results below
+// the normal range, which 1 / (1 + exp(-gate)) reaches from gate = -87.4 on while exp is
+// still finite: it is taken 16 times larger.
 __device__ inline float swiglu_fast(float gate, float up) {
-    return gate * __builtin_amdgcn_rcpf(1.0f + __expf(-gate)) * up;
+    return gate * (__builtin_amdgcn_rcpf(fmaf(__expf(-gate), 0.0625f, 0.0625f)) * 0.0625f) * up;
 }
 
 // Pins an accumulator to its AGPRs up to here. An epilogue that branches (whole tile or

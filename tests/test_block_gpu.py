@@ -285,8 +285,8 @@ def test_linear_plans(gpu, m, k, n, group, bias, gelu, kernel):
     assert gpu.last_kernel() == kernel
     edges = np.arange(64, m, 64)
     rows = np.unique(np.r_[0:m:max(1, m // 16), edges[:8], edges[:8] - 1, edges[-2:], edges[-2:] - 1, m - 1])
-    got = bf16(out.read()).reshape(m, n)[rows]
-    xv = bf16(x).reshape(m, k)[rows].astype(np.float64)
+    got = bf16(out.read().reshape(m, n)[rows])
+    xv = bf16(x.reshape(m, k)[rows]).astype(np.float64)
     for at in range(0, n, 4096):
         cols = slice(at, min(at + 4096, n))
         if group:
@@ -366,6 +366,41 @@ def test_mlp(gpu, m, k, hidden, n, group):
     met = metrics(got, want)
     assert met["rel_l2"] <= 4 * 2.0 ** -9, met
     for t in (tx, out, *ws):
+        gpu.free(t)
+
+
+@pytest.mark.parametrize("m,k,hidden", [(64, 64, 64), (2255, 128, 1920), (653, 960, 5632)])
+def test_mlp_gates_near_the_end_of_exp(gpu, m, k, hidden):
+    """silu(gate) * up where 1 / (1 + exp(-gate)) is below the normal FP32 range and the
+    product with a large up is not, in the mid, pipe and q8 kernels' epilogues: one input
+    value, gates of one column each, ups of 2^100 and an fc2 that copies the first columns."""
+    print(f"[mlp gates] m={m} k={k} hidden={hidden}", flush=True)
+    gates = np.array([-60.0, -86.5, -87.0, -87.5, -88.0, -88.5, -1.0, 80.0], np.float32)
+    x, w1, w2 = np.zeros((m, k), np.float32), np.zeros((2 * hidden, k), np.float32), np.zeros((64, hidden), np.float32)
+    x[:, 0] = 1
+    w1[:8, 0], w1[hidden:hidden + 8, 0] = gates, 2.0 ** 100
+    w2[np.arange(8), np.arange(8)] = 1
+    if hidden == 5632:      # codes of one scale per column
+        scales = np.ones(2 * hidden, np.float32)
+        scales[:8], scales[hidden:] = 0.5, 2.0 ** 100
+        codes = np.zeros((2 * hidden, k), np.int8)
+        gates = np.clip(gates, -63.5, 63.5)       # 127 codes of 0.5
+        scales[1:6] = np.array([86.5, 87.0, 87.5, 88.0, 88.5], np.float32) / 100
+        codes[:8, 0] = np.round(gates / 0.5)
+        codes[1:6, 0] = -100
+        codes[hidden:hidden + 8, 0] = 1
+        t1 = q8_weight(gpu, codes.reshape(-1), scales, 2 * hidden, k, k)
+        gates = bf16(synth.f32_to_bf16((codes[:8, 0] * scales[:8]).astype(np.float32)))
+    else:
+        t1 = gpu.from_bf16(synth.f32_to_bf16(w1.reshape(-1)))
+    tx, t2, out = gpu.from_bf16(synth.f32_to_bf16(x.reshape(-1))), gpu.from_bf16(synth.f32_to_bf16(w2.reshape(-1))), gpu.empty(m * 64)
+    run(gpu, gpu.lib.h3_gpu_mlp_bf16, out.handle, tx.handle, t1.handle, t2.handle, m, k, hidden, 64)
+    got = bf16(out.read()).reshape(m, 64)[:, :8].astype(np.float64)
+    gates = gates.astype(np.float64)
+    want = gates / (1 + np.exp(-gates)) * 2.0 ** 100
+    # One BF16 rounding of the activation, copied by fc2.
+    assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want)), got[0] / want
+    for t in (tx, t1, t2, out):
         gpu.free(t)
 
 
