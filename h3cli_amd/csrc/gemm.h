@@ -28,9 +28,13 @@ struct GemmRates {
 // the number of shares of the tiles of the last wave that it is least for. Shares run in one
 // round of the CUs: half of a wave or more stays whole (7168 -> 5376, BF16: 84 tiles in 3
 // shares 72 us (whole 114), in 4, so two rounds, 96; 168 tiles whole 128, in 3 shares 146).
-// Behind one whole wave also two rounds (14336 -> 5376, 420 tiles: 3 shares 621, whole 658),
-// behind eight or more none: what is left to gain is within the noise (5376 -> 28672, 8193
-// rows, 14.4 waves: 1788 either way).
+// Behind one whole wave also two rounds (14336 -> 5376, 420 tiles: 3 shares 621, whole 658).
+// Behind eight or more only long 256-row tiles. In us, split / whole: 8941 rows, 11264 ->
+// 15104, 9 shares: 2300 / 2521; 7000 rows, 5376 -> 28672, 3: 1626 / 1664; 5742 rows, 8704 ->
+// 23808, 2: 1948 / 2008 (of 34 such projections in two shares 32 are faster, by 1.3% in the
+// mean). Short ones have nothing to gain (11772 rows, 2240 -> 26112, 3: 1444 / 1409), and
+// 128-row tiles, slower there than their rates say, must not pass others by it (2572 rows,
+// 12608 -> 25856: 1732, 256 rows 1628).
 inline GemmPlan gemm_last_wave(const h3_gpu *g, unsigned tiles, unsigned units, const GemmRates &r, float size = 1.f,
                                unsigned least_units = 1) {
     const unsigned rest = tiles % g->cus, waves = tiles / g->cus, rounds_max = waves == 1 ? 2 : 1;
@@ -39,7 +43,7 @@ inline GemmPlan gemm_last_wave(const h3_gpu *g, unsigned tiles, unsigned units, 
     if (!rest) return p;
     const float before = p.us;
     p.us += units * unit((float)rest / g->cus) + r.start;
-    if (waves >= 8) return p;
+    if (waves >= 8 && (size < 1.f || units * r.full < 85.f)) return p;
     for (unsigned s = 2; s <= 32 && s * least_units <= units && rest * s <= rounds_max * g->cus; s++) {
         const unsigned rounds = (rest * s + g->cus - 1) / g->cus;
         const float busy = (float)(rest * s) / (rounds * g->cus);

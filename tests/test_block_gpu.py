@@ -241,6 +241,7 @@ PIPE_WHOLE, PIPE_SPLIT = (2255, 128, 3840), (1690, 256, 9472)     # 135 and 256 
       for shape, kernel in ((PIPE_WHOLE, "gemm_bf16_pipe"), (PIPE_SPLIT, "gemm_bf16_pipe shares=2"))
       for bias in (False, True) for gelu in (False, True)],
     (600, 7168, 5376, 0, True, True, "gemm_bf16_pipe shares=4"),              # no whole wave
+    (8400, 4096, 16128, 0, False, False, "gemm_bf16_pipe shares=4"),          # 31 tiles behind eight waves
     (1163, 128, 8192, 64, True, True, "gemm_bf16_pipe converted"),
     (2786, 512, 6144, 64, True, False, "gemm_bf16_pipe shares=4 converted"),
     (1076, 128, 7424, 128, False, True, "gemm_bf16_pipe converted"),
