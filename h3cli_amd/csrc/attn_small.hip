@@ -304,9 +304,12 @@ int launch(h3_gpu *g, const SmallArgs &a) {
 
 // Workgroup rounds and modelled microseconds: the kernels here by 64-key tiles per
 // wave, the 256-query tile kernel by 128-key groups, the V transpose and the
-// recomputation launch included. Measured (it in brackets): 1024 keys x 8 heads, one
-// block 17.0, two 24.5 (35.2); 300 x 4: 12.1, 18.6 (23.1); 2048 x 8: 41.8, 35.5 (53.1);
-// 4200 x 2: 73.8, 59.1 (86.4); 1024 x 24: 41.4, 47.0 (41.0).
+// recomputation launch included. Measured, calls back to back (it in brackets): 1024
+// keys x 8 heads, one block 15.2, two 22.0 (34.8); 300 x 4: 10.6, 15.9 (23.8); 2048 x
+// 8: 41.7, 36.0 (53.1); 4200 x 2: 69.2, 58.9 (87.2); 384 x 40: 20.1, 16.8 (27.1); 1024
+// x 24: 39.2, 42.8 (40.6); 729 x 56: 57.8, 54.7 (41.2). A second round is counted in
+// full though it starts beside the first, so that just past one round the tile kernel
+// runs where one block is faster: 448 x 40: 22.9, 28.4 (30.3); 512 x 40: 25.9, 31.1 (31.4).
 int h3_attention_small_blocks(const h3_gpu *g, uint32_t seq, uint32_t heads) {
     // Every other variant is one of the tile kernels (15: the default one).
     if (g->attention_variant || (size_t)seq * heads * D * 2 >= (1ull << 32)) return 0;   // 32-bit buffer offsets

@@ -18,7 +18,7 @@
 //  * gemm_q8.hip: per-column int8 weights converted in a hand-scheduled loop;
 //  * gemm_skinny.hip: at most 16 rows;
 //  * gemm_small, here: any shape.
-// Both tiled kernels compute C^T = W . X^T, so a lane owns one output row and
+// The tiled kernels compute C^T = W . X^T, so a lane owns one output row and
 // consecutive columns, move operands global -> LDS directly (XOR-swizzled 16-byte
 // chunks), and remap tile ids so that the workgroups an XCD runs together share
 // weight columns in its L2.

@@ -19,7 +19,7 @@
 // Bound by the MFMAs and the power they draw: 2.5 PFLOP/s at 18225 rows, 5376 -> 21504.
 // Measured against eight compiler-scheduled waves of 128 x 64 (two per SIMD), activation
 // packing included: 8193 rows, 5376 -> 21504: 780 us (925); 18225 rows: 1.69 ms (2.07);
-// 700 rows, 14336 -> 5376: 86 us (200); 60 rows, 5376 -> 21504: 45 us (74). Results equal
+// 700 rows, 14336 -> 5376: 75 us (200); 60 rows, 5376 -> 21504: 36 us (74). Results equal
 // that kernel's bit for bit but for split tiles. Row tiles per band (18225 rows / 8193
 // rows, 5376 -> 21504, in us): 2: 1686 / 804, 3: 1840 / 753, 4: 1690 / 832, 6: 1834 / 831,
 // 8: 1910 / 841; 4, spread evenly, is taken.

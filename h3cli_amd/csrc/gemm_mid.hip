@@ -12,10 +12,10 @@
 // split as in gemm_bf16_pipe.
 //
 // Bound by memory latency and the int8 conversion at 64 rows, by the LDS-fed products
-// at 256. Measured against the pipe kernel with its conversion pass: 33 rows, 5376 ->
-// 28672, int8: 68 us (171); 256 rows, 14336 -> 5376, int8: 70 us (113); 729 rows, 5376
-// -> 28672, int8: 247 us (287); 128 rows, 5120 -> 5120, BF16: 20 us (29); and against
-// one thread per output: 729 rows, 5376 -> 96: 16 us (337).
+// at 256. Measured against the pipe kernel with its conversion pass, int8 of group 64: 33
+// rows, 5376 -> 28672: 58 us (171); 256 rows, 14336 -> 5376: 65 us (113); 729 rows, 5376 ->
+// 28672: 263 us (281); without one, BF16: 128 rows, 5120 -> 5120: 21 us (29); and against
+// one thread per output: 729 rows, 5376 -> 96: 15 us (337).
 #include "common.h"
 #include "internal.h"
 #include "gemm.h"

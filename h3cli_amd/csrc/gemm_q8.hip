@@ -25,10 +25,10 @@
 // Bound by the power that the MFMAs draw and, behind them, LDS and the conversion (9% faster
 // without its VALU instructions). Scales per group of K, loaded with each K tile, cost 20%
 // here and stay with gemm_mid. Measured against gemm_mid or, for the 1200 rows, a conversion
-// pass and gemm_bf16_pipe, in microseconds: 729 rows, 5376 -> 28672: 246 (265), 5376 ->
-// 21504: 171 (184), 7168 -> 5376: 79 (95), 14336 -> 5376: 131 (146); 1200 rows, 13824 ->
-// 5120: 197 (211). A workgroup takes 10 us before its first and after its last product,
-// gemm_mid 2: 700 rows, 1024 -> 14336: 46.8 (40.4).
+// pass and gemm_bf16_pipe, in microseconds: 729 rows, 5376 -> 28672: 214 to 228 (259), 5376 ->
+// 21504: 149 (168), 7168 -> 5376: 71 (85), 14336 -> 5376: 114 (129); 1200 rows, 13824 ->
+// 5120: 166 (202). A wave of workgroups starts and stores in 16 us (gemm_mid: 7 to 12), which
+// leaves no gain for a short K: 700 rows, 1024 -> 14336: 38 (40).
 #include "common.h"
 #include "internal.h"
 #include "gemm.h"
